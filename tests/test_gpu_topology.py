@@ -195,3 +195,59 @@ def test_strip_restart_format_mismatch_is_an_error(gpu_device):
         bridge.render(spec)
     with pytest.raises(wgc.WgcError):
         runner.render(spec, gpu_device)
+
+
+# The tiled line path: lists of up to one wave's keys, sorted in LDS, past
+# the sort's 1024 keys and past a tile's bin (256 slots here), so that the
+# tile tests every primitive; and lines of every octant around the tile edges.
+@pytest.mark.parametrize("n", [40, 200, 1300])
+@pytest.mark.parametrize("mode", ["less", "last", "blend"])
+def test_tiled_lines_crowded_tile(gpu_device, gpu_device_ext, n, mode):
+    w, h = 77, 45
+    u = scenes.splitmix_f32(6100 + n, n * 4).reshape(n, 4).astype(np.float64)
+    # through the 16x16 tile at (16, 16), one in eight anywhere
+    far = (np.arange(n) % 8 == 0)[:, None]
+    a = np.where(far, u[:, 0:2] * (w, h), 17.0 + 14.0 * u[:, 0:2])
+    b = np.where(far, u[:, 2:4] * (w, h), 17.0 + 14.0 * u[:, 2:4])
+    vb = np.zeros((2 * n, 8), np.float32)
+    for k, p in ((0, a), (1, b)):
+        vb[k::2, 0] = p[:, 0] / w * 2.0 - 1.0
+        vb[k::2, 1] = 1.0 - p[:, 1] / h * 2.0
+    vb[:, 2] = 0.25 + 0.5 * scenes.splitmix_f32(6200 + n, 2 * n)
+    vb[:, 3] = 1.0
+    vb[:, 4:8] = scenes.splitmix_f32(6300 + n, 2 * n * 4).reshape(-1, 4)
+    vb[:, 7] = 0.4
+    depth = (wgc.LESS, True) if mode == "less" else None
+    d = draw(vb, LINES, depth=depth, blend=wgc.BLEND_ALPHA if mode == "blend" else wgc.BLEND_REPLACE)
+    ext = mode == "blend"
+    spec = scenes.PassSpec(w, h, has_depth=depth is not None, clear_depth=1.0, draws=[d],
+                           semantics=wgc.SEMANTICS_EXTENDED if ext else wgc.SEMANTICS_REFERENCE,
+                           name=f"crowded line tile n={n} {mode}")
+    both(spec, gpu_device_ext if ext else gpu_device)
+
+
+@pytest.mark.parametrize("blend", [False, True])
+def test_tiled_lines_every_octant_at_tile_edges(gpu_device, gpu_device_ext, blend):
+    """From pixels beside tile corners to every end point of a ring of
+    lengths around one, two and four tiles (and back)."""
+    w, h = 160, 150
+    ends = []
+    for r in (1, 15, 16, 17, 31, 32, 33, 64):
+        for t in range(-r, r + 1, max(1, r // 4)):
+            for dx, dy in ((r, t), (-r, t), (t, r), (t, -r)):
+                for x, y in ((63, 64), (64, 79)):
+                    ends.append(((x, y), (x + dx, y + dy)))
+                    ends.append(((x + dx, y + dy), (x, y)))
+    p = np.asarray(ends, np.float64).reshape(-1, 2) + 0.5
+    vb = np.zeros((len(p), 8), np.float32)
+    vb[:, 0] = p[:, 0] / w * 2.0 - 1.0
+    vb[:, 1] = 1.0 - p[:, 1] / h * 2.0
+    vb[:, 2] = scenes.splitmix_f32(6400, len(p))
+    vb[:, 3] = 1.0
+    vb[:, 4:8] = scenes.splitmix_f32(6401, len(p) * 4).reshape(-1, 4)
+    d = draw(vb, LINES, depth=None if blend else (wgc.LESS_EQUAL, True),
+             blend=wgc.BLEND_ALPHA if blend else wgc.BLEND_REPLACE)
+    spec = scenes.PassSpec(w, h, has_depth=not blend, clear_depth=1.0, draws=[d],
+                           semantics=wgc.SEMANTICS_EXTENDED if blend else wgc.SEMANTICS_REFERENCE,
+                           name=f"lines of every octant blend={blend}")
+    both(spec, gpu_device_ext if blend else gpu_device)

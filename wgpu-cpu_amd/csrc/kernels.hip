@@ -249,6 +249,14 @@ hipError_t launch_fill(void *dst, uint64_t bytes, uint32_t value, hipStream_t st
 
 // ---- points and lines ----
 
+uint32_t lp_prep_grid(const DrawParams &d)
+{
+    uint64_t lanes = (uint64_t)d.total_prims * (d.topology == TOPO_POINT_LIST ? 1u : kLpLanes);
+    return (uint32_t)((lanes + 255u) / 256u);
+}
+
+uint32_t lp_tiles_grid(const DrawParams &d) { return std::min(d.tiles_x * d.tiles_y, 1u << 20); }
+
 static hipError_t launch_lines_user(const UserKernels &k, const DrawParams &d0, const GroupLaunch &gl, hipStream_t st,
                                     KernelTimer *kt)
 {
@@ -256,19 +264,17 @@ static hipError_t launch_lines_user(const UserKernels &k, const DrawParams &d0, 
     unsigned long long *vis = gl.vis;
     void *lp = gl.lp;
     const int n = d.topology == TOPO_POINT_LIST ? 0 : 1;
-    uint32_t g = (d.total_prims + 255u) / 256u;
-    if (gl.ordered) {
-        if (!g) return hipSuccess;
-        WGC_MLAUNCH("k_lp_prep", k.lp_prep[n], g, 256, &d, &lp);
-        uint32_t tiles = ((d.width + kLpTile - 1u) / kLpTile) * ((d.height + kLpTile - 1u) / kLpTile);
-        WGC_MLAUNCH("k_lp_ordered", k.lp_ordered[n], std::min(tiles, 65535u), 256, &d, &lp);
+    if (!d.total_prims) return hipSuccess;
+    if (n == 1 || gl.ordered) {
+        WGC_MLAUNCH("k_lp_prep", k.lp_prep[n], lp_prep_grid(d), 256, &d, &lp);
+        WGC_MLAUNCH("k_lp_tiles", gl.ordered ? k.lp_ordered[n] : k.lp_tiles, lp_tiles_grid(d), 64, &d, &lp);
         return hipSuccess;
     }
-    if (!g) return hipSuccess;
+    uint32_t g = (d.total_prims + 255u) / 256u;
     hipError_t e = launch_fill(gl.vis, 8ull * d.width * d.height, 0xFFFFFFFFu, st, kt);
     if (e != hipSuccess) return e;
-    WGC_MLAUNCH("k_lp_visibility", k.lp_vis[n], g, 256, &d, &vis);
-    WGC_MLAUNCH("k_lp_shade", k.lp_shade[n], g, 256, &d, &vis);
+    WGC_MLAUNCH("k_point_visibility", k.point_vis, g, 256, &d, &vis);
+    WGC_MLAUNCH("k_point_shade", k.point_shade, g, 256, &d, &vis);
     return hipSuccess;
 }
 

@@ -22,6 +22,10 @@ uint32_t raster_blocks_per_cu_of(bool ordered, uint32_t cfg);
 // Workgroups per CU of the single-draw setup kernel that also clips.
 template <int PROG>
 uint32_t setup_clip_blocks_per_cu_of();
+// Grids of a tiled point / line draw: kLpLanes lanes per line (a lane per
+// point); one wave per screen tile.
+uint32_t lp_prep_grid(const DrawParams &d);
+uint32_t lp_tiles_grid(const DrawParams &d);
 // A point or line draw of the program.
 template <int PROG>
 hipError_t launch_lines_of(const DrawParams &d, const GroupLaunch &gl, hipStream_t st, KernelTimer *kt);

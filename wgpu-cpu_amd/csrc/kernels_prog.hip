@@ -113,28 +113,29 @@ uint32_t setup_clip_blocks_per_cu_of()
 }
 
 template <int PROG, int N>
-static hipError_t launch_lines_t(const DrawParams &d, const GroupLaunch &gl, hipStream_t st, KernelTimer *kt)
+static hipError_t launch_tiled_lines(const DrawParams &d, const GroupLaunch &gl, hipStream_t st, KernelTimer *kt)
 {
-    uint32_t g = (d.total_prims + 255u) / 256u;
-    if (gl.ordered) {
-        if (!g) return hipSuccess;
-        WGC_LAUNCH("k_lp_prep", (k_lp_prep<PROG, N>), g, 256, d, (LpPrim<N> *)gl.lp);
-        uint32_t tiles = ((d.width + kLpTile - 1u) / kLpTile) * ((d.height + kLpTile - 1u) / kLpTile);
-        WGC_LAUNCH("k_lp_ordered", (k_lp_ordered<PROG, N>), min(tiles, 65535u), 256, d, (const LpPrim<N> *)gl.lp);
-        return hipSuccess;
-    }
-    if (!g) return hipSuccess;
-    hipError_t e = launch_fill(gl.vis, 8ull * d.width * d.height, 0xFFFFFFFFu, st, kt);
-    if (e != hipSuccess) return e;
-    WGC_LAUNCH("k_lp_visibility", (k_lp_visibility<PROG, N>), g, 256, d, gl.vis);
-    WGC_LAUNCH("k_lp_shade", (k_lp_shade<PROG, N>), g, 256, d, (const unsigned long long *)gl.vis);
+    LpRec<N> *recs = (LpRec<N> *)gl.lp;
+    WGC_LAUNCH("k_lp_prep", (k_lp_prep<PROG, N>), lp_prep_grid(d), 256, d, recs);
+    if (N == 1 || gl.ordered)
+        WGC_LAUNCH("k_lp_tiles", (k_lp_tiles<PROG, N, true>), lp_tiles_grid(d), 64, d, (const LpRec<N> *)recs);
+    else if constexpr (N == 2)
+        WGC_LAUNCH("k_lp_tiles", (k_lp_tiles<PROG, N, false>), lp_tiles_grid(d), 64, d, (const LpRec<N> *)recs);
     return hipSuccess;
 }
 
 template <int PROG>
 hipError_t launch_lines_of(const DrawParams &d, const GroupLaunch &gl, hipStream_t st, KernelTimer *kt)
 {
-    return d.topology == TOPO_POINT_LIST ? launch_lines_t<PROG, 1>(d, gl, st, kt) : launch_lines_t<PROG, 2>(d, gl, st, kt);
+    if (!d.total_prims) return hipSuccess;
+    if (d.topology != TOPO_POINT_LIST) return launch_tiled_lines<PROG, 2>(d, gl, st, kt);
+    if (gl.ordered) return launch_tiled_lines<PROG, 1>(d, gl, st, kt);
+    uint32_t g = (d.total_prims + 255u) / 256u;
+    hipError_t e = launch_fill(gl.vis, 8ull * d.width * d.height, 0xFFFFFFFFu, st, kt);
+    if (e != hipSuccess) return e;
+    WGC_LAUNCH("k_point_visibility", (k_point_visibility<PROG>), g, 256, d, gl.vis);
+    WGC_LAUNCH("k_point_shade", (k_point_shade<PROG>), g, 256, d, (const unsigned long long *)gl.vis);
+    return hipSuccess;
 }
 
 template uint32_t setup_clip_blocks_per_cu_of<WGC_PROG>();

@@ -2218,8 +2218,8 @@ static int32_t build_draw(WgcDevice_T *dev, const PassCommand &pc, const PassSta
     // raster tile option: of the tile shapes it is the fastest for it (200k
     // blended triangles over 2560x2440: 0.63 ms, the others 0.74-3.0 ms) and
     // holds the most keys per pixel; WGSL pipelines' kernels are compiled for
-    // 16x16 tiles only
-    d.tile_shift = (d.resolve == RES_ORDERED || pl->user) ? 4u : tile_shift;
+    // 16x16 tiles only, and so are the point / line kernels (kLpTile)
+    d.tile_shift = (d.resolve == RES_ORDERED || pl->user || d.topology <= TOPO_LINE_STRIP) ? 4u : tile_shift;
     // points and lines: unsigned pixel indices (their keys and visibility buffer)
     if (d.topology <= TOPO_LINE_STRIP && (uint64_t)w * h > 0xFFFFFFFFull)
         return set_error(WGC_ERR_UNSUPPORTED, "target too large for points and lines");
@@ -2262,17 +2262,43 @@ static bool restart_strip(const DrawParams &d)
 
 static bool is_point_or_line(const DrawParams &d) { return d.topology <= TOPO_LINE_STRIP; }
 
-// Scratch of a point / line draw: the per-pixel visibility values, or for
-// an ordered draw the set-up primitives.
-static size_t layout_lines(Step &st, uint8_t *base, uint32_t *frag_px, size_t frag_px_size, WgcDevice_T *dev)
+// Points in order-independent depth modes resolve over a visibility buffer
+// of the target (a point is one pixel: one atomic per point, nothing to
+// bin); lines, and points applied in API order, go through screen tiles.
+static bool tiled_lines(const DrawParams &d)
+{
+    return d.topology != TOPO_POINT_LIST || d.resolve == RES_ORDERED;
+}
+
+// Key slots per tile of a tiled point / line draw: 256, or sixteen times
+// the draw's primitives per tile when that is more (a tile whose list is
+// longer tests every primitive's bounds instead), at most as many as there
+// are primitives and, together, 64 MiB.
+static uint64_t line_bin_cap(const DrawParams &d)
+{
+    uint64_t tiles = std::max<uint64_t>((uint64_t)d.tiles_x * d.tiles_y, 1);
+    uint64_t cap = std::max<uint64_t>(256, (16ull * d.total_prims + tiles - 1) / tiles);
+    return std::min<uint64_t>(std::min<uint64_t>(cap, d.total_prims), (64ull << 20) / (4 * tiles));
+}
+
+// Scratch of a point / line draw: the per-pixel visibility values, or the
+// set-up primitives and the tiles' bins.  `zone`: the tile counts (all
+// point / line steps of a plan share them: each tile kernel leaves them zero).
+static size_t layout_lines(Step &st, uint8_t *base, uint8_t *zone, uint32_t *frag_px, size_t frag_px_size,
+                           WgcDevice_T *dev)
 {
     DrawParams &d = st.draws[0];
-    bool ordered = d.resolve == RES_ORDERED;
-    size_t bytes = ordered ? align_up(std::max<uint64_t>((uint64_t)kLpPrimBytes * d.total_prims, 256), 256)
-                           : align_up(8ull * d.width * d.height, 256);
+    bool tiled = tiled_lines(d);
+    uint64_t cap = line_bin_cap(d), tiles = (uint64_t)d.tiles_x * d.tiles_y;
+    size_t rec = align_up((uint64_t)(d.topology == TOPO_POINT_LIST ? kPointRecBytes : kLineRecBytes) * d.total_prims, 256);
+    size_t bytes = tiled ? align_up(std::max<uint64_t>(rec + 4 * cap * tiles, 256), 256)
+                         : align_up(8ull * d.width * d.height, 256);
     if (!base) return bytes;
-    st.gl.vis = ordered ? nullptr : (unsigned long long *)base;
-    st.gl.lp = ordered ? (void *)base : nullptr;
+    st.gl.vis = tiled ? nullptr : (unsigned long long *)base;
+    st.gl.lp = tiled ? (void *)base : nullptr;
+    d.s.bins = tiled ? (uint32_t *)(base + rec) : nullptr;
+    d.s.bin_cap = (uint32_t)cap;
+    d.s.tile_count = (uint32_t *)zone;
     d.s.frags = dev->d_frags;
     d.s.error = dev->d_error;
     d.s.frag_px = (frag_px && frag_px_size == (size_t)d.width * d.height * 4u) ? frag_px : nullptr;
@@ -2662,8 +2688,9 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
                     add_group(plan.steps, {dw.d}, cfg, stage++);
                     continue;
                 }
-                // points and lines: the pass's clear (if still pending) first
-                if (dw.d.init_clear) {
+                // points and lines: the tile kernel applies the pass's clear (if
+                // still pending), else it comes first
+                if (dw.d.init_clear && (!tiled_lines(dw.d) || !dw.d.total_prims)) {
                     Step c;
                     c.kind = StepKind::Clear;
                     c.color = dw.d.clear_color_on ? (uint32_t *)dw.d.color : nullptr;
@@ -2724,7 +2751,7 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
     }
     // 3. scratch: the groups of a stage side by side, stages reusing the
     //    arena (they run one after another)
-    size_t need = 0, zneed = 0, kneed = 0;
+    size_t need = 0, zneed = 0, kneed = 0, line_zone = 0;
     size_t tables = 0;
     size_t stage_off = 0;
     uint32_t cur_stage = UINT32_MAX;
@@ -2737,10 +2764,12 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
         s.arena_off = stage_off;
         s.zone_off = zneed;
         s.keep_off = kneed;
-        size_t bytes = s.kind == StepKind::Lines ? layout_lines(s, nullptr, nullptr, 0, dev)
+        size_t bytes = s.kind == StepKind::Lines ? layout_lines(s, nullptr, nullptr, nullptr, 0, dev)
                                                   : layout_group(s, nullptr, nullptr, nullptr, nullptr, 0, dev);
         stage_off = align_up(stage_off + bytes, 256);
         need = std::max(need, stage_off);
+        if (s.kind == StepKind::Lines && tiled_lines(s.draws[0]))
+            line_zone = std::max<size_t>(line_zone, align_up(4ull * group_tiles(s), 256));
         if (s.kind == StepKind::Group) {
             // active-list entries hold the global tile in kItemShift bits
             if (group_tiles(s) >= (1ull << kItemShift))
@@ -2760,6 +2789,8 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
             tables = align_up(tables + n * sizeof(DrawParams) + 8 * (n + 1) + 4 * (waves + tiles), 256);
         }
     }
+    size_t line_zone_off = zneed;
+    zneed += line_zone;
     uint8_t *zone_base, *keep_base, *arena_base;
     if (noalloc) {
         // the static scratch: zero region, kept-zero region, then the stages
@@ -2814,8 +2845,8 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
     }
     for (Step &s : plan.steps) {
         if (s.kind == StepKind::Lines) {
-            layout_lines(s, arena_base + s.arena_off, dev->frag_px, dev->frag_px_size, dev);
-            plan.launches += s.draws[0].total_prims == 0 ? 0 : (s.gl.ordered ? 2 : 3);
+            layout_lines(s, arena_base + s.arena_off, zone_base + line_zone_off, dev->frag_px, dev->frag_px_size, dev);
+            plan.launches += s.draws[0].total_prims == 0 ? 0 : (tiled_lines(s.draws[0]) ? 2 : 3);
             plan.prims += s.draws[0].total_prims;
             continue;
         }

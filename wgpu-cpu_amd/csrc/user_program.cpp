@@ -387,11 +387,11 @@ bool build_user_program(int hip_device, const wgsl::Module &vm, const std::strin
         "wgc::k_clip<5, false>",           "wgc::k_clip<5, true>",
         "wgc::k_tiles<5, false, 16, 256>", "wgc::k_tiles<5, true, 16, 256>",
         "wgc::k_raster<5, false, 16, 256>", "wgc::k_raster<5, true, 16, 256>",
-        "wgc::k_lp_visibility<5, 1>",      "wgc::k_lp_visibility<5, 2>",
-        "wgc::k_lp_shade<5, 1>",           "wgc::k_lp_shade<5, 2>",
-        "wgc::k_lp_ordered<5, 1>",         "wgc::k_lp_ordered<5, 2>",
         "wgc::k_setup<5, false, true>",
+        "wgc::k_point_visibility<5>",      "wgc::k_point_shade<5>",
         "wgc::k_lp_prep<5, 1>",            "wgc::k_lp_prep<5, 2>",
+        "wgc::k_lp_tiles<5, 1, true>",     "wgc::k_lp_tiles<5, 2, true>",
+        "wgc::k_lp_tiles<5, 2, false>",
     };
     Compiled c;
     if (!rtc_build(hip_device, src, {{"wgc_user.h", g}}, names, c, err)) return false;
@@ -404,15 +404,15 @@ bool build_user_program(int hip_device, const wgsl::Module &vm, const std::strin
         k.clip[m] = c.fns[2 + m];
         k.tiles[m] = c.fns[4 + m];
         k.raster[m] = c.fns[6 + m];
-        k.lp_vis[m] = c.fns[8 + m];
-        k.lp_shade[m] = c.fns[10 + m];
-        k.lp_ordered[m] = c.fns[12 + m];
+        k.lp_prep[m] = c.fns[11 + m];
+        k.lp_ordered[m] = c.fns[13 + m];
         k.occ_tiles[m] = occupancy(k.tiles[m], 256);
         k.occ_raster[m] = occupancy(k.raster[m], 256);
     }
-    k.setup_clip = c.fns[14];
-    k.lp_prep[0] = c.fns[15];
-    k.lp_prep[1] = c.fns[16];
+    k.setup_clip = c.fns[8];
+    k.point_vis = c.fns[9];
+    k.point_shade = c.fns[10];
+    k.lp_tiles = c.fns[15];
     k.occ_setup_clip = occupancy(k.setup_clip, 256);
     return true;
 }

@@ -23,8 +23,8 @@ struct GroupLaunch {
     uint2 *clip_list;            // (draw, primitive) pairs that cross a clip plane
     uint32_t clip_cap;
     uint32_t inline_clip;        // single draw whose setup waves all fit at once: setup clips
-    unsigned long long *vis;     // points and lines: one visibility value per pixel
-    void *lp;                    // ordered points and lines: kLpPrimBytes per primitive (LpPrim)
+    unsigned long long *vis;     // order-independent points: one visibility value per pixel
+    void *lp;                    // lines and ordered points: a record per primitive (LpRec)
 };
 
 // Brackets launches with HIP events on the launching stream; the runtime
@@ -93,7 +93,8 @@ struct KernelTimer {
 struct UserKernels {
     hipModule_t module = nullptr;
     hipFunction_t setup[2]{}, clip[2]{}, tiles[2]{}, raster[2]{};
-    hipFunction_t lp_vis[2]{}, lp_shade[2]{}, lp_ordered[2]{}, lp_prep[2]{};   // index: points 0, lines 1
+    hipFunction_t point_vis{}, point_shade{};
+    hipFunction_t lp_prep[2]{}, lp_ordered[2]{}, lp_tiles{};   // index: points 0, lines 1; lp_tiles: lines
     hipFunction_t setup_clip{};   // single draws: setup that clips in place
     uint32_t occ_tiles[2]{}, occ_raster[2]{}, occ_setup_clip{};
 };
@@ -102,8 +103,8 @@ struct UserKernels {
 // `k`, the rest from the library.
 hipError_t launch_user(const UserKernels &k, const DrawParams &d, const BatchArgs &b, const GroupLaunch &gl,
                        bool multi, hipStream_t st, KernelTimer *kt);
-// A point or line draw: visibility + shading passes over its primitives
-// (or one ordered workgroup); gl.vis holds one 64-bit value per pixel.
+// A point or line draw: set-up and binning, then one wave per screen tile;
+// order-independent points: visibility and shading passes over gl.vis.
 hipError_t launch_lines(const DrawParams &d, const GroupLaunch &gl, hipStream_t st, KernelTimer *kt);
 
 // A single draw passes its parameters by value (b.draws unused, b.n == 1);
