@@ -1,0 +1,112 @@
+"""Consecutive draws of a pass that share one launch group, bit for bit
+against the oracle: draws with their own uniforms, textures, culling,
+interpolation, viewports and instance counts, of sizes around a wave of
+primitives, with triangles across the clip planes and over many tiles."""
+import numpy as np
+import pytest
+
+import wgc
+from oracle import bridge
+from wgc import runner, scenes
+
+from test_gpu_parity import announce, assert_parity, clip_color_draw, random_clip_triangles
+
+pytestmark = pytest.mark.gpu
+
+
+def triangles(n, seed, w, h, depth, blend=wgc.BLEND_REPLACE, **kw):
+    vb = random_clip_triangles(n, seed, w, h, spread=1.3, size_px=(3.0, 70.0), w_range=(0.5, 2.0),
+                               z_levels=[0.3, 0.5, 0.7], alpha=(0.2, 0.8))
+    vb[::9, :, 2] = -0.2 * vb[::9, :, 3]          # some beyond the near plane
+    vb[4::13, 0, 2] = 1.3 * vb[4::13, 0, 3]
+    return clip_color_draw(vb, depth=depth, blend=blend, **kw)
+
+
+def both(spec, dev):
+    assert_parity(spec, dev)
+    assert_parity(scenes.as_wgsl(spec), dev)
+
+
+@pytest.mark.parametrize("mode", [(wgc.LESS, True), (wgc.GREATER_EQUAL, True), (wgc.LESS, False), (wgc.ALWAYS, True),
+                                  (wgc.NOT_EQUAL, True), None, "blend"],
+                         ids=["less", "greater_equal", "less_no_write", "always", "not_equal", "no_depth", "blend"])
+@pytest.mark.parametrize("sizes", [(1, 63, 64, 65, 200), (700, 1, 900)], ids=["around_a_wave", "large"])
+def test_draws_of_one_pass(gpu_device, gpu_device_ext, mode, sizes):
+    w, h = 171, 133
+    ext = mode == "blend"
+    depth = None if ext else mode
+    draws = [triangles(n, 7000 + 10 * k, w, h, depth, wgc.BLEND_ALPHA if ext else wgc.BLEND_REPLACE)
+             for k, n in enumerate(sizes)]
+    draws[1].cull_mode = wgc.CULL_BACK
+    draws[1].instance_count = 2
+    draws[2].viewport = (-20.0, 9.0, 190.0, 140.0, 0.0, 1.0)
+    draws[0].interp = wgc.INTERP_FLAT
+    spec = scenes.PassSpec(w, h, clear_color=(0.1, 0.2, 0.3, 1.0), has_depth=depth is not None, clear_depth=0.6,
+                           draws=draws, semantics=wgc.SEMANTICS_EXTENDED if ext else wgc.SEMANTICS_REFERENCE,
+                           name=f"draws of one pass {mode} {sizes}")
+    both(spec, gpu_device_ext if ext else gpu_device)
+
+
+def test_groups_break_where_the_rule_changes(gpu_device_ext):
+    """Opaque, blended and opaque draws, one with a scissor rect of its own."""
+    w, h = 130, 90
+    draws = [triangles(150, 7100, w, h, (wgc.LESS, True)), triangles(90, 7101, w, h, (wgc.LESS, True)),
+             triangles(120, 7102, w, h, (wgc.LESS, False), wgc.BLEND_ALPHA),
+             triangles(80, 7103, w, h, (wgc.LESS, False), wgc.BLEND_ALPHA),
+             triangles(110, 7104, w, h, (wgc.LESS, True)), triangles(60, 7105, w, h, (wgc.LESS, True))]
+    draws[4].scissor = (20, 10, 77, 61)
+    spec = scenes.PassSpec(w, h, has_depth=True, clear_depth=1.0, draws=draws, semantics=wgc.SEMANTICS_EXTENDED,
+                           name="groups of draws")
+    both(spec, gpu_device_ext)
+
+
+@pytest.mark.parametrize("tile", [0, 1, 6])
+def test_textured_objects_with_their_own_uniforms(gpu_device, tile):
+    w, h = 200, 150
+    draws = []
+    for k in range(5):
+        d = scenes.config2_textured(seed=50 + k, width=w, height=h, segments=12, rings=6 + k).draws[0]
+        size = 8 << k
+        d.texture = (size, size, scenes.checker_texture(size, 3, 16, 90 + k), k % 2 == 1)
+        d.uniform = scenes.perspective_view(45.0 + 12 * k, w / h, 0.1, 10.0, 2.0 + 0.4 * k)
+        d.address_u = (wgc.REPEAT, wgc.CLAMP_TO_EDGE, wgc.MIRROR_REPEAT)[k % 3]
+        draws.append(d)
+    spec = scenes.PassSpec(w, h, has_depth=True, clear_depth=1.0, draws=draws, name=f"objects, tile option {tile}")
+    gpu_device.set_option(wgc.OPTION_RASTER_TILE, tile)
+    try:
+        both(spec, gpu_device)
+    finally:
+        gpu_device.set_option(wgc.OPTION_RASTER_TILE, 0)
+
+
+def test_primitive_index_and_big_triangles_across_draws(gpu_device):
+    """@builtin(primitive_index) counts from each draw's first primitive; a
+    triangle over the whole target in each draw goes through the big list."""
+    w, h = 260, 180
+    draws = []
+    for k in range(3):
+        d = scenes.fragment_test_scene(scenes.FS_PRIM_RED, scenes.EARLY_NONE, n=100 + 33 * k, width=w, height=h,
+                                       seed=7200 + k).draws[0]
+        vb = np.frombuffer(d.vertex_data, np.float32).copy().reshape(-1, 3, 8)
+        vb[7, :, :2] = ((-3.0, -3.0), (3.0, -3.0), (0.0, 4.0))
+        d.vertex_data = vb.tobytes()
+        draws.append(d)
+    spec = scenes.PassSpec(w, h, clear_color=(0, 0, 0, 1), has_depth=True, clear_depth=0.7, draws=draws,
+                           name="primitive index across draws")
+    assert_parity(spec, gpu_device)
+
+
+def test_noalloc_draws_one_at_a_time_equals_the_group(gpu_device):
+    announce("draws of one pass, allocation-free")
+    w, h = 171, 133
+    draws = [triangles(n, 7300 + n, w, h, (wgc.LESS, True)) for n in (40, 300, 65)]
+    spec = scenes.PassSpec(w, h, has_depth=True, clear_depth=1.0, draws=draws)
+    pp = runner.PreparedPass(gpu_device, spec)
+    pp.submit()
+    want = pp.results()[0]
+    gpu_device.submit_noalloc([pp.command_buffer])
+    got = pp.results()[0]
+    ref = bridge.render(spec)
+    for r in (want, got):
+        assert np.array_equal(r.color, ref.color)
+        assert np.array_equal(r.depth.view(np.uint32), ref.depth.view(np.uint32))

@@ -132,13 +132,34 @@ uint32_t raster_blocks_per_cu(uint32_t program, bool ordered, bool multi, uint32
     }
 }
 
-uint32_t setup_clip_blocks_per_cu(uint32_t program)
+uint32_t setup_clip_blocks_per_cu(uint32_t program, bool merged)
 {
     switch (program) {
-#define X(P) case P: return setup_clip_blocks_per_cu_of<P>();
+#define X(P) case P: return setup_clip_blocks_per_cu_of<P>(merged);
     WGC_EACH_PROGRAM(X)
 #undef X
     default: return 0;
+    }
+}
+
+uint32_t merged_blocks_per_cu(uint32_t program, bool ordered)
+{
+    switch (program) {
+#define X(P) case P: return merged_blocks_per_cu_of<P>(ordered);
+    WGC_EACH_PROGRAM(X)
+#undef X
+    default: return 1;
+    }
+}
+
+hipError_t launch_merged(const DrawParams &d0, const BatchArgs &b, const GroupLaunch &gl, hipStream_t st,
+                         KernelTimer *kt)
+{
+    switch (gl.program) {
+#define X(P) case P: return launch_merged_of<P>(d0, b, gl, st, kt);
+    WGC_EACH_PROGRAM(X)
+#undef X
+    default: return hipErrorInvalidValue;
     }
 }
 
@@ -159,38 +180,32 @@ uint32_t setup_clip_blocks_per_cu(uint32_t program)
         if (e_ != hipSuccess) return e_;                                                          \
     } while (0)
 
-template <bool MULTI>
-static hipError_t launch_user_t(const UserKernels &k, const DrawParams &d0, const BatchArgs &b0,
-                                const GroupLaunch &gl, hipStream_t st, KernelTimer *kt)
+hipError_t launch_user(const UserKernels &k, const DrawParams &d0, const BatchArgs &b0, const GroupLaunch &gl,
+                       bool multi, hipStream_t st, KernelTimer *kt)
 {
     DrawParams d = d0;
     BatchArgs b = b0;
     const uint2 *clip_list = gl.clip_list;
     uint32_t clip_cap = gl.clip_cap;
-    const int m = MULTI ? 1 : 0;
-    if (!MULTI && d.strip_restart && d.indexed && d.topology == TOPO_TRIANGLE_STRIP && d.count > 0) {
+    const int m = multi || gl.merged ? 1 : 0;
+    if (!m && d.strip_restart && d.indexed && d.topology == TOPO_TRIANGLE_STRIP && d.count > 0) {
         hipError_t e = launch_strip_prepass(d, st, kt);
         if (e != hipSuccess) return e;
     }
     if (gl.total_prims > 0) {
         uint32_t g = (gl.total_prims + 255u) / 256u;
-        if (!MULTI && gl.inline_clip) {
-            WGC_MLAUNCH("k_setup", k.setup_clip, g, 256, &d, &b);
+        if (gl.inline_clip) {
+            WGC_MLAUNCH("k_setup", k.setup_clip[m], g, 256, &d, &b);
         } else {
             WGC_MLAUNCH("k_setup", k.setup[m], g, 256, &d, &b);
             uint32_t gc = min(max(g / 2u, 1u), 2048u);
             WGC_MLAUNCH("k_clip", k.clip[m], gc, 256, &d, &b, &clip_list, &clip_cap);
         }
     }
-    if (gl.ordered) WGC_MLAUNCH("k_raster", k.raster[m], gl.raster_grid, 256, &d, &b);
-    else WGC_MLAUNCH("k_tiles", k.tiles[m], gl.raster_grid, 256, &d, &b);
+    if (gl.ordered)
+        WGC_MLAUNCH("k_raster", gl.merged ? k.raster_merged : k.raster[m], gl.raster_grid, 256, &d, &b);
+    else WGC_MLAUNCH("k_tiles", gl.merged ? k.tiles_merged : k.tiles[m], gl.raster_grid, 256, &d, &b);
     return hipSuccess;
-}
-
-hipError_t launch_user(const UserKernels &k, const DrawParams &d, const BatchArgs &b, const GroupLaunch &gl,
-                       bool multi, hipStream_t st, KernelTimer *kt)
-{
-    return multi ? launch_user_t<true>(k, d, b, gl, st, kt) : launch_user_t<false>(k, d, b, gl, st, kt);
 }
 
 // ---- copies (command encoder copy_* / clear_*) ----

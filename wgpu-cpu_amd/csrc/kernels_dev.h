@@ -376,14 +376,18 @@ __device__ __forceinline__ void clear_target(const DrawParams &d)
 }
 
 // CLIP: the primitives that cross a clip plane are clipped here, by their
-// wave (single draws whose waves all fit on the GPU at once: no k_clip
-// launch); otherwise they go to the clip list.
+// wave (groups of one target whose waves all fit on the GPU at once: no
+// k_clip launch); otherwise they go to the clip list.
+// MULTI: a table of draws, independent ones or consecutive ones of a pass
+// (d0 is the first of these).
 template <int PROG, bool MULTI, bool CLIP = false>
 __global__ __launch_bounds__(256) void k_setup(DrawParams d0, BatchArgs b)
 {
     uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t di = 0, p = g;
     if constexpr (MULTI) {
+        if constexpr (CLIP)   // (the draws of a pass; a batched group never pre-clears)
+            if (b.preclear) clear_target(d0);
         // draw ranges are padded to whole waves, so a wave never spans draws
         if (g >= b.total_prims) return;
         // every lane of the wave is in the same draw: look it up once, in
@@ -425,9 +429,10 @@ __global__ __launch_bounds__(256) void k_setup(DrawParams d0, BatchArgs b)
                         uint32_t tx0, ty0, tx1, ty1;
                         if (tile_bbox(d, s, tx0, ty0, tx1, ty1)) {
                             has_rec = true;
-                            rec = make_uint4(p << 7, tx0 | (ty0 << 16), tx1 | (ty1 << 16), di);
+                            uint32_t key = (d.s.key_base + p) << 7;
+                            rec = make_uint4(key, tx0 | (ty0 << 16), tx1 | (ty1 << 16), di);
                             ntiles = (tx1 - tx0 + 1) * (ty1 - ty0 + 1);
-                            write_record(d.s.tri + (size_t)p * kRecWords, r, v, p << 7, ff);
+                            write_record(d.s.tri + (size_t)p * kRecWords, r, v, key, ff);
                         }
                     }
                 } else if (cc == 1) {
@@ -631,7 +636,7 @@ __device__ __forceinline__ void clip_wave(uint32_t di, uint32_t p, bool act, Dra
             if (!coord_ok(r)) {
                 atomicOr(d.s.error, (uint32_t)ERR_COORD_RANGE);
             } else if (r.total != 0.0f && tile_bbox(d, s, tx0, ty0, tx1, ty1)) {
-                key = (gp << 7) | (leaf << 1) | 1u;
+                key = ((d.s.key_base + gp) << 7) | (leaf << 1) | 1u;
                 write_record(d.s.clip_tri + (size_t)slot * kRecWords, r, v, key, ff);
                 bin = true;
             }
@@ -809,6 +814,7 @@ struct RasterShared {
     ScanTri scan[kBatch];
     uint32_t wide[kBatch];
     uint32_t span[kBatch][TS];      // ordered path: per-row spans of the staged triangles
+    uint32_t draw[kBatch];          // draws of a pass: the triangle's
     uint32_t keys[kBatch];
     uint32_t nkeys;
 };
@@ -907,7 +913,7 @@ __device__ __forceinline__ void frag_position(const DrawParams &d, const TriLds 
 {
     float iw[3];
     if (T.key & 1u) {
-        uint32_t pr = T.key >> 7, sub = (T.key >> 1) & 63u;
+        uint32_t pr = (T.key >> 7) - d.s.key_base, sub = (T.key >> 1) & 63u;
         const float *ct = d.s.clip_tris + (size_t)(d.s.clip_base[pr] + sub) * kClipFloats;
 #pragma unroll
         for (int k = 0; k < 3; ++k) iw[k] = 1.0f / ct[k * 7 + 3];
@@ -976,8 +982,8 @@ __device__ __forceinline__ bool fragment_color(const DrawParams &d, const TriLds
                 var[c] = acc;
             }
         }
-        // primitive_index: the key's primitive within its instance
-        uint32_t prim = (T.key >> 7) % d.nprim;
+        // primitive_index: the key's primitive within its draw and instance
+        uint32_t prim = ((T.key >> 7) - d.s.key_base) % d.nprim;
         uint32_t rc = user_fragment(d, TriPos{d, T, lc}, T.ff != 0u, prim, var, color, frag_depth);
         if (rc == 0u) return true;
         if (rc != 3u) atomicOr(d.s.error, (uint32_t)ERR_SHADER);   // 3: discard
@@ -1101,10 +1107,15 @@ __device__ __forceinline__ void shade_fragment(const DrawParams &d, const TriLds
 // Colour and depth of a pixel's winning fragment: its triangle record is
 // read back (from L2, shared by the neighbouring pixels it won) and the same
 // barycentrics are evaluated again, bit for bit.
-template <int PROG>
-__device__ __forceinline__ uint32_t winner_color(const DrawParams &d, uint32_t key, float pxf, float pyf, float &z,
-                                                 const float *srgb)
+// MERGED (the draws of a pass): `d` is the first draw, whose record arrays
+// hold every draw's records by the group's primitive; the winner's draw
+// shades it, the lanes of each draw together (its parameters stay scalar).
+template <int PROG, bool MERGED>
+__device__ __forceinline__ uint32_t winner_color(const DrawParams &d, const BatchArgs &b, uint32_t key, float pxf,
+                                                 float pyf, float &z, const float *srgb)
 {
+    uint32_t di = 0;
+    if constexpr (MERGED) di = b.wave_draw[key >> 13];
     TriLds T;
     ScanTri S;
     uint32_t wide;
@@ -1115,7 +1126,17 @@ __device__ __forceinline__ uint32_t winner_color(const DrawParams &d, uint32_t k
     // pipelines whose fragment shader can discard use the ordered path, so
     // the winner always writes (an aborted invocation raised ERR_SHADER)
     float unused = z;
-    (void)fragment_color<PROG>(d, T, lc, color, srgb, &unused);
+    if constexpr (MERGED) {
+        for (;;) {
+            uint32_t u = __builtin_amdgcn_readfirstlane(di);
+            if (di == u) {
+                (void)fragment_color<PROG>(b.draws[u], T, lc, color, srgb, &unused);
+                break;
+            }
+        }
+    } else {
+        (void)fragment_color<PROG>(d, T, lc, color, srgb, &unused);
+    }
     return pack_color(color, d.color_bgra);
 }
 
@@ -1163,14 +1184,17 @@ __device__ __forceinline__ bool oi_pass(const DrawParams &d, float z, float init
 }
 
 // Stages sh.keys[0..n) into LDS and applies them to this lane's pixels.
-template <int PROG, bool ORDERED, int TS, int NT>
-__device__ __forceinline__ void raster_batch(const DrawParams &d, RasterShared<TS> &sh, uint32_t n, uint32_t x0,
-                                             uint32_t y0, PixelState (&ps)[TS * TS / NT],
+template <int PROG, bool ORDERED, int TS, int NT, bool MERGED>
+__device__ __forceinline__ void raster_batch(const DrawParams &d, const BatchArgs &b, RasterShared<TS> &sh, uint32_t n,
+                                             uint32_t x0, uint32_t y0, PixelState (&ps)[TS * TS / NT],
                                              uint32_t (&nfrag)[TS * TS / NT])
 {
     constexpr int PPT = TS * TS / NT;
     uint32_t tid = threadIdx.x;
-    if (tid < n) stage_record(d, sh.keys[tid], sh.tri[tid], sh.scan[tid], sh.wide[tid]);
+    if (tid < n) {
+        if constexpr (MERGED) sh.draw[tid] = b.wave_draw[sh.keys[tid] >> 13];
+        stage_record(d, sh.keys[tid], sh.tri[tid], sh.scan[tid], sh.wide[tid]);
+    }
     __syncthreads();
     // per-row spans inside the scissor and the tile, tile-relative
     int64_t sx0 = d.scissor[0], sy0 = d.scissor[1];
@@ -1199,7 +1223,10 @@ __device__ __forceinline__ void raster_batch(const DrawParams &d, RasterShared<T
             uint32_t sp = sh.span[e][ly];
             if (lx < (sp & 0xFFFFu) || lx > (sp >> 16)) continue;
             nfrag[k]++;
-            shade_fragment<PROG, ORDERED>(d, sh.tri[e], pxf, pyf, ps[k]);
+            if constexpr (MERGED)
+                shade_fragment<PROG, ORDERED>(b.draws[__builtin_amdgcn_readfirstlane(sh.draw[e])], sh.tri[e], pxf, pyf,
+                                              ps[k]);
+            else shade_fragment<PROG, ORDERED>(d, sh.tri[e], pxf, pyf, ps[k]);
         }
     });
     __syncthreads();
@@ -1311,9 +1338,10 @@ __device__ __forceinline__ void sort_olist(uint32_t *olist, uint32_t total)
 
 // One tile of an ordered draw: load or clear, apply its triangles in API
 // order, store.
-template <int PROG, int TS, int NT>
-__device__ __forceinline__ void raster_tile(const DrawParams &d, uint32_t tile, RasterShared<TS> &sh,
-                                            uint32_t *olist, uint32_t &olist_n, uint32_t &frag_acc)
+template <int PROG, int TS, int NT, bool MERGED>
+__device__ __forceinline__ void raster_tile(const DrawParams &d, const BatchArgs &b, uint32_t tile,
+                                            RasterShared<TS> &sh, uint32_t *olist, uint32_t &olist_n,
+                                            uint32_t &frag_acc)
 {
     constexpr bool ORDERED = true;
     constexpr int PPT = TS * TS / NT;
@@ -1392,7 +1420,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &d, uint32_t tile, 
             uint32_t n = min((uint32_t)kBatch, total - fpos);
             if (tid < n) sh.keys[tid] = olist[fpos + tid];
             fpos += n;
-            raster_batch<PROG, ORDERED, TS, NT>(d, sh, n, x0, y0, ps, nfrag);
+            raster_batch<PROG, ORDERED, TS, NT, MERGED>(d, b, sh, n, x0, y0, ps, nfrag);
         }
         if (!overflow || hi > 0xFFFFFFFFull) break;
         // the next chunk: the keys from hi on, at most kOrderedCap of them
@@ -1426,7 +1454,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &d, uint32_t tile, 
                           (d.resolve != RES_PASS_LAST || d.depth_compare == CMP_EQUAL ||
                            d.depth_compare == CMP_ALWAYS);
             float zw;
-            ps[k].col = ps[k].has ? winner_color<PROG>(d, ps[k].key, (float)px, (float)py, zw, d.srgb_lut)
+            ps[k].col = ps[k].has ? winner_color<PROG, MERGED>(d, b, ps[k].key, (float)px, (float)py, zw, d.srgb_lut)
                                   : init_col[k];
         }
         if (d.color) store_color(d, pix, ps[k].col);
@@ -1698,8 +1726,8 @@ __device__ __forceinline__ uint32_t vis_batch(const DrawParams &d, VisShared<TS,
 // and the same barycentrics are evaluated again, bit for bit.  Colour and
 // depth are stored where the pass changes them (a winner, or the
 // LoadOp::Clear values).
-template <int PROG, int TS, int NT>
-__device__ __forceinline__ void raster_tile_oi(const DrawParams &d, uint32_t tile, uint32_t item,
+template <int PROG, int TS, int NT, bool MERGED>
+__device__ __forceinline__ void raster_tile_oi(const DrawParams &d, const BatchArgs &b, uint32_t tile, uint32_t item,
                                                VisShared<TS, NT> &sh, const float *srgb, uint32_t &frag_acc)
 {
     constexpr int PPT = TS * TS / NT;
@@ -1787,7 +1815,7 @@ __device__ __forceinline__ void raster_tile_oi(const DrawParams &d, uint32_t til
         unsigned long long v = sh.best[q];
         if (v != ~0ull) {
             float z;
-            uint32_t col = winner_color<PROG>(d, oi_key(d.resolve, v), (float)px, (float)py, z, srgb);
+            uint32_t col = winner_color<PROG, MERGED>(d, b, oi_key(d.resolve, v), (float)px, (float)py, z, srgb);
             if (d.color) store_color(d, pix, col);
             if (d.depth) {
                 if (write_depth_mode) store_depth(d, pix, z);
@@ -1936,7 +1964,9 @@ __device__ __forceinline__ void count_fragments(const DrawParams &d0, const Batc
 // scheduled (no shared work counter); each tile's fragments are applied in
 // API order.  First the active tiles, then the untouched ones in chunks,
 // strided over the whole grid.
-template <int PROG, bool MULTI, int TS, int NT>
+// MERGED: consecutive draws of one pass (d0 the first of them), one list of
+// tiles for all.
+template <int PROG, bool MULTI, int TS, int NT, bool MERGED = false>
 __global__ __launch_bounds__(NT) void k_raster(DrawParams d0, BatchArgs b)
 {
     constexpr int PPT = TS * TS / NT;
@@ -1960,7 +1990,7 @@ __global__ __launch_bounds__(NT) void k_raster(DrawParams d0, BatchArgs b)
         if (dyn && threadIdx.x == 0) tk = atomicAdd(w.queue(b), 1u);
         uint32_t di, tile, it;
         locate_tile<MULTI>(d0, b, e, di, tile, it);
-        raster_tile<PROG, TS, NT>(draw_at<MULTI>(d0, b, di), tile, sh, olist, olist_n, frag_acc);
+        raster_tile<PROG, TS, NT, MERGED>(draw_at<MULTI>(d0, b, di), b, tile, sh, olist, olist_n, frag_acc);
         if (!dyn) break;
         if (threadIdx.x == 0) ticket = tk;
         __syncthreads();
@@ -1971,7 +2001,7 @@ __global__ __launch_bounds__(NT) void k_raster(DrawParams d0, BatchArgs b)
     if (untouched_pass(b))
         for (uint32_t c = gridDim.x - 1u - w.first; c < b.n_chunks; c += gridDim.x)
             untouched_chunk<MULTI, TS, NT>(d0, b, c, kinds, [&](const DrawParams &d, uint32_t tile) {
-                raster_tile<PROG, TS, NT>(d, tile, sh, olist, olist_n, frag_acc);
+                raster_tile<PROG, TS, NT, MERGED>(d, b, tile, sh, olist, olist_n, frag_acc);
             });
     count_fragments<MULTI, NT>(d0, b, frag_acc, wave_frags);
 }
@@ -1979,7 +2009,7 @@ __global__ __launch_bounds__(NT) void k_raster(DrawParams d0, BatchArgs b)
 // Order-independent draws: visibility and shading of every active tile
 // (raster_tile_oi), then the untouched tiles in chunks, strided over the
 // whole grid.
-template <int PROG, bool MULTI, int TS, int NT>
+template <int PROG, bool MULTI, int TS, int NT, bool MERGED = false>
 __global__ __launch_bounds__(NT, (TilesOccupancy<TS, NT>::value)) void k_tiles(DrawParams d0, BatchArgs b)
 {
     constexpr int PPT = TS * TS / NT;
@@ -2011,7 +2041,7 @@ __global__ __launch_bounds__(NT, (TilesOccupancy<TS, NT>::value)) void k_tiles(D
         if (dyn && threadIdx.x == 0) tk = atomicAdd(w.queue(b), 1u);
         uint32_t di, tile, it;
         locate_tile<MULTI>(d0, b, e, di, tile, it);
-        raster_tile_oi<PROG, TS, NT>(draw_at<MULTI>(d0, b, di), tile, it, sh, srgb, frag_acc);
+        raster_tile_oi<PROG, TS, NT, MERGED>(draw_at<MULTI>(d0, b, di), b, tile, it, sh, srgb, frag_acc);
         if (!dyn) break;
         if (threadIdx.x == 0) ticket = tk;
         __syncthreads();
@@ -2022,7 +2052,7 @@ __global__ __launch_bounds__(NT, (TilesOccupancy<TS, NT>::value)) void k_tiles(D
     if (untouched_pass(b))
         for (uint32_t c = gridDim.x - 1u - w.first; c < b.n_chunks; c += gridDim.x)
             untouched_chunk<MULTI, TS, NT>(d0, b, c, kinds, [&](const DrawParams &d, uint32_t tile) {
-                raster_tile_oi<PROG, TS, NT>(d, tile, 0u, sh, srgb, frag_acc);
+                raster_tile_oi<PROG, TS, NT, MERGED>(d, b, tile, 0u, sh, srgb, frag_acc);
             });
     count_fragments<MULTI, NT>(d0, b, frag_acc, wave_frags);
 }

@@ -19,9 +19,16 @@ hipError_t launch_program(const DrawParams &d, const BatchArgs &b, const GroupLa
 // cfg) resident on one CU at once.
 template <int PROG, bool MULTI>
 uint32_t raster_blocks_per_cu_of(bool ordered, uint32_t cfg);
-// Workgroups per CU of the single-draw setup kernel that also clips.
+// Consecutive draws of one pass: setup (and clip) over the table of draws,
+// then one raster launch over their target.
 template <int PROG>
-uint32_t setup_clip_blocks_per_cu_of();
+hipError_t launch_merged_of(const DrawParams &d0, const BatchArgs &b, const GroupLaunch &gl, hipStream_t st,
+                            KernelTimer *kt);
+template <int PROG>
+uint32_t merged_blocks_per_cu_of(bool ordered);
+// Workgroups per CU of the setup kernels that also clip.
+template <int PROG>
+uint32_t setup_clip_blocks_per_cu_of(bool merged);
 // Grids of a tiled point / line draw: kLpLanes lanes per line (a lane per
 // point); one wave per screen tile.
 uint32_t lp_prep_grid(const DrawParams &d);

@@ -74,6 +74,10 @@ uint32_t raster_blocks_per_cu_of(bool ordered, uint32_t cfg)
     }
 }
 
+// Clip workgroups for g setup workgroups (kClipPerWave primitives per wave;
+// the count is only known on the device).
+static uint32_t clip_grid(uint32_t g) { return min(max(g / 2u, 1u), 2048u); }
+
 template <int PROG, bool MULTI>
 hipError_t launch_program(const DrawParams &d, const BatchArgs &b, const GroupLaunch &gl, hipStream_t st,
                           KernelTimer *kt)
@@ -91,9 +95,7 @@ hipError_t launch_program(const DrawParams &d, const BatchArgs &b, const GroupLa
             }
         }
         WGC_LAUNCH("k_setup", (k_setup<PROG, MULTI>), g, 256, d, b);
-        // kClipPerWave primitives per wave; the count is only known on the device
-        uint32_t gc = min(max(g / 2u, 1u), 2048u);
-        WGC_LAUNCH("k_clip", (k_clip<PROG, MULTI>), gc, 256, d, b, gl.clip_list, gl.clip_cap);
+        WGC_LAUNCH("k_clip", (k_clip<PROG, MULTI>), clip_grid(g), 256, d, b, gl.clip_list, gl.clip_cap);
     }
     return launch_raster<PROG, MULTI>(d, b, gl, st, kt);
 }
@@ -105,11 +107,39 @@ template uint32_t raster_blocks_per_cu_of<WGC_PROG, WGC_MULTI != 0>(bool, uint32
 #if !WGC_MULTI
 
 template <int PROG>
-uint32_t setup_clip_blocks_per_cu_of()
+uint32_t setup_clip_blocks_per_cu_of(bool merged)
 {
-    static uint32_t r = 0;
-    if (!r) r = occupancy_of(k_setup<PROG, false, true>, 256);
-    return r;
+    static uint32_t r[2] = {0, 0};
+    if (!r[merged]) r[merged] = merged ? occupancy_of(k_setup<PROG, true, true>, 256)
+                                       : occupancy_of(k_setup<PROG, false, true>, 256);
+    return r[merged];
+}
+
+template <int PROG>
+uint32_t merged_blocks_per_cu_of(bool ordered)
+{
+    static uint32_t r[2] = {0, 0};
+    if (!r[ordered]) r[ordered] = ordered ? occupancy_of(k_raster<PROG, false, 16, 256, true>, 256)
+                                          : occupancy_of(k_tiles<PROG, false, 16, 256, true>, 256);
+    return r[ordered];
+}
+
+template <int PROG>
+hipError_t launch_merged_of(const DrawParams &d0, const BatchArgs &b, const GroupLaunch &gl, hipStream_t st,
+                            KernelTimer *kt)
+{
+    if (gl.total_prims > 0) {
+        uint32_t g = (gl.total_prims + 255u) / 256u;
+        if (gl.inline_clip) {
+            WGC_LAUNCH("k_setup", (k_setup<PROG, true, true>), g, 256, d0, b);
+        } else {
+            WGC_LAUNCH("k_setup", (k_setup<PROG, true>), g, 256, d0, b);
+            WGC_LAUNCH("k_clip", (k_clip<PROG, true>), clip_grid(g), 256, d0, b, gl.clip_list, gl.clip_cap);
+        }
+    }
+    if (gl.ordered) WGC_LAUNCH("k_raster", (k_raster<PROG, false, 16, 256, true>), gl.raster_grid, 256, d0, b);
+    else WGC_LAUNCH("k_tiles", (k_tiles<PROG, false, 16, 256, true>), gl.raster_grid, 256, d0, b);
+    return hipSuccess;
 }
 
 template <int PROG, int N>
@@ -138,7 +168,10 @@ hipError_t launch_lines_of(const DrawParams &d, const GroupLaunch &gl, hipStream
     return hipSuccess;
 }
 
-template uint32_t setup_clip_blocks_per_cu_of<WGC_PROG>();
+template uint32_t setup_clip_blocks_per_cu_of<WGC_PROG>(bool);
+template uint32_t merged_blocks_per_cu_of<WGC_PROG>(bool);
+template hipError_t launch_merged_of<WGC_PROG>(const DrawParams &, const BatchArgs &, const GroupLaunch &, hipStream_t,
+                                               KernelTimer *);
 template hipError_t launch_lines_of<WGC_PROG>(const DrawParams &, const GroupLaunch &, hipStream_t, KernelTimer *);
 
 #endif

@@ -399,7 +399,8 @@ enum class StepKind { Group, Clear, Copy, Lines };
 
 struct Step {
     StepKind kind = StepKind::Group;
-    bool multi = false;
+    bool multi = false;              // independent draws, each with its own target
+    bool merged = false;             // consecutive draws of one pass
     std::vector<DrawParams> draws;   // the group's draws (scratch filled when laid out)
     GroupLaunch gl{};
     BatchArgs batch{};
@@ -1503,7 +1504,8 @@ extern "C" int32_t wgc_wgsl_check_pipeline(const char *source, size_t length, co
     bool has_fs = false;
     for (auto &e : m.entries) has_fs = has_fs || e.stage == wgsl::Stage::Fragment;
     if (!build_user_program(-1, m, vertex_entry ? vertex_entry : "", has_fs ? &m : nullptr,
-                            fragment_entry ? fragment_entry : "", semantics == WGC_SEMANTICS_EXTENDED, up, err))
+                            fragment_entry ? fragment_entry : "", semantics == WGC_SEMANTICS_EXTENDED, PipelineUses{}, up,
+                            err))
         return set_error(err.compare(0, 5, "hipRT") == 0 ? WGC_ERR_DEVICE : WGC_ERR_INVALID, err);
     return WGC_OK;
 }
@@ -1525,6 +1527,8 @@ extern "C" int32_t wgc_wgsl_translate(const char *source, size_t length, uint32_
     }
     return WGC_OK;
 }
+
+static uint32_t resolve_mode(const WgcRenderPipelineDescriptor &p, bool depth_test, bool blend);
 
 extern "C" int32_t wgc_render_pipeline_create(WgcDevice device, const WgcRenderPipelineDescriptor *desc,
                                               WgcRenderPipeline *out)
@@ -1574,10 +1578,18 @@ extern "C" int32_t wgc_render_pipeline_create(WgcDevice device, const WgcRenderP
         auto up = std::make_shared<UserProgram>();
         std::string err;
         const WgcShaderModule_T *fm = desc->fragment_module;
+        bool extended = device->semantics == WGC_SEMANTICS_EXTENDED;
+        PipelineUses uses;
+        uses.points = desc->topology == WGC_TOPOLOGY_POINT_LIST;
+        uses.lines = desc->topology == WGC_TOPOLOGY_LINE_LIST ||
+                     desc->topology == WGC_TOPOLOGY_LINE_STRIP;
+        uses.triangles = !uses.points && !uses.lines;
+        uses.ordered = resolve_mode(*desc, desc->has_depth_stencil != 0, extended && desc->blend == WGC_BLEND_ALPHA) ==
+                       RES_ORDERED;
         if (!build_user_program(device->hip_device, *desc->vertex_module->wgsl,
                                 desc->vertex_entry ? desc->vertex_entry : "", fm ? fm->wgsl.get() : nullptr,
                                 desc->fragment_entry ? desc->fragment_entry : "",
-                                device->semantics == WGC_SEMANTICS_EXTENDED, *up, err)) {
+                                extended, uses, *up, err)) {
             release(p);
             return set_error(err.compare(0, 5, "hipRT") == 0 || err.compare(0, 5, "hipMo") == 0 ? WGC_ERR_DEVICE
                                                                                              : WGC_ERR_INVALID,
@@ -2305,11 +2317,21 @@ static size_t layout_lines(Step &st, uint8_t *base, uint8_t *zone, uint32_t *fra
     return bytes;
 }
 
+// The targets of a group: one per draw, or one for the draws of a pass.
+static size_t group_targets(const Step &st) { return st.merged ? 1 : st.draws.size(); }
+
 static uint64_t group_tiles(const Step &st)
 {
     uint64_t tiles = 0;
-    for (const DrawParams &d : st.draws) tiles += (uint64_t)d.tiles_x * d.tiles_y;
+    for (size_t i = 0; i < group_targets(st); ++i) tiles += (uint64_t)st.draws[i].tiles_x * st.draws[i].tiles_y;
     return tiles;
+}
+
+// A draw's primitives in its group's numbering: whole waves where the
+// group's setup runs over a table of draws (a wave never spans two).
+static uint64_t group_prims(const Step &st, const DrawParams &d)
+{
+    return st.multi || st.merged ? align_up(d.total_prims, 64) : d.total_prims;
 }
 
 // A group's words in the zero region: its header, per-draw counters, tile
@@ -2317,14 +2339,14 @@ static uint64_t group_tiles(const Step &st)
 static size_t zone_bytes(const Step &st)
 {
     uint64_t tiles = group_tiles(st);
-    return align_up(4ull * H_NUM, 256) + align_up(4ull * C_NUM * st.draws.size(), 256) + 2 * align_up(4ull * tiles, 256);
+    return align_up(4ull * H_NUM, 256) + align_up(4ull * C_NUM * group_targets(st), 256) + 2 * align_up(4ull * tiles, 256);
 }
 
 // A group's bytes in the kept-zero region: the merged winners of split
 // tiles (order-independent groups only), 8 bytes per tile pixel.
 static size_t keep_bytes(const Step &st)
 {
-    if (st.gl.ordered || st.multi || st.draws.empty()) return 0;
+    if (st.gl.ordered || st.multi || st.draws.empty()) return 0;   // (draws of a pass: one target, split as well)
     uint64_t tile_px = 1ull << (2 * st.draws[0].tile_shift);
     return align_up(8ull * tile_px * group_tiles(st), 256);
 }
@@ -2333,8 +2355,8 @@ static size_t keep_bytes(const Step &st)
 // tile shape, so that a tile of two batches or more spreads over several
 // workgroups (a single pass has about one tile per resident workgroup, and
 // its kernel lasts as long as its slowest tile) while ordinary ones stay
-// whole.  Single order-independent draws only: ordered tiles are never
-// split, and a batched group has many tiles per workgroup anyway.
+// whole.  Order-independent groups of one target only: ordered tiles are
+// never split, and a batched group has many tiles per workgroup anyway.
 static uint32_t split_for(const Step &st)
 {
     if (st.gl.ordered || st.multi) return 0;
@@ -2345,21 +2367,27 @@ static uint32_t split_for(const Step &st)
 static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep, uint32_t *frag_px,
                            size_t frag_px_size, WgcDevice_T *dev)
 {
-    uint32_t n = (uint32_t)st.draws.size();
-    uint64_t total_tiles = 0, clip_rec_cap = 0, prims = 0, prims_padded = 0;
+    // one unit of tiles, bins, records and counters per target
+    uint32_t n = (uint32_t)group_targets(st);
+    uint64_t total_tiles = 0, clip_rec_cap = 0, prims = 0, all_prims = 0;
     bool any_clear = false;
-    std::vector<uint64_t> clip_cap(n);
+    std::vector<uint64_t> unit_prims(n), clip_cap(n);
     for (uint32_t i = 0; i < n; ++i) {
         const DrawParams &d = st.draws[i];
         total_tiles += (uint64_t)d.tiles_x * d.tiles_y;
-        clip_cap[i] = 2ull * d.total_prims + 1024ull;
-        clip_rec_cap += clip_cap[i];
-        prims += d.total_prims;
-        prims_padded += st.multi ? align_up(d.total_prims, 64) : d.total_prims;
         any_clear = any_clear || d.init_clear;
     }
-    // bins, per draw: slots for twice the tile's pixels, or four times the
-    // draw's primitives per tile when that is more (a bin rarely fills; the
+    for (size_t k = 0; k < st.draws.size(); ++k) {
+        prims += st.draws[k].total_prims;
+        all_prims += group_prims(st, st.draws[k]);
+        unit_prims[st.merged ? 0 : k] += st.merged ? group_prims(st, st.draws[k]) : st.draws[k].total_prims;
+    }
+    for (uint32_t i = 0; i < n; ++i) {
+        clip_cap[i] = 2ull * unit_prims[i] + 1024ull;
+        clip_rec_cap += clip_cap[i];
+    }
+    // bins, per target: slots for twice the tile's pixels, or four times the
+    // target's primitives per tile when that is more (a bin rarely fills; the
     // entries past it go to the spill list, which holds every entry at most)
     uint64_t tile_px = st.draws.empty() ? 0 : (1ull << (2 * st.draws[0].tile_shift));
     std::vector<uint64_t> bin_cap(n);
@@ -2367,14 +2395,14 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
     for (uint32_t i = 0; i < n; ++i) {
         const DrawParams &d = st.draws[i];
         uint64_t tiles = std::max<uint64_t>((uint64_t)d.tiles_x * d.tiles_y, 1);
-        uint64_t per_tile = (4ull * d.total_prims + tiles - 1) / tiles;
+        uint64_t per_tile = (4ull * unit_prims[i] + tiles - 1) / tiles;
         uint64_t cap = 2 * tile_px;
         while (cap < per_tile) cap <<= 1;
-        cap = std::min<uint64_t>(cap, d.total_prims + clip_cap[i]);   // no tile holds more
+        cap = std::min<uint64_t>(cap, unit_prims[i] + clip_cap[i]);   // no tile holds more
         bin_cap[i] = std::max<uint64_t>(std::min<uint64_t>(cap, 0xFFFFFFFFull / tiles), 1);
         bins_total += bin_cap[i] * tiles;
     }
-    uint64_t spill_cap = (prims_padded + clip_rec_cap) * (uint64_t)kMaxBinTiles;
+    uint64_t spill_cap = (all_prims + clip_rec_cap) * (uint64_t)kMaxBinTiles;
     size_t off = 0;
     auto take = [&](size_t bytes) {
         size_t o = off;
@@ -2387,13 +2415,13 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
     std::vector<size_t> o_big(n), o_tri(n), o_ctri(n), o_ct(n), o_cb(n), o_ss(n);
     for (uint32_t i = 0; i < n; ++i) {
         const DrawParams &d = st.draws[i];
-        uint64_t rc = d.total_prims + clip_cap[i];
+        uint64_t rc = unit_prims[i] + clip_cap[i];
         o_ss[i] = take(restart_strip(d) ? 4ull * ((d.count + kStripChunk - 1) / kStripChunk) : 0);
         o_big[i] = take(16 * rc);
-        o_tri[i] = take(4ull * kRecWords * d.total_prims);
+        o_tri[i] = take(4ull * kRecWords * unit_prims[i]);
         o_ctri[i] = take(4ull * kRecWords * clip_cap[i]);
         o_ct[i] = take(4ull * kClipFloats * clip_cap[i]);
-        o_cb[i] = take(4ull * d.total_prims);
+        o_cb[i] = take(4ull * unit_prims[i]);
     }
     if (!base) return off;
     GroupLaunch &gl = st.gl;
@@ -2408,17 +2436,17 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
     uint32_t split = split_for(st);
     gl.clip_list = (uint2 *)(base + o_cl);
     gl.clip_cap = (uint32_t)prims;
-    // a single triangle draw whose setup workgroups are all resident at
-    // once clips in setup (no separate clip launch)
+    // a group of one target whose setup workgroups are all resident at once
+    // clips in setup (no separate clip launch)
     gl.inline_clip = 0;
     if (!st.multi && !is_point_or_line(st.draws[0])) {
-        uint64_t blocks = (prims + 255) / 256;
-        uint32_t per_cu = gl.user ? gl.user->occ_setup_clip : setup_clip_blocks_per_cu(gl.program);
+        uint64_t blocks = (all_prims + 255) / 256;
+        uint32_t per_cu = gl.user ? gl.user->occ_setup_clip[st.merged] : setup_clip_blocks_per_cu(gl.program, st.merged);
         gl.inline_clip = blocks <= (uint64_t)dev->cu_count * per_cu ? 1u : 0u;
     }
     gl.vis = nullptr;
     gl.lp = nullptr;
-    b.n = n;
+    b.n = (uint32_t)st.draws.size();
     b.total_tiles = (uint32_t)total_tiles;
     b.n_chunks = (uint32_t)((total_tiles + kClearChunk - 1) / kClearChunk);
     b.header = gl.header;
@@ -2426,21 +2454,22 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
     b.active_list = (uint32_t *)(base + o_al);
     b.counters = gl.counters;
     b.n_counters = gl.n_counters;
-    // a single draw clears its whole target in setup when setup has a thread
-    // for every 32 pixels (then the stores drain while setup waits on its
-    // loads and atomics); the tile kernel then skips the untouched tiles and
-    // stores only the pixels the draw writes.  (A batched group leaves its
-    // clears to the tile kernel, where they hide behind latency-bound work:
-    // stored separately they cost more than they save.)
+    // a group of one target clears the whole of it in setup when setup has a
+    // thread for every 32 pixels (then the stores drain while setup waits on
+    // its loads and atomics); the tile kernel then skips the untouched tiles
+    // and stores only the pixels the draw writes.  (A batched group leaves
+    // its clears to the tile kernel, where they hide behind latency-bound
+    // work: stored separately they cost more than they save.)  The setup over
+    // a table of draws does so in its form that clips.
     bool preclear = false;
-    if (!st.multi && any_clear && prims > 0) {
-        uint64_t threads = align_up(prims, 256), px = (uint64_t)st.draws[0].width * st.draws[0].height;
+    if (!st.multi && any_clear && prims > 0 && (!st.merged || gl.inline_clip)) {
+        uint64_t threads = align_up(all_prims, 256), px = (uint64_t)st.draws[0].width * st.draws[0].height;
         preclear = threads * 32 >= px;
     }
     b.preclear = preclear ? 1u : 0u;
     b.any_clear = (any_clear && !b.preclear) ? 1u : 0u;
     b.pad = 0;
-    if (!st.multi) {
+    if (!st.multi && !st.merged) {
         b.draws = nullptr;
         b.prim_base = nullptr;
         b.tile_base = nullptr;
@@ -2451,14 +2480,18 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
     uint32_t occ = 1;
     if (gl.user) {
         int m = st.multi ? 1 : 0;
-        occ = gl.ordered ? gl.user->occ_raster[m] : gl.user->occ_tiles[m];
+        if (st.merged) occ = gl.ordered ? gl.user->occ_raster_merged : gl.user->occ_tiles_merged;
+        else occ = gl.ordered ? gl.user->occ_raster[m] : gl.user->occ_tiles[m];
+    } else if (st.merged) {
+        occ = merged_blocks_per_cu(gl.program, gl.ordered != 0);
     } else {
         occ = raster_blocks_per_cu(gl.program, gl.ordered != 0, st.multi, gl.raster_cfg);
     }
     gl.raster_grid = resident_grid(dev, occ, total_tiles + b.n_chunks);
-    uint64_t tile_base = 0, bin_base = 0;
-    for (uint32_t i = 0; i < n; ++i) {
-        DrawParams &d = st.draws[i];
+    uint64_t tile_base = 0, bin_base = 0, prim_base = 0;
+    for (size_t k = 0; k < st.draws.size(); ++k) {
+        uint32_t i = st.merged ? 0u : (uint32_t)k;   // the draw's target
+        DrawParams &d = st.draws[k];
         Scratch &s = d.s;
         d.preclear = (preclear && d.init_clear) ? 1u : 0u;
         s.tile_count = gl.tile_count + tile_base;
@@ -2467,16 +2500,18 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
         s.split = split;
         s.split_inv = split ? 1.0f / (float)split : 0.0f;
         s.bins = (uint32_t *)(base + o_bins) + bin_base;
-        bin_base += bin_cap[i] * std::max<uint64_t>((uint64_t)d.tiles_x * d.tiles_y, 1);
         s.spill = (uint2 *)(base + o_sp);
         s.active_list = b.active_list;
         s.header = gl.header;
         s.clip_list = gl.clip_list;
         s.big = (uint4 *)(base + o_big[i]);
-        s.tri = (uint32_t *)(base + o_tri[i]);
+        // the draws of a pass: consecutive ranges of the target's arrays
+        s.key_base = (uint32_t)prim_base;
+        s.tri = (uint32_t *)(base + o_tri[i]) + prim_base * kRecWords;
         s.clip_tri = (uint32_t *)(base + o_ctri[i]);
         s.clip_tris = (float *)(base + o_ct[i]);
-        s.clip_base = (uint32_t *)(base + o_cb[i]);
+        s.clip_base = (uint32_t *)(base + o_cb[i]) + prim_base;
+        if (st.merged) prim_base += group_prims(st, d);
         s.strip_sep = restart_strip(d) ? (int32_t *)(base + o_ss[i]) : nullptr;
         s.counters = gl.counters + C_NUM * i;
         s.frags = dev->d_frags;
@@ -2487,10 +2522,13 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
         s.bin_cap = (uint32_t)bin_cap[i];
         s.spill_cap = (uint32_t)std::min<uint64_t>(spill_cap, 0xFFFFFFFFull);
         s.active_cap = (uint32_t)(total_tiles * kMaxItems);
-        s.big_cap = (uint32_t)(d.total_prims + clip_cap[i]);
+        s.big_cap = (uint32_t)(unit_prims[i] + clip_cap[i]);
         s.clip_list_cap = (uint32_t)prims;
         s.clip_tri_cap = (uint32_t)clip_cap[i];
-        tile_base += (uint64_t)d.tiles_x * d.tiles_y;
+        if (!st.merged) {
+            bin_base += bin_cap[i] * std::max<uint64_t>((uint64_t)d.tiles_x * d.tiles_y, 1);
+            tile_base += (uint64_t)d.tiles_x * d.tiles_y;
+        }
     }
     return off;
 }
@@ -2566,18 +2604,49 @@ static int32_t collect_pass(WgcDevice_T *dev, const PassCommand &pc, uint32_t ti
     return WGC_OK;
 }
 
-static void add_group(std::vector<Step> &steps, std::vector<DrawParams> draws, uint32_t cfg, uint32_t stage)
+// Whether a draw may share a launch group with the draws of its pass before
+// it: the same shaders, and the same per-pixel rule, so that the group
+// resolves its fragments as one draw with the draws' primitives one after
+// the other would (keys number them in API order).  What a triangle or a
+// fragment shader reads of its draw (buffers, bindings, viewport, culling,
+// interpolation) is looked up per draw.
+static bool same_group(const DrawParams &a, const DrawParams &b)
+{
+    return a.program == b.program && a.user == b.user && a.resolve == b.resolve && a.blend == b.blend &&
+           a.depth_test == b.depth_test && a.depth_compare == b.depth_compare && a.depth_write == b.depth_write &&
+           a.fs_early == b.fs_early && a.fs_depth_tested == b.fs_depth_tested &&
+           !memcmp(a.scissor, b.scissor, sizeof a.scissor) && !is_point_or_line(b) && !restart_strip(b);
+}
+
+// Primitives of a merged group at most: its scratch is about 1.1 KB a
+// primitive for all its draws at once, and launches of this size are long
+// against the gaps between them (a draw of 500k triangles runs 100 us).
+static constexpr uint64_t kMergedPrims = 1ull << 20;
+
+// A launch group of one draw, of independent draws, or (`merged`) of
+// consecutive draws of a pass (16x16 tiles under every tile option).
+static void add_group(std::vector<Step> &steps, std::vector<DrawParams> draws, uint32_t cfg, uint32_t stage,
+                      bool merged = false)
 {
     Step s;
     s.stage = stage;
     s.kind = StepKind::Group;
-    s.multi = draws.size() > 1;
+    s.merged = merged;
+    s.multi = draws.size() > 1 && !merged;
+    s.gl.merged = merged ? 1u : 0u;
     s.gl.program = draws[0].program;
     s.gl.ordered = draws[0].resolve == RES_ORDERED;
     s.gl.user = (const UserKernels *)draws[0].user;
-    s.gl.raster_cfg = s.gl.user ? (uint32_t)RASTER_16x16_256 : cfg;
+    s.gl.raster_cfg = s.gl.user || merged ? (uint32_t)RASTER_16x16_256 : cfg;
     uint64_t prims = 0;
-    for (auto &d : draws) prims += s.multi ? align_up(d.total_prims, 64) : d.total_prims;
+    for (auto &d : draws) {
+        prims += group_prims(s, d);
+        if (merged) {
+            d.tile_shift = 4u;
+            d.tiles_x = (d.width + 15u) >> 4;
+            d.tiles_y = (d.height + 15u) >> 4;
+        }
+    }
     s.gl.total_prims = (uint32_t)prims;
     s.draws = std::move(draws);
     steps.push_back(std::move(s));
@@ -2683,9 +2752,24 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
                 pw.copy_step.stage = stage++;
                 plan.steps.push_back(pw.copy_step);
             }
-            for (auto &dw : pw.draws) {
+            for (size_t k = 0; k < pw.draws.size(); ++k) {
+                DrawWork &dw = pw.draws[k];
                 if (!is_point_or_line(dw.d)) {
-                    add_group(plan.steps, {dw.d}, cfg, stage++);
+                    // consecutive draws with the same shaders and per-pixel
+                    // rule run as one group (the allocation-free form has no
+                    // table of draws).  24 objects of about 3000 triangles
+                    // over 1366x768: 640 us a draw at a time, 73 us as
+                    // one group
+                    std::vector<DrawParams> run{dw.d};
+                    uint64_t prims = align_up(dw.d.total_prims, 64);
+                    while (!noalloc && !restart_strip(dw.d) && k + 1 < pw.draws.size() &&
+                           same_group(dw.d, pw.draws[k + 1].d) &&
+                           prims + align_up(pw.draws[k + 1].d.total_prims, 64) <= kMergedPrims) {
+                        run.push_back(pw.draws[++k].d);
+                        prims += align_up(run.back().total_prims, 64);
+                    }
+                    bool merged = run.size() > 1;
+                    add_group(plan.steps, std::move(run), cfg, stage++, merged);
                     continue;
                 }
                 // points and lines: the tile kernel applies the pass's clear (if
@@ -2777,15 +2861,12 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
             zneed += zone_bytes(s);
             kneed += keep_bytes(s);
         }
-        if (s.multi) {
+        if (s.multi || s.merged) {
             // draws, primitive and tile prefixes, the draw of every wave of
-            // primitives and of every tile
+            // primitives and (independent draws) of every tile
             s.table_off = tables;
-            size_t n = s.draws.size(), waves = 0, tiles = 0;
-            for (const DrawParams &d : s.draws) {
-                waves += align_up(d.total_prims, 64) / 64;
-                tiles += (size_t)d.tiles_x * d.tiles_y;
-            }
+            size_t n = s.draws.size(), waves = 0, tiles = s.multi ? group_tiles(s) : 0;
+            for (const DrawParams &d : s.draws) waves += align_up(d.total_prims, 64) / 64;
             tables = align_up(tables + n * sizeof(DrawParams) + 8 * (n + 1) + 4 * (waves + tiles), 256);
         }
     }
@@ -2858,7 +2939,7 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
                      dev->frag_px_size, dev);
         plan.launches += (s.gl.total_prims > 0 ? (s.gl.inline_clip ? 2 : 3) : 1) + (!s.multi && restart_strip(s.draws[0]) ? 2 : 0);
         for (auto &d : s.draws) plan.prims += d.total_prims;
-        if (!s.multi) continue;
+        if (!s.multi && !s.merged) continue;
         uint32_t n = (uint32_t)s.draws.size();
         uint8_t *h = plan.h_tables + s.table_off;
         uint8_t *dptr = plan.d_tables + s.table_off;
@@ -2870,7 +2951,7 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
             pb[k] = acc_p;
             tb[k] = acc_t;
             acc_p += (uint32_t)align_up(s.draws[k].total_prims, 64);
-            acc_t += s.draws[k].tiles_x * s.draws[k].tiles_y;
+            if (s.multi) acc_t += s.draws[k].tiles_x * s.draws[k].tiles_y;
         }
         pb[n] = acc_p;
         tb[n] = acc_t;
@@ -2886,7 +2967,6 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
         s.batch.tile_draw = s.batch.wave_draw + acc_p / 64;
         s.batch.n = n;
         s.batch.total_prims = acc_p;
-        s.batch.total_tiles = acc_t;
     }
     if (tables)
         HIP_TRY(hipMemcpyAsync(plan.d_tables, plan.h_tables, tables, hipMemcpyHostToDevice, dev->stream),
@@ -2908,6 +2988,7 @@ static hipError_t launch_step(WgcDevice_T *dev, const Step &s, hipStream_t st, K
     }
     if (s.kind == StepKind::Lines) return launch_lines(s.draws[0], s.gl, st, kt);
     if (s.gl.user) return launch_user(*s.gl.user, s.draws[0], s.batch, s.gl, s.multi, st, kt);
+    if (s.merged) return launch_merged(s.draws[0], s.batch, s.gl, st, kt);
     if (s.multi) return launch_batch(s.draws[0], s.batch, s.gl, st, kt);
     return launch_draw(s.draws[0], s.batch, s.gl, st, kt);
 }

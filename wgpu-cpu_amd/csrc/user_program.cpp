@@ -39,7 +39,7 @@ struct Compiled {
 };
 
 std::mutex g_cache_mu;
-std::map<std::pair<int, std::string>, Compiled> g_cache;   // (device, source) -> program
+std::map<std::pair<int, std::string>, Compiled> g_cache;   // (device, source and kernels) -> program
 
 // Compiles `src` (with the embedded headers and `extra` headers) and loads
 // it on device `hip_device` (< 0: compile only); `names` are name
@@ -49,6 +49,7 @@ bool rtc_build(int hip_device, const std::string &src, const std::vector<std::pa
 {
     std::string key = src;
     for (auto &h : extra) key += "\n//--" + h.first + "\n" + h.second;
+    for (auto &n : names) key += "\n//--" + n;
     {
         std::lock_guard<std::mutex> g(g_cache_mu);
         auto it = g_cache.find({hip_device, key});
@@ -183,8 +184,8 @@ int find_entry(const wgsl::Module &m, const std::string &name, wgsl::Stage stage
 }
 
 bool build_user_program(int hip_device, const wgsl::Module &vm, const std::string &vs_entry,
-                        const wgsl::Module *fm, const std::string &fs_entry, bool extended, UserProgram &out,
-                        std::string &err)
+                        const wgsl::Module *fm, const std::string &fs_entry, bool extended, const PipelineUses &uses,
+                        UserProgram &out, std::string &err)
 {
     int vi = find_entry(vm, vs_entry, wgsl::Stage::Vertex, err);
     if (vi < 0) return false;
@@ -382,38 +383,55 @@ bool build_user_program(int hip_device, const wgsl::Module &vm, const std::strin
     g += "}  // namespace wgc\n";
     // the glue follows the kernels: it uses their staged-triangle type
     std::string src = "#define WGC_USER_PROGRAM 1\n#include \"kernels_dev.h\"\n#include \"wgc_user.h\"\n";
-    std::vector<std::string> names = {
-        "wgc::k_setup<5, false>",          "wgc::k_setup<5, true>",
-        "wgc::k_clip<5, false>",           "wgc::k_clip<5, true>",
-        "wgc::k_tiles<5, false, 16, 256>", "wgc::k_tiles<5, true, 16, 256>",
-        "wgc::k_raster<5, false, 16, 256>", "wgc::k_raster<5, true, 16, 256>",
-        "wgc::k_setup<5, false, true>",
-        "wgc::k_point_visibility<5>",      "wgc::k_point_shade<5>",
-        "wgc::k_lp_prep<5, 1>",            "wgc::k_lp_prep<5, 2>",
-        "wgc::k_lp_tiles<5, 1, true>",     "wgc::k_lp_tiles<5, 2, true>",
-        "wgc::k_lp_tiles<5, 2, false>",
-    };
+    // the kernels the pipeline can reach (each costs compile time: all of
+    // them about a third more than those of one triangle pipeline)
+    UserKernels &k = out.kernels;
+    bool ordered = uses.ordered || out.discards || out.early_depth || out.frag_depth_tested;
+    bool free_order = !(out.discards || out.early_depth || out.frag_depth_tested);
+    std::vector<std::pair<std::string, hipFunction_t *>> want;
+    if (uses.triangles) {
+        want.insert(want.end(), {{"k_setup<5, false>", &k.setup[0]},
+                                 {"k_setup<5, true>", &k.setup[1]},
+                                 {"k_setup<5, false, true>", &k.setup_clip[0]},
+                                 {"k_setup<5, true, true>", &k.setup_clip[1]},
+                                 {"k_clip<5, false>", &k.clip[0]},
+                                 {"k_clip<5, true>", &k.clip[1]}});
+        if (free_order)
+            want.insert(want.end(), {{"k_tiles<5, false, 16, 256>", &k.tiles[0]},
+                                     {"k_tiles<5, true, 16, 256>", &k.tiles[1]},
+                                     {"k_tiles<5, false, 16, 256, true>", &k.tiles_merged}});
+        if (ordered)
+            want.insert(want.end(), {{"k_raster<5, false, 16, 256>", &k.raster[0]},
+                                     {"k_raster<5, true, 16, 256>", &k.raster[1]},
+                                     {"k_raster<5, false, 16, 256, true>", &k.raster_merged}});
+    }
+    if (uses.points) {
+        if (free_order)
+            want.insert(want.end(), {{"k_point_visibility<5>", &k.point_vis}, {"k_point_shade<5>", &k.point_shade}});
+        if (ordered)
+            want.insert(want.end(), {{"k_lp_prep<5, 1>", &k.lp_prep[0]}, {"k_lp_tiles<5, 1, true>", &k.lp_ordered[0]}});
+    }
+    if (uses.lines) {
+        want.push_back({"k_lp_prep<5, 2>", &k.lp_prep[1]});
+        if (free_order) want.push_back({"k_lp_tiles<5, 2, false>", &k.lp_tiles});
+        if (ordered) want.push_back({"k_lp_tiles<5, 2, true>", &k.lp_ordered[1]});
+    }
+    std::vector<std::string> names;
+    for (auto &w : want) names.push_back("wgc::" + w.first);
     Compiled c;
     if (!rtc_build(hip_device, src, {{"wgc_user.h", g}}, names, c, err)) return false;
     if (hip_device < 0) return true;
     out.code = c.code;
-    UserKernels &k = out.kernels;
     k.module = c.code->module;
+    for (size_t i = 0; i < want.size(); ++i) *want[i].second = c.fns[i];
+    auto occ = [](hipFunction_t f) { return f ? occupancy(f, 256) : 1u; };
     for (int m = 0; m < 2; ++m) {
-        k.setup[m] = c.fns[0 + m];
-        k.clip[m] = c.fns[2 + m];
-        k.tiles[m] = c.fns[4 + m];
-        k.raster[m] = c.fns[6 + m];
-        k.lp_prep[m] = c.fns[11 + m];
-        k.lp_ordered[m] = c.fns[13 + m];
-        k.occ_tiles[m] = occupancy(k.tiles[m], 256);
-        k.occ_raster[m] = occupancy(k.raster[m], 256);
+        k.occ_tiles[m] = occ(k.tiles[m]);
+        k.occ_raster[m] = occ(k.raster[m]);
+        k.occ_setup_clip[m] = occ(k.setup_clip[m]);
     }
-    k.setup_clip = c.fns[8];
-    k.point_vis = c.fns[9];
-    k.point_shade = c.fns[10];
-    k.lp_tiles = c.fns[15];
-    k.occ_setup_clip = occupancy(k.setup_clip, 256);
+    k.occ_tiles_merged = occ(k.tiles_merged);
+    k.occ_raster_merged = occ(k.raster_merged);
     return true;
 }
 

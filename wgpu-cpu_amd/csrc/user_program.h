@@ -39,14 +39,21 @@ struct UserProgram {
     uint32_t early_depth = 0;
 };
 
+// What a pipeline may draw: its primitives, and whether its state can make
+// a draw ordered (blending, NotEqual + write).  What the shaders make so
+// (discard, an early depth test, a tested frag_depth) is known from them.
+struct PipelineUses {
+    bool triangles = true, points = true, lines = true, ordered = true;
+};
+
 // Pairs a vertex entry point with an optional fragment entry point (entry
 // names may be empty: the module's only entry point of that stage), checks
-// the stage interface and compiles the kernels (hip_device < 0: compile
-// only, without loading).  `extended` allows the perspective interpolation
+// the stage interface and compiles the kernels that `uses` can reach
+// (hip_device < 0: compile only, without loading).  `extended` allows the perspective interpolation
 // the reference leaves as todo!().
 bool build_user_program(int hip_device, const wgsl::Module &vm, const std::string &vs_entry,
-                        const wgsl::Module *fm, const std::string &fs_entry, bool extended, UserProgram &out,
-                        std::string &err);
+                        const wgsl::Module *fm, const std::string &fs_entry, bool extended, const PipelineUses &uses,
+                        UserProgram &out, std::string &err);
 
 // Per invocation of an entry-point run: abort code, the position (vertex)
 // or frag depth (fragment), then 16 locations x 4 words of outputs.

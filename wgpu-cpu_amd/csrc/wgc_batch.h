@@ -10,9 +10,10 @@ namespace wgc {
 
 struct DrawParams;
 
-// Group-level arguments of every kernel: the table of independent draws
-// that share the launches (batched form; empty for a single draw passed by
-// value) and the group's tile bookkeeping.
+// Group-level arguments of every kernel: the table of draws that share the
+// launches (independent draws of the batched form, or consecutive draws of
+// one pass; empty for a single draw passed by value) and the group's tile
+// bookkeeping.
 struct BatchArgs {
     const DrawParams *draws;     // device array of n draws
     const uint32_t *prim_base;   // n + 1 prefix of primitives, padded to multiples of 64
@@ -26,7 +27,7 @@ struct BatchArgs {
     uint32_t *counters;          // C_NUM per draw
     uint32_t n_counters;
     uint32_t any_clear;          // the tile kernel stores LoadOp::Clear values into untouched tiles
-    uint32_t preclear;           // single draw: setup stores the LoadOp::Clear values into the whole target
+    uint32_t preclear;           // one target: setup stores the LoadOp::Clear values into the whole of it
     uint32_t pad;
 };
 

@@ -129,6 +129,8 @@ struct Scratch {
     unsigned long long *gvis;   // split tiles: the merged winners, TS*TS per tile (kept zero between uses)
     uint32_t *tile_done;     // split tiles: their items that have finished (zero region)
     uint32_t tile0;          // global index of the draw's first tile
+    uint32_t key_base;       // draws of one pass in one group: the first of this draw's primitives among
+                             // the group's (keys hold the group's primitive; 0 for other groups)
     uint32_t bin_cap;        // slots per tile bin
     uint32_t split;          // bin entries per work item of a tile (0: one item per tile)
     float split_inv;         // 1 / split

@@ -22,7 +22,8 @@ struct GroupLaunch {
     uint32_t *tile_count, *counters, *header;
     uint2 *clip_list;            // (draw, primitive) pairs that cross a clip plane
     uint32_t clip_cap;
-    uint32_t inline_clip;        // single draw whose setup waves all fit at once: setup clips
+    uint32_t merged;             // consecutive draws of one pass
+    uint32_t inline_clip;        // one target whose setup waves all fit at once: setup clips
     unsigned long long *vis;     // order-independent points: one visibility value per pixel
     void *lp;                    // lines and ordered points: a record per primitive (LpRec)
 };
@@ -95,8 +96,9 @@ struct UserKernels {
     hipFunction_t setup[2]{}, clip[2]{}, tiles[2]{}, raster[2]{};
     hipFunction_t point_vis{}, point_shade{};
     hipFunction_t lp_prep[2]{}, lp_ordered[2]{}, lp_tiles{};   // index: points 0, lines 1; lp_tiles: lines
-    hipFunction_t setup_clip{};   // single draws: setup that clips in place
-    uint32_t occ_tiles[2]{}, occ_raster[2]{}, occ_setup_clip{};
+    hipFunction_t setup_clip[2]{};   // setup that clips in place (0 single draw, 1 the draws of a pass)
+    hipFunction_t tiles_merged{}, raster_merged{};   // the draws of a pass
+    uint32_t occ_tiles[2]{}, occ_raster[2]{}, occ_setup_clip[2]{}, occ_tiles_merged{}, occ_raster_merged{};
 };
 
 // Launch group of a WGSL pipeline (16x16 tiles): the shader kernels from
@@ -108,17 +110,22 @@ hipError_t launch_user(const UserKernels &k, const DrawParams &d, const BatchArg
 hipError_t launch_lines(const DrawParams &d, const GroupLaunch &gl, hipStream_t st, KernelTimer *kt);
 
 // A single draw passes its parameters by value (b.draws unused, b.n == 1);
-// a batch passes the device table in b.draws (d0 unused).
+// a batch passes the device table in b.draws (d0 unused); the draws of a
+// pass (launch_merged) pass both, d0 being the first of them.
 hipError_t launch_draw(const DrawParams &d, const BatchArgs &b, const GroupLaunch &gl, hipStream_t st,
                        KernelTimer *kt);
 hipError_t launch_batch(const DrawParams &d0, const BatchArgs &b, const GroupLaunch &gl, hipStream_t st,
                         KernelTimer *kt);
+hipError_t launch_merged(const DrawParams &d0, const BatchArgs &b, const GroupLaunch &gl, hipStream_t st,
+                         KernelTimer *kt);
 // Workgroups of the raster kernel for (program, ordered, batched, tile
 // shape) that fit on one CU at once.
 uint32_t raster_blocks_per_cu(uint32_t program, bool ordered, bool multi, uint32_t cfg);
-// Workgroups per CU of the setup kernel that also clips (single draws of a
-// built-in program); 0 for other programs.
-uint32_t setup_clip_blocks_per_cu(uint32_t program);
+// The same for the draws of a pass (16x16 tiles).
+uint32_t merged_blocks_per_cu(uint32_t program, bool ordered);
+// Workgroups per CU of the setup kernel that also clips (a single draw, or
+// the draws of a pass, of a built-in program); 0 for other programs.
+uint32_t setup_clip_blocks_per_cu(uint32_t program, bool merged);
 // Zeroes the submission counters (fragment slots and error bits).
 hipError_t launch_reset(unsigned long long *frags, uint32_t *error, hipStream_t st);
 // Copies the submission counters to host memory (16 bytes, aligned: the
