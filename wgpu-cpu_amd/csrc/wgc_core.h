@@ -259,13 +259,12 @@ __device__ __forceinline__ uint32_t f32_as_u32(float f)
     return (uint32_t)f;
 }
 
-// texture.rs:376-379: (v * 255).clamp(0, 255) as u8
+// texture.rs:376-379: (v * 255).clamp(0, 255) as u8.  The maximum takes 0
+// for a NaN, which is what the conversion makes of it; two operations
+// instead of three compares and selects.
 __device__ __forceinline__ uint32_t f32_to_unorm8(float v)
 {
-    float x = v * 255.0f;
-    if (x < 0.0f) x = 0.0f;
-    if (x > 255.0f) x = 255.0f;
-    if (!(x == x)) return 0u;
+    float x = fminf(fmaxf(v * 255.0f, 0.0f), 255.0f);
     return (uint32_t)x;
 }
 
@@ -778,54 +777,50 @@ __device__ __forceinline__ void scan_cols(const ScanTri &s, int32_t &col0, int32
     else { col0 = min(min(s.ax, s.bx), s.cx); col1 = max(max(s.ax, s.bx), s.cx); }
 }
 
+// (num * i) / den truncated toward zero, for |num| < 2^15 and 0 <= i <= den
+// < 2^15, den > 0.  The quotient is at most |num|, so the binary32 estimate
+// (reciprocal within 1 ulp and two products: 2^-22 of it together) is within
+// one of it, and the remainder (24-bit products, full rate) says which way.
+// About half of what the general 32-bit division takes.  With the two edges
+// of scan_span chosen before they are divided: the tile kernel of 200k
+// overwriting triangles issues 40.5M instead of 49.6M VALU instructions, the
+// blending one 198M instead of 234M (the passes 183 -> 172 and 490 -> 445 us).
+__device__ __forceinline__ int32_t span_div(int32_t num, int32_t i, int32_t den)
+{
+    uint32_t n = (uint32_t)(num < 0 ? -num : num);
+    uint32_t q = (uint32_t)((float)n * ((float)i * __builtin_amdgcn_rcpf((float)den)));
+    int32_t r = (int32_t)(__umul24(n, (uint32_t)i) - __umul24(q, (uint32_t)den));
+    q = r < 0 ? q - 1u : (r >= den ? q + 1u : q);
+    return num < 0 ? -(int32_t)q : (int32_t)q;
+}
+
 // Inclusive span [x1, x2] of row y (scanline.rs:107-166).  Returns false
 // when the iterator emits no row y.  Rust's isize `/` truncates toward zero,
 // as does C++'s; products fit in 32 bits for coordinates below 2^15, and use
-// 64 bits above.
+// 64 bits above (`wide`).  Both edges of the row are chosen first and
+// divided after: lanes on rows of different kinds run two divisions, not
+// two per kind.
 __device__ __forceinline__ bool scan_span(const ScanTri &s, int32_t y, int32_t &x1, int32_t &x2, bool wide)
 {
+    // mode 0 is the one row a.y.  Else the long edge a-c, and a-b above b
+    // (mode 1 has no such rows) or b-c from b on (none when b is as low as c)
+    int32_t i = y - s.ay, acy = s.cy - s.ay;
+    bool upper = s.mode == 2 && y < s.by;
+    int32_t num = upper ? s.bx - s.ax : s.cx - s.bx, den = upper ? s.by - s.ay : s.cy - s.by;
+    int32_t i2 = upper ? i : y - s.by, from = upper ? s.ax : s.bx;
+    bool flat = s.mode == 0;
+    bool ok = flat ? i == 0 : (i >= 0 && i <= acy && den != 0);
+    if (!ok) return false;
     int32_t a, b;
-    if (s.mode == 0) {
-        if (y != s.ay) return false;
-        x1 = s.ax; x2 = s.cx;
-        return true;
-    }
-    int32_t acx = s.cx - s.ax, acy = s.cy - s.ay;
-    int32_t i = y - s.ay;
-    if (s.mode == 1) {
-        if (y < s.ay || y > s.cy) return false;
-        int32_t bcx = s.cx - s.bx, bcy = s.cy - s.by;
-        if (wide) {
-            a = s.ax + (int32_t)(((int64_t)acx * i) / acy);
-            b = s.bx + (int32_t)(((int64_t)bcx * i) / bcy);
-        } else {
-            a = s.ax + (acx * i) / acy;
-            b = s.bx + (bcx * i) / bcy;
-        }
+    if (flat) {
+        a = s.ax;
+        b = s.cx;
+    } else if (wide) {
+        a = s.ax + (int32_t)(((int64_t)(s.cx - s.ax) * i) / acy);
+        b = from + (int32_t)(((int64_t)num * i2) / den);
     } else {
-        if (y < s.ay) return false;
-        if (y < s.by) {
-            int32_t abx = s.bx - s.ax, aby = s.by - s.ay;
-            if (wide) {
-                a = s.ax + (int32_t)(((int64_t)acx * i) / acy);
-                b = s.ax + (int32_t)(((int64_t)abx * i) / aby);
-            } else {
-                a = s.ax + (acx * i) / acy;
-                b = s.ax + (abx * i) / aby;
-            }
-        } else {
-            int32_t bcy = s.cy - s.by;
-            if (bcy == 0 || y > s.cy) return false;
-            int32_t bcx = s.cx - s.bx;
-            int32_t i2 = y - s.by;
-            if (wide) {
-                a = s.ax + (int32_t)(((int64_t)acx * i) / acy);
-                b = s.bx + (int32_t)(((int64_t)bcx * i2) / bcy);
-            } else {
-                a = s.ax + (acx * i) / acy;
-                b = s.bx + (bcx * i2) / bcy;
-            }
-        }
+        a = s.ax + span_div(s.cx - s.ax, i, acy);
+        b = from + span_div(num, i2, den);
     }
     x1 = min(a, b);
     x2 = max(a, b);
