@@ -169,3 +169,57 @@ def test_ordered_tile_beyond_one_sort_batched(gpu_device_ext):
         want += ref.fragments
         assert_same(s, r, ref, per_pass_count=False)
     assert total == want
+
+
+# Single waves take the tiles of an ordered draw when more than four tiles
+# per resident workgroup are active (1024 workgroups here): a target of 4347
+# tiles, every one covered, with tiles past 64 keys and past 1024 fragments
+# (crowds, large triangles), triangles across the target's edge (clipped)
+# and beyond it, under every state that makes a draw ordered.
+@pytest.mark.parametrize("mode", ["blend", "blend_depth", "not_equal", "discard", "two_draws"])
+def test_ordered_tiles_by_single_waves(gpu_device, gpu_device_ext, mode):
+    w, h = 1103, 1005
+    flags = scenes.FS_DISCARD | scenes.FS_PRIM_RED if mode == "discard" else 0
+    n = 24000
+
+    def scene_draw(seed, count):
+        d = scenes.fragment_test_scene(flags, scenes.EARLY_NONE, compare=wgc.NOT_EQUAL, n=count, width=w, height=h,
+                                       seed=seed, alpha=(0.3, 0.9)).draws[0]
+        vb = np.frombuffer(d.vertex_data, np.float32).copy().reshape(count, 3, 8)
+        u = scenes.splitmix_f32(seed ^ 0x99, count * 2).reshape(count, 2)
+        size = np.where(np.arange(count) % 400 == 0, 300.0, np.where(np.arange(count) % 11 == 0, 60.0, 22.0))
+        for k in range(3):
+            ang = 2.1 * k + 6.28 * u[:, 0]
+            px = scenes.splitmix_f32(seed ^ 0x31, count) * (w + 30) - 15 + size * np.cos(ang)
+            py = scenes.splitmix_f32(seed ^ 0x77, count) * (h + 30) - 15 + size * np.sin(ang)
+            crowd = np.arange(count) % 90 == 7          # hundreds of small ones in a few tiles
+            px = np.where(crowd, 500.0 + 25 * u[:, 0] + 4 * np.cos(ang), px)
+            py = np.where(crowd, 400.0 + 25 * u[:, 1] + 4 * np.sin(ang), py)
+            vb[:, k, 0] = px / w * 2 - 1
+            vb[:, k, 1] = 1 - py / h * 2
+        d.vertex_data = vb.tobytes()
+        if not flags:
+            d.wgsl = None
+        return d
+
+    ext = mode in ("blend", "blend_depth", "two_draws")
+    draws = [scene_draw(8100, n)] if mode != "two_draws" else [scene_draw(8101, n // 2), scene_draw(8102, n // 2)]
+    depth = {"blend": None, "two_draws": None, "blend_depth": (wgc.LESS, False), "not_equal": (wgc.NOT_EQUAL, True),
+             "discard": (wgc.LESS_EQUAL, True)}[mode]
+    for d in draws:
+        d.depth = depth
+        d.blend = wgc.BLEND_ALPHA if ext else wgc.BLEND_REPLACE
+    spec = scenes.PassSpec(w, h, has_depth=depth is not None, clear_depth=0.6, draws=draws,
+                           semantics=wgc.SEMANTICS_EXTENDED if ext else wgc.SEMANTICS_REFERENCE,
+                           name=f"ordered tiles by single waves {mode}")
+    dev = gpu_device_ext if ext else gpu_device
+    # without per-pixel counts (with them the workgroup's form runs)
+    for s in (spec, scenes.as_wgsl(spec)) if mode in ("blend", "two_draws") else (spec,):
+        announce(s.name)
+        ref = bridge.render(s)
+        dev.enable_fragment_counts(0, 0)
+        got = runner.render(s, dev)
+        assert got.fragments == ref.fragments
+        assert np.array_equal(got.color, ref.color)
+        if depth is not None:
+            assert np.array_equal(got.depth.view(np.uint32), ref.depth.view(np.uint32))

@@ -1284,12 +1284,14 @@ __device__ __forceinline__ uint32_t tile_key_select(const DrawParams &d, const T
     return prefix;
 }
 
-// The wave's 64 values in ascending order of lanes (a bitonic network over
-// the lanes).
-__device__ __forceinline__ uint32_t sort_lanes(uint32_t v, uint32_t lane)
+// The values of the wave's first n lanes (the others at least as large as
+// any of them) in ascending order of lanes: a bitonic network over the
+// lanes, as far as n needs it.
+__device__ __forceinline__ uint32_t sort_lanes(uint32_t v, uint32_t lane, uint32_t n)
 {
 #pragma unroll
     for (uint32_t k = 2; k <= 64u; k <<= 1) {
+        if (k >= 2u * n) break;
 #pragma unroll
         for (uint32_t j = k >> 1; j > 0; j >>= 1) {
             uint32_t o = (uint32_t)__shfl_xor((int)v, (int)j);
@@ -1311,7 +1313,7 @@ __device__ __forceinline__ void sort_olist(uint32_t *olist, uint32_t total)
     uint32_t tid = threadIdx.x;
     if (total <= 64u) {
         if (tid < 64u) {
-            uint32_t v = sort_lanes(tid < total ? olist[tid] : 0xFFFFFFFFu, tid);
+            uint32_t v = sort_lanes(tid < total ? olist[tid] : 0xFFFFFFFFu, tid, total);
             if (tid < total) olist[tid] = v;
         }
         __syncthreads();
@@ -1462,6 +1464,258 @@ __device__ __forceinline__ void raster_tile(const DrawParams &d, const BatchArgs
         if (d.s.frag_px && nfrag[k]) d.s.frag_px[pix] += nfrag[k];
     });
     frag_acc += f;
+}
+
+// ------------------------------------------------------------------
+// ordered tiles of few fragments, one wave each
+// ------------------------------------------------------------------
+
+// A tile of at most 64 unclipped keys and about kLightFrags fragments is
+// taken by one wave, fragment by fragment: the keys sorted in registers, up
+// to kLightTris records at a time copied to LDS, a lane per covered row for
+// its span, the spans' pixels listed in order, then 64 fragments at a time
+// shaded side by side -- every lane has one -- and applied to the tile's
+// pixels in LDS, the lanes that hold the same pixel in turn, lowest (first
+// in API order) first.  The workgroup's form below runs the shader per
+// triangle and 16x4 strip of pixels, whatever part of the strip is covered:
+// on 200k blended triangles of about 75 pixels over 2560x2440 a fifth of its
+// lanes had a fragment, with the VALU busy 89% of the time.  Tiles of large
+// triangles fill those strips, and one wave alone would take longer over
+// them, so they stay there; so do clipped sub-triangles (their barycentrics
+// are not in the record), spilled and big triangles.
+constexpr uint32_t kLightTris = 24;
+constexpr uint32_t kLightFrags = 1024;
+constexpr uint32_t kLightStride = kRecWords + 1;   // odd: lanes reading different triangles meet different banks
+
+struct LightWave {
+    uint32_t rec[kLightTris * kLightStride];
+    uint16_t rows[kLightTris * 16];     // triangle | tile row << 8
+    uint16_t frag[kLightFrags];         // triangle | pixel of the tile << 8
+    uint32_t draw[kLightTris];          // draws of a pass: the triangle's
+    uint32_t claim[256];
+    uint32_t col[256];
+    float dep[256];
+};
+
+// A wave's LDS traffic is in program order; this keeps the compiler's so.
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// One fragment's source: barycentrics, depth and, for the built-in programs,
+// the shaded colour (the arithmetic of bary_depth and fragment_color on an
+// unclipped record).
+__device__ __forceinline__ void light_triangle(const uint32_t *r, TriLds &T)
+{
+    const float *f = reinterpret_cast<const float *>(r);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        T.vpx[k] = f[R_VP + 2 * k];
+        T.vpy[k] = f[R_VP + 2 * k + 1];
+        T.z[k] = f[R_Z + k];
+        T.iw[k] = f[R_IW + k];
+#pragma unroll
+        for (int c = 0; c < kMaxVar; ++c) T.var[k][c] = f[R_VAR + k * kMaxVar + c];
+    }
+    T.k0 = f[R_K + 0];
+    T.k1 = f[R_K + 1];
+    T.k2 = f[R_K + 2];
+    T.total = f[R_K + 3];
+    T.key = r[R_KEY];
+    T.ff = (r[R_MODE] >> 9) & 1u;
+}
+
+// bary_depth of an unclipped triangle.  The identity composition, lc[0] =
+// (1 l0 + 0 l1) + 0 l2 and so on, is l + (+0) bit for bit where every l is
+// finite and one of them positive (their sum says so): the other products
+// are zeros, of which one at least is +0 where an l of -0 meets them.
+__device__ __forceinline__ float light_depth(const TriLds &T, float pxf, float pyf, float lc[3])
+{
+    float l0 = (((T.vpy[1] - pyf) * (T.vpx[1] + pxf) + T.k0) + (pyf - T.vpy[2]) * (pxf + T.vpx[2])) / T.total;
+    float l1 = (((pyf - T.vpy[0]) * (pxf + T.vpx[0]) + (T.vpy[2] - pyf) * (T.vpx[2] + pxf)) + T.k1) / T.total;
+    float l2 = ((T.k2 + (pyf - T.vpy[1]) * (pxf + T.vpx[1])) + (T.vpy[0] - pyf) * (T.vpx[0] + pxf)) / T.total;
+    float s = (l0 + l1) + l2;
+    lc[0] = l0 + 0.0f;
+    lc[1] = l1 + 0.0f;
+    lc[2] = l2 + 0.0f;
+    if (!(s > 0.0f && s < __builtin_inff())) {
+        lc[0] = (1.0f * l0 + 0.0f * l1) + 0.0f * l2;
+        lc[1] = (0.0f * l0 + 1.0f * l1) + 0.0f * l2;
+        lc[2] = (0.0f * l0 + 0.0f * l1) + 1.0f * l2;
+    }
+    float z = T.z[0] * lc[0];
+    z = z + T.z[1] * lc[1];
+    z = z + T.z[2] * lc[2];
+    return z;
+}
+
+// Returns false, with nothing stored, when the tile is not one for a single
+// wave.  Every lane of the wave calls it with the same tile.
+template <int PROG, bool MERGED>
+__device__ __forceinline__ bool light_tile(const DrawParams &d, const BatchArgs &b, uint32_t tile, LightWave &w,
+                                           uint32_t &frag_acc)
+{
+    constexpr uint32_t TS = 16, PX = TS * TS;
+    uint32_t lane = lane_id();
+    uint32_t x0 = (tile % d.tiles_x) * TS, y0 = (tile / d.tiles_x) * TS;
+    uint32_t n = d.s.tile_count[tile];
+    if (n > 64u || n > d.s.bin_cap || d.s.frag_px || in_big_union(d, tile)) return false;
+    uint32_t key = lane < n ? d.s.bins[(size_t)tile * d.s.bin_cap + lane] : 0xFFFFFFFFu;
+    if (__ballot(lane < n && (key & 1u))) return false;
+    key = sort_lanes(key, lane, n);
+
+    // the tile's pixels
+#pragma unroll
+    for (uint32_t k = 0; k < PX / 64u; ++k) {
+        uint32_t q = lane + k * 64u, px = x0 + q % TS, py = y0 + q / TS;
+        size_t pix = (size_t)py * d.width + px;
+        bool in = px < d.width && py < d.height;
+        uint32_t c = d.clear_rgba;
+        float z = d.clear_depth;
+        if (in && d.color && !(d.init_clear && d.clear_color_on)) c = reinterpret_cast<const uint32_t *>(d.color)[pix];
+        if (in && d.depth && !(d.init_clear && d.clear_depth_on)) z = d.depth[pix];
+        w.col[q] = c;
+        w.dep[q] = z;
+        w.claim[q] = 0xFFFFFFFFu;
+    }
+    int32_t rx0 = (int32_t)max(x0, d.scissor[0]);
+    int32_t rx1 = (int32_t)(min((uint64_t)x0 + TS, (uint64_t)d.scissor[0] + d.scissor[2])) - 1;
+    int32_t ry0 = (int32_t)max(y0, d.scissor[1]);
+    int32_t ry1 = (int32_t)(min((uint64_t)y0 + TS, (uint64_t)d.scissor[1] + d.scissor[3])) - 1;
+    uint32_t frags = 0;
+    for (uint32_t t0 = 0; t0 < n; t0 += kLightTris) {
+        uint32_t nt = min(kLightTris, n - t0);
+        wave_sync();   // the records of the batch before have been read
+        // records: a lane per 16 bytes
+        constexpr uint32_t QUADS = kRecWords / 4;
+        for (uint32_t i = lane; i < ((nt * QUADS + 63u) & ~63u); i += 64u) {
+            uint32_t t = min(i / QUADS, nt - 1u), part = i % QUADS;
+            uint32_t k = (uint32_t)__shfl((int)key, (int)(t0 + t));
+            if (i < nt * QUADS) {
+                uint4 v = reinterpret_cast<const uint4 *>(d.s.tri + (size_t)(k >> 7) * kRecWords)[part];
+                uint32_t *o = w.rec + t * kLightStride + part * 4u;
+                o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+            }
+        }
+        if constexpr (MERGED) {
+            uint32_t k = (uint32_t)__shfl((int)key, (int)min(t0 + lane, 63u));
+            if (lane < nt) w.draw[lane] = b.wave_draw[k >> 13];
+        }
+        wave_sync();
+        // covered rows, in triangle order
+        uint32_t cnt = 0, first = 0;
+        if (lane < nt) {
+            const int32_t *r = reinterpret_cast<const int32_t *>(w.rec + lane * kLightStride);
+            ScanTri S{r[R_SCAN], r[R_SCAN + 1], r[R_SCAN + 2], r[R_SCAN + 3], r[R_SCAN + 4], r[R_SCAN + 5],
+                      r[R_MODE] & 0xFF, 0};
+            int32_t r0, r1;
+            scan_rows(S, r0, r1);
+            r0 = max(r0, ry0);
+            r1 = min(r1, ry1);
+            if (r0 <= r1) {
+                cnt = (uint32_t)(r1 - r0) + 1u;
+                first = (uint32_t)r0 - y0;
+            }
+        }
+        uint32_t sum = wave_inclusive_sum(cnt);
+        uint32_t rows = lane_value(sum, 63);
+        for (uint32_t j = 0; j < cnt; ++j) w.rows[sum - cnt + j] = (uint16_t)(lane | ((first + j) << 8));
+        wave_sync();
+        // their spans, and the pixels listed in order
+        uint32_t nf = 0;
+        for (uint32_t i0 = 0; i0 < rows; i0 += 64u) {
+            uint32_t len = 0, q0 = 0, t = 0;
+            if (i0 + lane < rows) {
+                uint32_t e = w.rows[i0 + lane];
+                t = e & 255u;
+                int32_t row = (int32_t)(e >> 8);
+                const int32_t *r = reinterpret_cast<const int32_t *>(w.rec + t * kLightStride);
+                ScanTri S{r[R_SCAN], r[R_SCAN + 1], r[R_SCAN + 2], r[R_SCAN + 3], r[R_SCAN + 4], r[R_SCAN + 5],
+                          r[R_MODE] & 0xFF, 0};
+                int32_t a, c;
+                if (scan_span(S, (int32_t)y0 + row, a, c, ((r[R_MODE] >> 8) & 1) != 0)) {
+                    a = max(a, rx0);
+                    c = min(c, rx1);
+                    if (a <= c) {
+                        len = (uint32_t)(c - a) + 1u;
+                        q0 = (uint32_t)row * TS + ((uint32_t)a - x0);
+                    }
+                }
+            }
+            uint32_t end = wave_inclusive_sum(len), total = lane_value(end, 63);
+            if (nf + total > kLightFrags) return false;
+            uint32_t o = nf + end - len;
+            for (uint32_t j = 0; j < len; ++j) w.frag[o + j] = (uint16_t)(t | ((q0 + j) << 8));
+            nf += total;
+        }
+        // (the first batch stands for the others)
+        if (t0 == 0u && nf * n > 3u * kLightFrags / 2u * nt) return false;
+        frags += nf;
+        wave_sync();
+        for (uint32_t f0 = 0; f0 < nf; f0 += 64u) {
+            bool pending = f0 + lane < nf;
+            uint32_t e = pending ? w.frag[f0 + lane] : 0u;
+            uint32_t t = e & 255u, q = e >> 8;
+            TriLds T;
+            light_triangle(w.rec + t * kLightStride, T);
+            float lc[3], color[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            float z = light_depth(T, (float)(x0 + q % TS), (float)(y0 + q / TS), lc);
+            // the shader of the fragment's draw: draws of a pass one after
+            // the other, the lanes of each together
+            auto shade = [&](float *frag_depth) {
+                bool ok = false;
+                if constexpr (MERGED) {
+                    uint32_t di = w.draw[t];
+                    for (;;) {
+                        uint32_t u = __builtin_amdgcn_readfirstlane(di);
+                        if (di == u) {
+                            ok = fragment_color<PROG>(b.draws[u], T, lc, color, d.srgb_lut, frag_depth);
+                            break;
+                        }
+                    }
+                } else {
+                    ok = fragment_color<PROG>(d, T, lc, color, d.srgb_lut, frag_depth);
+                }
+                return ok;
+            };
+            if constexpr (PROG != PROG_USER) {
+                // no side effects, no discard: once for all rounds
+                float unused = z;
+                (void)shade(&unused);
+            }
+            while (__ballot(pending)) {
+                if (pending) atomicMin(&w.claim[q], lane);
+                wave_sync();
+                if (pending && w.claim[q] == lane) {
+                    float dz = d.depth_test ? w.dep[q] : 0.0f;
+                    bool ok = depth_and_shade(d, z, dz, [&](float *frag_depth) {
+                        if constexpr (PROG == PROG_USER) return shade(frag_depth);
+                        else return true;
+                    });
+                    if (d.depth_test && d.depth_write) w.dep[q] = dz;
+                    if (ok)
+                        w.col[q] = d.blend ? blend_over(color, w.col[q], d.color_bgra) : pack_color(color, d.color_bgra);
+                    w.claim[q] = 0xFFFFFFFFu;
+                    pending = false;
+                }
+                wave_sync();
+            }
+        }
+    }
+    wave_sync();
+#pragma unroll
+    for (uint32_t k = 0; k < PX / 64u; ++k) {
+        uint32_t q = lane + k * 64u, px = x0 + q % TS, py = y0 + q / TS;
+        if (px >= d.width || py >= d.height) continue;
+        size_t pix = (size_t)py * d.width + px;
+        if (d.color) store_color(d, pix, w.col[q]);
+        if (d.depth) store_depth(d, pix, w.dep[q]);
+    }
+    if (lane == 0u) frag_acc += frags;
+    return true;
 }
 
 // What the visibility pass needs of a triangle: its record without the
@@ -1960,48 +2214,84 @@ __device__ __forceinline__ void count_fragments(const DrawParams &d0, const Batc
     }
 }
 
-// Ordered draws (blending, NotEqual + write): persistent and statically
-// scheduled (no shared work counter); each tile's fragments are applied in
-// API order.  First the active tiles, then the untouched ones in chunks,
-// strided over the whole grid.
+// Ordered draws (blending, NotEqual + write), persistent: each tile's
+// fragments are applied in API order.  Work items are entries of the active
+// list, or four of them: a wave takes each if it can (light_tile), and the
+// workgroup the ones it could not, together.  Then the untouched tiles in
+// chunks, strided over the whole grid.
 // MERGED: consecutive draws of one pass (d0 the first of them), one list of
 // tiles for all.
+// 200k blended triangles over 2560x2440, the pass: 446 us with a workgroup
+// per tile, 312 with its light tiles by single waves (247 of them this
+// kernel, VALU instructions 198M -> 90M); 100k over 1280x720 (3600 tiles)
+// 290 either way, so short lists stay with workgroups.
 template <int PROG, bool MULTI, int TS, int NT, bool MERGED = false>
-__global__ __launch_bounds__(NT) void k_raster(DrawParams d0, BatchArgs b)
+__global__ __launch_bounds__(NT, 4) void k_raster(DrawParams d0, BatchArgs b)
 {
     constexpr int PPT = TS * TS / NT;
-    static_assert(NT >= kBatch && PPT >= 1 && TS * TS == PPT * NT, "tile shape");
-    __shared__ RasterShared<TS> sh;
-    __shared__ uint32_t olist[kOrderedCap];
+    constexpr uint32_t WAVES = NT / 64;
+    static_assert(NT >= kBatch && PPT >= 1 && TS * TS == PPT * NT && TS == 16, "tile shape");
+    struct Together {
+        RasterShared<TS> sh;
+        uint32_t olist[kOrderedCap];
+    };
+    __shared__ union {
+        Together together;
+        LightWave light[WAVES];
+    } u;
     __shared__ uint32_t olist_n;
     __shared__ uint32_t ticket;
+    __shared__ uint32_t heavy[WAVES];
     __shared__ uint32_t wave_frags[NT / 64];
     __shared__ uint32_t kinds[kClearChunk];
 
     ActiveSchedule w(b);
     uint32_t frag_acc = 0;
+    // with more than four entries per workgroup, items of four, a wave each;
+    // with fewer, a tile's waves work on it together (256x256, 5000 blended
+    // triangles: 86 us a pass, by single waves 201)
+    uint32_t entries = w.n;
+    bool waves = entries > WAVES * gridDim.x;
+    if (waves) w.n = (entries + WAVES - 1u) / WAVES;
+    uint32_t wave = threadIdx.x >> 6;
     bool dyn = w.dynamic();
     uint32_t raw = w.e0;
     for (uint32_t item = w.first; item < w.n;) {
-        uint32_t e = __builtin_amdgcn_readfirstlane(raw);
         // the ticket of this workgroup's next item, taken while this one is
         // processed (thread 0 takes it, the workgroup reads it after)
         uint32_t tk = 0u;
         if (dyn && threadIdx.x == 0) tk = atomicAdd(w.queue(b), 1u);
         uint32_t di, tile, it;
-        locate_tile<MULTI>(d0, b, e, di, tile, it);
-        raster_tile<PROG, TS, NT, MERGED>(draw_at<MULTI>(d0, b, di), b, tile, sh, olist, olist_n, frag_acc);
+        if (waves) {
+            uint32_t at = __builtin_amdgcn_readfirstlane(item * WAVES + wave);
+            uint32_t mine = 0xFFFFFFFFu;   // this wave's entry, when the workgroup has to take it
+            if (at < entries) {
+                uint32_t e = __builtin_amdgcn_readfirstlane(b.active_list[at]);
+                locate_tile<MULTI>(d0, b, e, di, tile, it);
+                if (!light_tile<PROG, MERGED>(draw_at<MULTI>(d0, b, di), b, tile, u.light[wave], frag_acc)) mine = e;
+            }
+            if (lane_id() == 0u) heavy[wave] = mine;
+            __syncthreads();
+        }
+        for (uint32_t k = 0; k < (waves ? WAVES : 1u); ++k) {
+            uint32_t e = __builtin_amdgcn_readfirstlane(waves ? heavy[k] : raw);
+            if (waves && e == 0xFFFFFFFFu) continue;
+            locate_tile<MULTI>(d0, b, e, di, tile, it);
+            raster_tile<PROG, TS, NT, MERGED>(draw_at<MULTI>(d0, b, di), b, tile, u.together.sh, u.together.olist,
+                                              olist_n, frag_acc);
+        }
         if (!dyn) break;
         if (threadIdx.x == 0) ticket = tk;
-        __syncthreads();
+        __syncthreads();   // (and every thread has read heavy)
         item = w.index_of(ticket);
-        raw = w.load(b, item);
+        if (!waves) raw = w.load(b, item);
     }
+    __syncthreads();
     // workgroups late in the schedule have the fewest active tiles: chunks from there
     if (untouched_pass(b))
         for (uint32_t c = gridDim.x - 1u - w.first; c < b.n_chunks; c += gridDim.x)
             untouched_chunk<MULTI, TS, NT>(d0, b, c, kinds, [&](const DrawParams &d, uint32_t tile) {
-                raster_tile<PROG, TS, NT, MERGED>(d, b, tile, sh, olist, olist_n, frag_acc);
+                raster_tile<PROG, TS, NT, MERGED>(d, b, tile, u.together.sh, u.together.olist, olist_n, frag_acc);
             });
     count_fragments<MULTI, NT>(d0, b, frag_acc, wave_frags);
 }
@@ -2464,7 +2754,7 @@ __device__ __forceinline__ void sort_wave(uint32_t *list, uint32_t total)
     uint32_t lane = threadIdx.x;
     if (total <= 64u) {
         uint32_t v = lane < total ? list[lane] : 0xFFFFFFFFu;
-        v = sort_lanes(v, lane);
+        v = sort_lanes(v, lane, total);
         if (lane < total) list[lane] = v;
         __syncthreads();
         return;
