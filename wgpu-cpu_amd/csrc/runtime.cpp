@@ -14,12 +14,14 @@
 #include <cstddef>
 #include <cstdio>
 #include <cstring>
+#include <deque>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
 #include <tuple>
+#include <unordered_map>
 #include <vector>
 
 #include "../../include/wgc.h"
@@ -423,6 +425,8 @@ struct Step {
     uint32_t rows = 0;
 };
 
+struct Lane;
+
 struct Plan {
     WgcDevice_T *dev = nullptr;      // set (and retained) while the plan holds pooled memory or a graph
     uint64_t arena_gen = UINT64_MAX;
@@ -447,13 +451,15 @@ struct Plan {
 
 struct WgcCommandBuffer_T : Object {
     std::vector<PassCommand> passes;
-    std::unique_ptr<Plan> plan{new Plan()};  // launch plan cached for resubmission
+    std::unique_ptr<Plan> plans[2]{std::unique_ptr<Plan>(new Plan()), std::unique_ptr<Plan>(new Plan())};  // launch
+                                             // plans cached for resubmission, one per lane it ran on
+    bool lane0 = false;                      // no room for it on lane 1
     // the same passes laid out in the static scratch, for the allocation-free
     // submission (built on its first use)
     std::unique_ptr<Plan> plan_noalloc{new Plan()};
     ~WgcCommandBuffer_T() override
     {
-        plan.reset();
+        for (auto &p : plans) p.reset();
         plan_noalloc.reset();
         for (auto &p : passes) p.drop();
     }
@@ -488,8 +494,38 @@ struct HostCounters {
     uint32_t pad2[12];
 };
 
+// What a submission runs on: a stream, the scratch arena its plans are laid
+// out in, and its counters.  Lane 0 is the device's own stream, with every
+// transfer, fill and timestamp; lane 1 takes single render passes that may
+// run beside what lane 0 executes (choose_lane).
+struct Lane {
+    hipStream_t stream = nullptr;
+    // per-draw scratch arena, reused by every draw (they run in stream order);
+    // its first zone_size bytes are zero when a plan starts (the kernel that
+    // ends a submission clears what the submission's plan used there)
+    uint8_t *arena = nullptr;
+    size_t arena_size = 0;
+    size_t zone_size = 0;
+    size_t keep_size = 0;   // then keep_size bytes that every use leaves zero (split-tile winners)
+    uint64_t arena_gen = 0; // bumped whenever memory a cached plan points at moves
+    DevCounters *d_counters = nullptr;
+    bool counters_dirty = false;            // a submission stopped before taking its counters
+    uint32_t *d_error = nullptr;            // &d_counters->error
+    unsigned long long *d_frags = nullptr;  // d_counters->frags
+    uint64_t last = 0;      // index of the last submission on this lane
+    uint32_t queued = 0;    // submissions on this lane that have not retired
+    // per resource, the last submissions on this lane that wrote and read it
+    // (entries of retired ones are dropped now and then; a stale one of a
+    // freed object can only make a later submission wait)
+    struct Use {
+        uint64_t wrote = 0, read = 0;
+    };
+    std::unordered_map<const void *, Use> uses;
+};
+
 struct Inflight {
     uint64_t index;
+    uint32_t lane;
     hipEvent_t done;
     std::vector<Object *> keep;  // command buffers used by the submission
     HostCounters *slot;          // pinned host copy of the counters
@@ -522,22 +558,15 @@ struct WgcDevice_T : Object {
     hipStream_t side = nullptr;     // second stream for the independent groups of a stage
     hipEvent_t fork = nullptr, join = nullptr;
     std::mutex mu;
-    // per-draw scratch arena, reused by every draw (they run in stream order);
-    // its first zone_size bytes are zero when a plan starts (the kernel that
-    // ends a submission clears what the submission's plan used there)
-    uint8_t *arena = nullptr;
-    size_t arena_size = 0;
-    size_t zone_size = 0;
-    size_t keep_size = 0;   // then keep_size bytes that every use leaves zero (split-tile winners)
-    // persistent device words
-    DevCounters *d_counters = nullptr;
-    bool counters_dirty = false;            // a submission stopped before taking its counters
-    uint32_t *d_error = nullptr;            // &d_counters->error
-    unsigned long long *d_frags = nullptr;  // d_counters->frags
+    Lane lanes[2];                  // lanes[0].stream == stream
+    hipEvent_t mark = nullptr;      // lane 1 starts after what lane 0 held then
+    uint64_t main_ops = 0;          // transfers, fills and timestamps on lane 0 so far; their number
+    uint64_t ops_lane1 = 0;         // when lane 1 was last made to wait for them, and
+    uint64_t ops_last = 0;          // at the last submission
     float *d_srgb = nullptr;
     uint64_t next_index = 1;
     uint64_t last_done = 0;
-    std::vector<Inflight> inflight;
+    std::deque<Inflight> inflight;
     std::vector<hipEvent_t> event_pool;
     std::vector<HostCounters *> slot_pool;   // free pinned counter slots
     std::vector<HostCounters *> slot_blocks;
@@ -558,7 +587,6 @@ struct WgcDevice_T : Object {
     KernelTimer timer;
     std::map<std::string, std::pair<double, uint64_t>> ktimes;
     uint64_t last_prims = 0, last_launches = 0;
-    uint64_t arena_gen = 0;        // bumped whenever memory a cached plan points at moves
     uint32_t cu_count = 256;        // compute units of the device
     uint32_t raster_cfg = RASTER_16x16_256;
     bool batching = true;          // merge independent single-draw passes into launch groups
@@ -574,7 +602,8 @@ struct WgcDevice_T : Object {
     ~WgcDevice_T() override
     {
         (void)hipSetDevice(hip_device);
-        if (stream) (void)hipStreamSynchronize(stream);
+        for (auto &l : lanes)
+            if (l.stream) (void)hipStreamSynchronize(l.stream);
         for (auto &f : inflight) {
             (void)hipEventDestroy(f.done);
             for (auto *o : f.keep) release(o);
@@ -595,8 +624,12 @@ struct WgcDevice_T : Object {
             (void)hipEventDestroy(p.end);
         }
         for (auto e : timer.pool) (void)hipEventDestroy(e);
-        if (arena) (void)hipFree(arena);
-        if (d_counters) (void)hipFree(d_counters);
+        for (auto &l : lanes) {
+            if (l.arena) (void)hipFree(l.arena);
+            if (l.d_counters) (void)hipFree(l.d_counters);
+        }
+        if (mark) (void)hipEventDestroy(mark);
+        if (lanes[1].stream) (void)hipStreamDestroy(lanes[1].stream);
         if (d_srgb) (void)hipFree(d_srgb);
         if (frag_px) (void)hipFree(frag_px);
         for (auto *b : pending_maps) release(b);
@@ -717,6 +750,9 @@ extern "C" int32_t wgc_device_create(const WgcDeviceDescriptor *desc, WgcDevice 
     hipError_t e = hipSetDevice(d->hip_device);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&d->lanes[1].stream, hipStreamNonBlocking);
+    d->lanes[0].stream = d->stream;
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&d->mark, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&d->fork, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&d->join, hipEventDisableTiming);
     if (e == hipSuccess) {
@@ -725,12 +761,15 @@ extern "C" int32_t wgc_device_create(const WgcDeviceDescriptor *desc, WgcDevice 
         if (e == hipSuccess && cus > 0) d->cu_count = (uint32_t)cus;
     }
     if (e == hipSuccess) e = scratch_address(d->hip_device, d->scratch);
-    if (e == hipSuccess) e = hipMalloc(&d->d_counters, sizeof(DevCounters));
     if (e == hipSuccess) e = hipMalloc(&d->d_srgb, 256 * sizeof(float));
-    if (e == hipSuccess) e = stream_zero(d->stream, d->d_counters, sizeof(DevCounters));
+    for (auto &l : d->lanes) {
+        if (e == hipSuccess) e = hipMalloc(&l.d_counters, sizeof(DevCounters));
+        if (e == hipSuccess) e = stream_zero(d->stream, l.d_counters, sizeof(DevCounters));
+        if (e != hipSuccess) break;
+        l.d_error = &l.d_counters->error;
+        l.d_frags = l.d_counters->frags;
+    }
     if (e == hipSuccess) {
-        d->d_error = &d->d_counters->error;
-        d->d_frags = d->d_counters->frags;
         d->table_pool.block_size = 16ull << 20;
         d->staging_pool.pinned = true;
         d->staging_pool.block_size = 16ull << 20;
@@ -819,8 +858,9 @@ static int32_t retire(WgcDevice_T *d, uint64_t upto, bool wait, uint64_t timeout
         d->last_prims = f.prims;
         d->last_launches = f.launches;
         d->slot_pool.push_back(f.slot);
+        d->lanes[f.lane].queued--;
         std::vector<Object *> keep = std::move(f.keep);
-        d->inflight.erase(d->inflight.begin());
+        d->inflight.pop_front();
         for (auto *o : keep) release(o);  // may reset plans, which defer their memory
     }
     // memory whose last reader has executed goes back to its pool, and
@@ -837,6 +877,31 @@ static int32_t retire(WgcDevice_T *d, uint64_t upto, bool wait, uint64_t timeout
         }
     }
     return WGC_OK;
+}
+
+// ---- the lanes ----
+
+// Makes `stream` wait for submission `index` of the other lane, if it has
+// not retired.  The queue holds consecutive submissions.
+static hipError_t wait_for(WgcDevice_T *d, hipStream_t stream, uint64_t index)
+{
+    if (d->inflight.empty() || index < d->inflight.front().index) return hipSuccess;
+    return hipStreamWaitEvent(stream, d->inflight[index - d->inflight.front().index].done, 0);
+}
+
+// Before work of its own goes to lane 0 (a transfer, a timestamp): lane 1's
+// submissions so far come first -- those that use `resource`, or with none
+// all of them -- and lane 1's later ones after it (choose_lane).
+static hipError_t before_main_op(WgcDevice_T *d, const void *resource = nullptr)
+{
+    d->main_ops++;
+    const Lane &l = d->lanes[1];
+    uint64_t index = l.last;
+    if (resource) {
+        auto it = l.uses.find(resource);
+        index = it == l.uses.end() ? 0 : std::max(it->second.wrote, it->second.read);
+    }
+    return wait_for(d, d->stream, index);
 }
 
 static int32_t resolve_timers(WgcDevice_T *d)
@@ -951,7 +1016,7 @@ extern "C" int32_t wgc_device_debug_fragment_counts(WgcDevice device, uint32_t w
         HIP_TRY(stream_copy(device->stream, host_out, device->frag_px, need, hipMemcpyDeviceToHost), "readback");
         return WGC_OK;
     }
-    device->arena_gen++;  // cached plans point at the counts buffer
+    for (auto &l : device->lanes) l.arena_gen++;  // cached plans point at the counts buffer
     if (device->frag_px) {
         HIP_TRY(hipFree(device->frag_px), "hipFree");
         device->frag_px = nullptr;
@@ -981,7 +1046,8 @@ extern "C" int32_t wgc_buffer_create(WgcDevice device, uint64_t size, WgcBuffer 
         hipError_t e = hipMalloc(&b->ptr, size);
         if (e == hipSuccess) {
             std::lock_guard<std::mutex> lk(device->mu);
-            e = stream_zero_async(device->stream, b->ptr, size);
+            e = before_main_op(device, b);
+            if (e == hipSuccess) e = stream_zero_async(device->stream, b->ptr, size);
         }
         if (e != hipSuccess) {
             release(b);
@@ -1025,6 +1091,7 @@ extern "C" int32_t wgc_queue_write_buffer(WgcDevice device, WgcBuffer buffer, ui
     if (!size) return WGC_OK;
     std::lock_guard<std::mutex> lk(device->mu);
     HIP_TRY(hipSetDevice(device->hip_device), "hipSetDevice");
+    HIP_TRY(before_main_op(device, buffer), "write_buffer");
     HIP_TRY(staged_upload(device, buffer->ptr + offset, data, size), "write_buffer");
     return WGC_OK;
 }
@@ -1060,6 +1127,7 @@ extern "C" int32_t wgc_buffer_map_async(WgcBuffer buffer, uint32_t mode, uint64_
     MapState &m = buffer->map;
     if (size) HIP_TRY(hipHostMalloc((void **)&m.host, size, hipHostMallocDefault), "map staging");
     hipError_t e = hipEventCreateWithFlags(&m.done, hipEventDisableTiming);
+    if (e == hipSuccess) e = before_main_op(d, buffer);
     // a write mapping starts from the buffer's contents as well
     if (e == hipSuccess && size) e = hipMemcpyAsync(m.host, buffer->ptr + offset, size, hipMemcpyDeviceToHost, d->stream);
     if (e == hipSuccess) e = hipEventRecord(m.done, d->stream);
@@ -1115,6 +1183,7 @@ extern "C" int32_t wgc_buffer_unmap(WgcBuffer buffer)
             (void)hipEventSynchronize(m.done);
         } else if (m.mode == WGC_MAP_WRITE && m.size) {
             // the written bytes go back to the buffer, ordered before later submissions
+            HIP_TRY(before_main_op(d, buffer), "unmap");
             HIP_TRY(stream_copy(d->stream, buffer->ptr + m.offset, m.host, m.size, hipMemcpyHostToDevice), "unmap");
         }
         (void)hipEventDestroy(m.done);
@@ -1182,7 +1251,8 @@ extern "C" int32_t wgc_texture_create(WgcDevice device, uint32_t width, uint32_t
     hipError_t e = hipMalloc(&t->ptr, t->size);
     if (e == hipSuccess) {
         std::lock_guard<std::mutex> lk(device->mu);
-        e = stream_zero_async(device->stream, t->ptr, t->size);
+        e = before_main_op(device, t);
+        if (e == hipSuccess) e = stream_zero_async(device->stream, t->ptr, t->size);
     }
     if (e != hipSuccess) {
         release(t);
@@ -1255,7 +1325,8 @@ extern "C" int32_t wgc_buffer_create_in_heap(WgcHeap heap, uint64_t size, WgcBuf
     b->size = size;
     std::lock_guard<std::mutex> lk(device->mu);
     HIP_TRY(hipSetDevice(device->hip_device), "hipSetDevice");
-    hipError_t e = stream_zero_async(device->stream, ptr, size);
+    hipError_t e = before_main_op(device, b);
+    if (e == hipSuccess) e = stream_zero_async(device->stream, ptr, size);
     if (e != hipSuccess) {
         release(b);
         return hip_fail(e, "buffer zero fill");
@@ -1289,7 +1360,8 @@ extern "C" int32_t wgc_texture_create_in_heap(WgcHeap heap, uint32_t width, uint
     t->size = size;
     std::lock_guard<std::mutex> lk(device->mu);
     HIP_TRY(hipSetDevice(device->hip_device), "hipSetDevice");
-    hipError_t e = stream_zero_async(device->stream, ptr, size);
+    hipError_t e = before_main_op(device, t);
+    if (e == hipSuccess) e = stream_zero_async(device->stream, ptr, size);
     if (e != hipSuccess) {
         release(t);
         return hip_fail(e, "texture zero fill");
@@ -1312,6 +1384,7 @@ extern "C" int32_t wgc_queue_write_texture(WgcDevice device, WgcTexture texture,
         return set_error(WGC_ERR_INVALID, "write_texture past the texture (reference: slice panic)");
     std::lock_guard<std::mutex> lk(device->mu);
     HIP_TRY(hipSetDevice(device->hip_device), "hipSetDevice");
+    HIP_TRY(before_main_op(device, texture), "write_texture");
     HIP_TRY(staged_upload(device, texture->ptr, (const uint8_t *)data + offset, n), "write_texture");
     return WGC_OK;
 }
@@ -2297,7 +2370,7 @@ static uint64_t line_bin_cap(const DrawParams &d)
 // set-up primitives and the tiles' bins.  `zone`: the tile counts (all
 // point / line steps of a plan share them: each tile kernel leaves them zero).
 static size_t layout_lines(Step &st, uint8_t *base, uint8_t *zone, uint32_t *frag_px, size_t frag_px_size,
-                           WgcDevice_T *dev)
+                           const Lane &lane)
 {
     DrawParams &d = st.draws[0];
     bool tiled = tiled_lines(d);
@@ -2311,8 +2384,8 @@ static size_t layout_lines(Step &st, uint8_t *base, uint8_t *zone, uint32_t *fra
     d.s.bins = tiled ? (uint32_t *)(base + rec) : nullptr;
     d.s.bin_cap = (uint32_t)cap;
     d.s.tile_count = (uint32_t *)zone;
-    d.s.frags = dev->d_frags;
-    d.s.error = dev->d_error;
+    d.s.frags = lane.d_frags;
+    d.s.error = lane.d_error;
     d.s.frag_px = (frag_px && frag_px_size == (size_t)d.width * d.height * 4u) ? frag_px : nullptr;
     return bytes;
 }
@@ -2365,7 +2438,7 @@ static uint32_t split_for(const Step &st)
 }
 
 static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep, uint32_t *frag_px,
-                           size_t frag_px_size, WgcDevice_T *dev)
+                           size_t frag_px_size, WgcDevice_T *dev, const Lane &lane)
 {
     // one unit of tiles, bins, records and counters per target
     uint32_t n = (uint32_t)group_targets(st);
@@ -2514,8 +2587,8 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
         if (st.merged) prim_base += group_prims(st, d);
         s.strip_sep = restart_strip(d) ? (int32_t *)(base + o_ss[i]) : nullptr;
         s.counters = gl.counters + C_NUM * i;
-        s.frags = dev->d_frags;
-        s.error = dev->d_error;
+        s.frags = lane.d_frags;
+        s.error = lane.d_error;
         // debug counts are only written when they were sized for this pass
         s.frag_px = (frag_px && frag_px_size == (size_t)d.width * d.height * 4u) ? frag_px : nullptr;
         s.tile0 = (uint32_t)tile_base;
@@ -2708,7 +2781,12 @@ static void copy_step(const PassCommand &pc, Step &s)
     }
 }
 
-static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, bool noalloc)
+// Lane 1's arena at most, and build_plan's answer where a plan does not get
+// one there (it runs on lane 0 then).
+static constexpr size_t kLane1Arena = 2ull << 30;
+static constexpr int32_t kNoLane1 = 1;
+
+static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, Plan &plan, bool noalloc)
 {
     plan.reset();
     plan.noalloc = noalloc;
@@ -2848,8 +2926,8 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
         s.arena_off = stage_off;
         s.zone_off = zneed;
         s.keep_off = kneed;
-        size_t bytes = s.kind == StepKind::Lines ? layout_lines(s, nullptr, nullptr, nullptr, 0, dev)
-                                                  : layout_group(s, nullptr, nullptr, nullptr, nullptr, 0, dev);
+        size_t bytes = s.kind == StepKind::Lines ? layout_lines(s, nullptr, nullptr, nullptr, 0, lane)
+                                                  : layout_group(s, nullptr, nullptr, nullptr, nullptr, 0, dev, lane);
         stage_off = align_up(stage_off + bytes, 256);
         need = std::max(need, stage_off);
         if (s.kind == StepKind::Lines && tiled_lines(s.draws[0]))
@@ -2886,29 +2964,33 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
         zone_base = dev->scratch;
         keep_base = dev->scratch + zone;
         arena_base = dev->scratch + zone + keep;
-    } else if (zneed > dev->zone_size || kneed > dev->keep_size ||
-        dev->zone_size + dev->keep_size + need > dev->arena_size) {
-        HIP_TRY(hipStreamSynchronize(dev->stream), "arena");
-        if (dev->arena) HIP_TRY(hipFree(dev->arena), "arena");
-        dev->arena = nullptr;
-        dev->arena_size = 0;
-        size_t zone = align_up(std::max(zneed, dev->zone_size), 4096);
-        size_t keep = align_up(std::max(kneed, dev->keep_size), 4096);
+    } else if (zneed > lane.zone_size || kneed > lane.keep_size ||
+               lane.zone_size + lane.keep_size + need > lane.arena_size) {
+        size_t zone = align_up(std::max(zneed, lane.zone_size), 4096);
+        size_t keep = align_up(std::max(kneed, lane.keep_size), 4096);
         size_t grow = zone + keep + std::max(need, (size_t)64 << 20);
-        if (hipMalloc(&dev->arena, grow) != hipSuccess) {
-            dev->zone_size = dev->keep_size = 0;
+        if (&lane != &dev->lanes[0] && grow > kLane1Arena) return kNoLane1;
+        HIP_TRY(hipStreamSynchronize(lane.stream), "arena");
+        if (lane.arena) HIP_TRY(hipFree(lane.arena), "arena");
+        lane.arena = nullptr;
+        lane.arena_size = 0;
+        lane.arena_gen++;   // (also when the allocation fails: the old arena is gone)
+        if (hipMalloc(&lane.arena, grow) != hipSuccess) {
+            lane.arena = nullptr;
+            lane.zone_size = lane.keep_size = 0;
+            (void)hipGetLastError();
+            if (&lane != &dev->lanes[0]) return kNoLane1;
             return set_error(WGC_ERR_OUT_OF_MEMORY, "scratch arena");
         }
-        HIP_TRY(hipMemsetAsync(dev->arena, 0, zone + keep, dev->stream), "arena zero regions");
-        dev->arena_size = grow;
-        dev->zone_size = zone;
-        dev->keep_size = keep;
-        dev->arena_gen++;
+        HIP_TRY(hipMemsetAsync(lane.arena, 0, zone + keep, lane.stream), "arena zero regions");
+        lane.arena_size = grow;
+        lane.zone_size = zone;
+        lane.keep_size = keep;
     }
     if (!noalloc) {
-        zone_base = dev->arena;
-        keep_base = dev->arena + dev->zone_size;
-        arena_base = dev->arena + dev->zone_size + dev->keep_size;
+        zone_base = lane.arena;
+        keep_base = lane.arena + lane.zone_size;
+        arena_base = lane.arena + lane.zone_size + lane.keep_size;
     }
     // draw tables: pooled device memory, uploaded from pooled pinned staging
     // without a host wait (the upload is ordered before the plan's launches)
@@ -2926,7 +3008,7 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
     }
     for (Step &s : plan.steps) {
         if (s.kind == StepKind::Lines) {
-            layout_lines(s, arena_base + s.arena_off, zone_base + line_zone_off, dev->frag_px, dev->frag_px_size, dev);
+            layout_lines(s, arena_base + s.arena_off, zone_base + line_zone_off, dev->frag_px, dev->frag_px_size, lane);
             plan.launches += s.draws[0].total_prims == 0 ? 0 : (tiled_lines(s.draws[0]) ? 2 : 3);
             plan.prims += s.draws[0].total_prims;
             continue;
@@ -2936,7 +3018,7 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
             continue;
         }
         layout_group(s, arena_base + s.arena_off, zone_base + s.zone_off, keep_base + s.keep_off, dev->frag_px,
-                     dev->frag_px_size, dev);
+                     dev->frag_px_size, dev, lane);
         plan.launches += (s.gl.total_prims > 0 ? (s.gl.inline_clip ? 2 : 3) : 1) + (!s.multi && restart_strip(s.draws[0]) ? 2 : 0);
         for (auto &d : s.draws) plan.prims += d.total_prims;
         if (!s.multi && !s.merged) continue;
@@ -2969,9 +3051,9 @@ static int32_t build_plan(WgcDevice_T *dev, WgcCommandBuffer_T *cb, Plan &plan, 
         s.batch.total_prims = acc_p;
     }
     if (tables)
-        HIP_TRY(hipMemcpyAsync(plan.d_tables, plan.h_tables, tables, hipMemcpyHostToDevice, dev->stream),
+        HIP_TRY(hipMemcpyAsync(plan.d_tables, plan.h_tables, tables, hipMemcpyHostToDevice, lane.stream),
                 "draw tables");
-    plan.arena_gen = dev->arena_gen;
+    plan.arena_gen = lane.arena_gen;
     plan.zone_used = zneed;
     plan.keep_used = kneed;
     plan.raster_cfg = cfg;
@@ -2993,11 +3075,11 @@ static hipError_t launch_step(WgcDevice_T *dev, const Step &s, hipStream_t st, K
     return launch_draw(s.draws[0], s.batch, s.gl, st, kt);
 }
 
-// Steps run in order on the device stream, except that the steps of one
-// stage (independent launch groups) alternate between the device stream and
-// a second stream, forked from and joined back into the device stream with
-// events (the same under hipGraph capture).
-static hipError_t launch_plan(WgcDevice_T *dev, const Plan &plan, KernelTimer *kt)
+// Steps run in order on the lane's stream, except that the steps of one
+// stage (independent launch groups; lane 0 only) alternate between it and
+// a second stream, forked from and joined back into it with events (the same
+// under hipGraph capture).
+static hipError_t launch_plan(WgcDevice_T *dev, hipStream_t stream, const Plan &plan, KernelTimer *kt)
 {
     hipError_t e = hipSuccess;
     size_t i = 0;
@@ -3005,17 +3087,17 @@ static hipError_t launch_plan(WgcDevice_T *dev, const Plan &plan, KernelTimer *k
         size_t j = i + 1;
         while (j < plan.steps.size() && plan.steps[j].stage == plan.steps[i].stage) ++j;
         if (j - i == 1) {
-            e = launch_step(dev, plan.steps[i], dev->stream, kt);
+            e = launch_step(dev, plan.steps[i], stream, kt);
             if (e != hipSuccess) return e;
             i = j;
             continue;
         }
-        e = hipEventRecord(dev->fork, dev->stream);
+        e = hipEventRecord(dev->fork, stream);
         if (e == hipSuccess) e = hipStreamWaitEvent(dev->side, dev->fork, 0);
         for (size_t k = i; k < j && e == hipSuccess; ++k)
-            e = launch_step(dev, plan.steps[k], ((k - i) & 1u) ? dev->side : dev->stream, kt);
+            e = launch_step(dev, plan.steps[k], ((k - i) & 1u) ? dev->side : stream, kt);
         if (e == hipSuccess) e = hipEventRecord(dev->join, dev->side);
-        if (e == hipSuccess) e = hipStreamWaitEvent(dev->stream, dev->join, 0);
+        if (e == hipSuccess) e = hipStreamWaitEvent(stream, dev->join, 0);
         if (e != hipSuccess) return e;
         i = j;
     }
@@ -3024,20 +3106,20 @@ static hipError_t launch_plan(WgcDevice_T *dev, const Plan &plan, KernelTimer *k
 
 // The first submission of a plan launches directly; a command buffer that
 // is submitted again is captured into a hipGraph then and replayed.
-static int32_t submit_plan(WgcDevice_T *dev, Plan &plan)
+static int32_t submit_plan(WgcDevice_T *dev, hipStream_t stream, Plan &plan)
 {
     KernelTimer *kt = dev->timing ? &dev->timer : nullptr;
     bool graph = dev->use_graphs && !kt && (plan.exec || plan.submits > 0);
     plan.submits++;
     if (!graph) {
-        HIP_TRY(launch_plan(dev, plan, kt), "launch");
+        HIP_TRY(launch_plan(dev, stream, plan, kt), "launch");
         return WGC_OK;
     }
     if (!plan.exec) {
-        HIP_TRY(hipStreamBeginCapture(dev->stream, hipStreamCaptureModeThreadLocal), "graph capture");
-        hipError_t e = launch_plan(dev, plan, nullptr);
+        HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "graph capture");
+        hipError_t e = launch_plan(dev, stream, plan, nullptr);
         hipGraph_t g = nullptr;
-        hipError_t e2 = hipStreamEndCapture(dev->stream, &g);
+        hipError_t e2 = hipStreamEndCapture(stream, &g);
         if (e != hipSuccess) {
             if (g) (void)hipGraphDestroy(g);
             return hip_fail(e, "graph capture launch");
@@ -3050,7 +3132,7 @@ static int32_t submit_plan(WgcDevice_T *dev, Plan &plan)
         }
         HIP_TRY(hipGraphInstantiate(&plan.exec, g, nullptr, nullptr, 0), "graph instantiate");
     }
-    HIP_TRY(hipGraphLaunch(plan.exec, dev->stream), "graph launch");
+    HIP_TRY(hipGraphLaunch(plan.exec, stream), "graph launch");
     return WGC_OK;
 }
 
@@ -3104,6 +3186,143 @@ static int32_t take_slot_and_event(WgcDevice_T *d, bool noalloc, HostCounters *&
 static int32_t submit_plans(WgcDevice_T *device, uint32_t count, const WgcCommandBuffer *buffers, bool noalloc,
                             Inflight &f);
 
+// f(resource, written) for what a render pass reads and writes on the device.
+template <class F>
+static void pass_resources(const PassCommand &pc, F &&f)
+{
+    if (pc.color) f(pc.color, true);
+    if (pc.depth) f(pc.depth, true);
+    for (const SubCommand &c : pc.cmds) {
+        if (!c.obj) continue;
+        if (c.kind == CmdKind::SetVertexBuffer || c.kind == CmdKind::SetIndexBuffer) {
+            f(c.obj, false);
+        } else if (c.kind == CmdKind::SetBindGroup) {
+            for (const BindingSlot &e : ((const WgcBindGroup_T *)c.obj)->entries) {
+                if (e.buffer) f(e.buffer, false);
+                if (e.texture) f(e.texture, false);
+            }
+        }
+    }
+}
+
+// The last submission of lane `l` that the pass has to follow: one that
+// wrote what it reads or writes, or read what it writes (0: none).
+static uint64_t conflict_with(const Lane &l, const PassCommand &pc)
+{
+    uint64_t index = 0;
+    pass_resources(pc, [&](const void *r, bool written) {
+        auto it = l.uses.find(r);
+        if (it == l.uses.end()) return;
+        index = std::max(index, it->second.wrote);
+        if (written) index = std::max(index, it->second.read);
+    });
+    return index;
+}
+
+// The lane of a submission, after making that lane wait for what the
+// submission has to follow on the other.  A pass at a time leaves most of the
+// GPU idle (a chain of latency-bound launches), so independent single passes
+// alternate between two streams: passes over three targets in turn, 1080p
+// mesh 35 -> 24 us a pass, 24 objects 60 -> 41, 200k blended triangles 312 ->
+// 236 (a third stream: 28, 45 and 256 where two gave 23, 35 and 227).  A pass
+// goes behind the submission that it has to follow (no wait between streams,
+// 5 to 10 us on an idle one) if that is the last of its lane, or this lane is
+// the shorter one, or next to nothing is queued (with a deep queue the event
+// has long passed when the wait is reached); one that has none to follow goes
+// where fewer submissions queue.  Passes on one target in turn stay on a lane.
+// Lane 0 also has the transfers, fills and timestamps: a pass goes to lane 1
+// only with none since the submission before it (a program that writes a
+// uniform every frame stays in order on lane 0), and waits there, once, for
+// those before that.  Command buffers of several passes or copies, several
+// command buffers at once, the allocation-free form, and devices that time
+// kernels, replay graphs or count fragments per pixel use lane 0, after
+// everything on lane 1.
+static int32_t choose_lane(WgcDevice_T *d, uint32_t count, const WgcCommandBuffer *buffers, bool noalloc,
+                           uint32_t &lane)
+{
+    lane = 0;
+    bool single = count == 1 && buffers[0]->passes.size() == 1 && buffers[0]->passes[0].copy_kind == COPY_NONE &&
+                  !buffers[0]->lane0 && !noalloc && !d->timing && !d->use_graphs && !d->frag_px;
+    Lane &l0 = d->lanes[0], &l1 = d->lanes[1];
+    if (!single) {
+        HIP_TRY(wait_for(d, l0.stream, l1.last), "lane");
+        return WGC_OK;
+    }
+    const PassCommand &pc = buffers[0]->passes[0];
+    uint64_t c0 = conflict_with(l0, pc), c1 = conflict_with(l1, pc);
+    if (d->main_ops == d->ops_last && !d->inflight.empty()) {
+        uint64_t c = std::max(c0, c1);
+        if (c < d->inflight.front().index) {
+            lane = l1.queued < l0.queued ? 1u : 0u;
+        } else {
+            const Lane &mine = c1 > c0 ? l1 : l0, &other = c1 > c0 ? l0 : l1;
+            bool stay = mine.last == c || mine.queued <= other.queued ||
+                        (d->inflight.size() < 4 && mine.queued == other.queued + 1u);
+            lane = (stay ? &mine : &other) == &l1 ? 1u : 0u;
+        }
+    }
+    if (lane == 1 && d->ops_lane1 != d->main_ops) {
+        HIP_TRY(hipEventRecord(d->mark, l0.stream), "lane");
+        HIP_TRY(hipStreamWaitEvent(l1.stream, d->mark, 0), "lane");
+        d->ops_lane1 = d->main_ops;
+    }
+    if (lane == 0) HIP_TRY(wait_for(d, l0.stream, c1), "lane");
+    else HIP_TRY(wait_for(d, l1.stream, c0), "lane");
+    return WGC_OK;
+}
+
+// Notes what submission `index` on lane `l` uses.
+static void note_uses(WgcDevice_T *d, Lane &l, uint64_t index, uint32_t count, const WgcCommandBuffer *buffers)
+{
+    if (l.uses.size() > 4096)
+        for (auto it = l.uses.begin(); it != l.uses.end();)
+            it = std::max(it->second.wrote, it->second.read) <= d->last_done ? l.uses.erase(it) : std::next(it);
+    for (uint32_t i = 0; i < count; ++i)
+        for (const PassCommand &pc : buffers[i]->passes) {
+            if (pc.copy_src) l.uses[pc.copy_src].read = index;
+            if (pc.copy_dst) l.uses[pc.copy_dst].wrote = index;
+            pass_resources(pc, [&](const void *r, bool written) {
+                Lane::Use &u = l.uses[r];
+                if (written) u.wrote = index;
+                else u.read = index;
+            });
+        }
+}
+
+// Launches a submission on lane f.lane and gives it its index.  On failure
+// nothing of it is left running and its references are let go.
+static int32_t submit_on_lane(WgcDevice_T *device, uint32_t count, const WgcCommandBuffer *buffers, bool noalloc,
+                              Inflight &f)
+{
+    Lane &lane = device->lanes[f.lane];
+    // the counters are zero here: every submission takes (and zeroes) them
+    // at its end, or is followed by this reset when it stopped before that
+    if (lane.counters_dirty) {
+        // a submission that stopped early may also have left launch-group
+        // words in the arena's zero region
+        hipError_t e0 = launch_reset(lane.d_frags, lane.d_error, lane.stream);
+        if (e0 == hipSuccess && lane.arena && lane.zone_size + lane.keep_size)
+            e0 = launch_fill(lane.arena, lane.zone_size + lane.keep_size, 0u, lane.stream, nullptr);
+        if (e0 != hipSuccess) return hip_fail(e0, "counter reset");
+        lane.counters_dirty = false;
+    }
+    f.prims = f.launches = 0;
+    lane.counters_dirty = true;
+    int32_t r = submit_plans(device, count, buffers, noalloc, f);
+    if (r != WGC_OK) {
+        // the counters stay dirty; the next submission resets them.  Kernels
+        // of the plans launched before the failure may still run on the
+        // command buffers' resources: they finish before those are let go.
+        (void)hipStreamSynchronize(lane.stream);
+        for (auto *o : f.keep) release(o);
+        f.keep.clear();
+        return r;
+    }
+    lane.counters_dirty = false;
+    f.index = device->next_index++;
+    return WGC_OK;
+}
+
 // Both submission forms.  `noalloc`: plans laid out in the static scratch,
 // launched directly (no graph), no device or pinned allocation.
 static int32_t submit(WgcDevice_T *device, uint32_t count, const WgcCommandBuffer *buffers,
@@ -3125,33 +3344,28 @@ static int32_t submit(WgcDevice_T *device, uint32_t count, const WgcCommandBuffe
         device->slot_pool.push_back(f.slot);
         device->event_pool.push_back(f.done);
     };
-    // the counters are zero here: every submission takes (and zeroes) them
-    // at its end, or is followed by this reset when it stopped before that
-    if (device->counters_dirty) {
-        // a submission that stopped early may also have left launch-group
-        // words in the arena's zero region
-        hipError_t e0 = launch_reset(device->d_frags, device->d_error, device->stream);
-        if (e0 == hipSuccess && device->arena && device->zone_size + device->keep_size)
-            e0 = launch_fill(device->arena, device->zone_size + device->keep_size, 0u, device->stream, nullptr);
-        if (e0 != hipSuccess) {
-            give_back();
-            return hip_fail(e0, "counter reset");
-        }
-        device->counters_dirty = false;
+    r0 = choose_lane(device, count, buffers, noalloc, f.lane);
+    if (r0 != WGC_OK) {
+        give_back();
+        return r0;
     }
-    f.index = device->next_index++;
-    device->counters_dirty = true;
-    int32_t r = submit_plans(device, count, buffers, noalloc, f);
+    int32_t r = submit_on_lane(device, count, buffers, noalloc, f);
+    if (r == kNoLane1) {
+        // no arena there: in order on lane 0, after everything on lane 1
+        f.lane = 0;
+        buffers[0]->lane0 = true;
+        hipError_t e = wait_for(device, device->stream, device->lanes[1].last);
+        r = e == hipSuccess ? submit_on_lane(device, count, buffers, noalloc, f) : hip_fail(e, "lane");
+    }
     if (r != WGC_OK) {
-        // the counters stay dirty; the next submission resets them.  Kernels
-        // of the plans launched before the failure may still run on the
-        // command buffers' resources: they finish before those are let go.
-        (void)hipStreamSynchronize(device->stream);
-        for (auto *o : f.keep) release(o);
         give_back();
         return r;
     }
-    device->counters_dirty = false;
+    Lane &lane = device->lanes[f.lane];
+    lane.last = f.index;
+    lane.queued++;
+    device->ops_last = device->main_ops;
+    note_uses(device, lane, f.index, count, buffers);
     if (submission_index) *submission_index = f.index;
     device->inflight.push_back(std::move(f));
     // keep the queue short: retire what is already done
@@ -3164,41 +3378,42 @@ static int32_t submit_plans(WgcDevice_T *device, uint32_t count, const WgcComman
                             Inflight &f)
 {
     KernelTimer *kt = (device->timing && !noalloc) ? &device->timer : nullptr;
+    Lane &lane = device->lanes[f.lane];
     size_t zone_dirty = 0;   // bytes of the zero region the plans launched so far have used
-    uint8_t *zone = noalloc ? device->scratch : device->arena;
+    uint8_t *zone = noalloc ? device->scratch : lane.arena;
     for (uint32_t i = 0; i < count; ++i) {
         WgcCommandBuffer_T *cb = buffers[i];
-        Plan &plan = noalloc ? *cb->plan_noalloc : *cb->plan;
-        if (plan.arena_gen != device->arena_gen || plan.raster_cfg != device->raster_cfg ||
+        Plan &plan = noalloc ? *cb->plan_noalloc : *cb->plans[f.lane];
+        if (plan.arena_gen != lane.arena_gen || plan.raster_cfg != device->raster_cfg ||
             (!noalloc && plan.batching != device->batching) || plan.hip_device != device->hip_device) {
-            int32_t r = build_plan(device, cb, plan, noalloc);
+            int32_t r = build_plan(device, lane, cb, plan, noalloc);
             if (r != WGC_OK) {
                 plan.reset();
                 return r;
             }
             // growing the arena may have invalidated plans built before
-            if (plan.arena_gen != device->arena_gen) {
-                r = build_plan(device, cb, plan, noalloc);
+            if (plan.arena_gen != lane.arena_gen) {
+                r = build_plan(device, lane, cb, plan, noalloc);
                 if (r != WGC_OK) return r;
             }
-            zone = noalloc ? device->scratch : device->arena;
+            zone = noalloc ? device->scratch : lane.arena;
         }
         if (noalloc) {
             // the scratch keeps whatever the last user left in it (another
             // device object on this GPU, a submission that stopped early):
             // its zero and kept-zero regions are cleared before each plan
             size_t z = align_up(plan.zone_used, 256) + align_up(plan.keep_used, 256);
-            HIP_TRY(launch_fill(device->scratch, z, 0u, device->stream, nullptr), "scratch zero regions");
+            HIP_TRY(launch_fill(device->scratch, z, 0u, lane.stream, nullptr), "scratch zero regions");
             zone_dirty = 0;
         } else if (zone_dirty && plan.zone_used) {
             // the plans of one submission share the zero region
-            HIP_TRY(launch_fill(device->arena, zone_dirty, 0u, device->stream, nullptr), "zero region");
+            HIP_TRY(launch_fill(lane.arena, zone_dirty, 0u, lane.stream, nullptr), "zero region");
             zone_dirty = 0;
         }
         if (noalloc) {
-            HIP_TRY(launch_plan(device, plan, kt), "launch");
+            HIP_TRY(launch_plan(device, lane.stream, plan, kt), "launch");
         } else {
-            int32_t r = submit_plan(device, plan);
+            int32_t r = submit_plan(device, lane.stream, plan);
             if (r != WGC_OK) return r;
         }
         zone_dirty = std::max(zone_dirty, plan.zone_used);
@@ -3210,7 +3425,7 @@ static int32_t submit_plans(WgcDevice_T *device, uint32_t count, const WgcComman
     // the submission's counters, read by the host once its event has passed
     // (the event is the end kernel's own completion: one packet less than a
     // separate record, about 1 us per submission)
-    HIP_TRY(launch_end_submission(device->d_frags, device->d_error, f.slot, zone, zone_dirty, device->stream, f.done),
+    HIP_TRY(launch_end_submission(lane.d_frags, lane.d_error, f.slot, zone, zone_dirty, lane.stream, f.done),
             "counter readback");
     return WGC_OK;
 }
@@ -3263,6 +3478,7 @@ extern "C" int32_t wgc_device_timestamp(WgcDevice device, uint32_t slot)
     std::lock_guard<std::mutex> lk(device->mu);
     HIP_TRY(hipSetDevice(device->hip_device), "hipSetDevice");
     if (!device->ts[slot]) HIP_TRY(hipEventCreate(&device->ts[slot]), "hipEventCreate");
+    HIP_TRY(before_main_op(device), "timestamp");
     HIP_TRY(hipEventRecord(device->ts[slot], device->stream), "hipEventRecord");
     device->ts_recorded[slot] = true;
     return WGC_OK;
