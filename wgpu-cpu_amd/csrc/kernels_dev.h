@@ -19,7 +19,7 @@
 //  k_tiles     persistent workgroups, statically scheduled over the active
 //              tiles: the winners of each pixel (an order-independent minimum
 //              of depth and API-order key in LDS), then the winners shaded,
-//              one coalesced colour and depth store; then chunks of untouched
+//              one coalesced colour and depth store; then the untouched
 //              tiles (the LoadOp::Clear values, or only big triangles).
 //  k_raster    the same schedule for ordered draws: each tile's keys sorted
 //              into API order, colour and depth in registers from load or
@@ -705,7 +705,9 @@ __global__ __launch_bounds__(256) void k_clip(DrawParams d0, BatchArgs b, const 
 __device__ __forceinline__ bool in_big_union(const DrawParams &d, uint32_t tile)
 {
     if (d.s.counters[C_BIG] == 0u) return false;
-    uint32_t tx = tile % d.tiles_x, ty = tile / d.tiles_x;
+    uint32_t tiles_x = d.tiles_x;
+    asm volatile("" : "+v"(tiles_x));   // the division is set up here, not held in registers
+    uint32_t tx = tile % tiles_x, ty = tile / tiles_x;
     return tx >= 65535u - d.s.counters[C_BIG_NX0] && tx <= d.s.counters[C_BIG_X1] &&
            ty >= 65535u - d.s.counters[C_BIG_NY0] && ty <= d.s.counters[C_BIG_Y1];
 }
@@ -2097,35 +2099,67 @@ __device__ __forceinline__ void raster_tile_oi(const DrawParams &d, const BatchA
 }
 
 // Stores the clear values into one tile.
-template <int TS, int NT>
+// One wave stores the LoadOp::Clear values into a tile: 16 bytes a lane where
+// the rows allow it (a 16x16 tile is one store per texture).
+template <int TS>
 __device__ __forceinline__ void clear_tile(const DrawParams &d, uint32_t tile)
 {
-    constexpr int PPT = TS * TS / NT;
     uint32_t x0 = (tile % d.tiles_x) * TS, y0 = (tile / d.tiles_x) * TS;
-#pragma unroll
-    for (int k = 0; k < PPT; ++k) {
-        uint32_t q = threadIdx.x + (uint32_t)k * NT;
+    uint32_t width = d.width, height = d.height, lane = lane_id();
+    uint32_t *color = d.clear_color_on ? reinterpret_cast<uint32_t *>(d.color) : nullptr;
+    uint32_t *depth = d.clear_depth_on ? reinterpret_cast<uint32_t *>(d.depth) : nullptr;
+    uint32_t c = d.clear_rgba, z = __float_as_uint(d.clear_depth);
+    asm volatile("" : "+v"(lane), "+v"(c), "+v"(z));   // as in untouched_tiles
+    if (width % 4u == 0u && (((uint64_t)color | (uint64_t)depth) & 15u) == 0u) {
+#pragma unroll 1
+        for (uint32_t q = lane; q < TS * TS / 4; q += 64u) {
+            uint32_t px = x0 + q % (TS / 4) * 4u, py = y0 + q / (TS / 4);
+            if (px >= width || py >= height) continue;
+            size_t pix = (size_t)py * width + px;
+            if (color) store_stream4(color + pix, c);
+            if (depth) store_stream4(depth + pix, z);
+        }
+        return;
+    }
+#pragma unroll 1
+    for (uint32_t q = lane; q < TS * TS; q += 64u) {
         uint32_t px = x0 + q % TS, py = y0 + q / TS;
-        if (px >= d.width || py >= d.height) continue;
-        size_t pix = (size_t)py * d.width + px;
-        if (d.color && d.clear_color_on) store_color(d, pix, d.clear_rgba);
-        if (d.depth && d.clear_depth_on) store_depth(d, pix, d.clear_depth);
+        if (px >= width || py >= height) continue;
+        size_t pix = (size_t)py * width + px;
+        if (color) store_stream(color + pix, c);
+        if (depth) store_stream(depth + pix, z);
     }
 }
 
-// The tiles without binned records, kClearChunk per work item: those in
-// the footprint union of their draw's big triangles are rastered (`tile_fn`),
-// the others get the LoadOp::Clear values (when the draw clears).  The
-// chunk's bin counts are read together, one per lane.
+// The tiles without binned records: those in the footprint union of their
+// draw's big triangles are rastered by the workgroup (`tile_fn`), the others
+// get the LoadOp::Clear values (when the draw clears), a wave a tile.  The
+// grid takes runs of 2^kClearRunShift tiles (their rows lie together) in turn.
+// When the group has big triangles it takes single tiles, since those that
+// are rastered cost as much as any other and lie together (eight in a row by
+// one workgroup: 734x772 of 175 triangles 42 us a pass, now 26; 3633x2012 of
+// 410 90, now 70), or pairs (whole 128-byte lines) when there are many for
+// each workgroup (256 passes: 667 us with eights or pairs, 683 with singles).
+// 64 tiles are looked up at a time, one a lane (by every wave for itself: no
+// LDS, no barrier).  Registers that hold something for the whole loop spill
+// the tile kernel (12 of them: 1080p 21.7 -> 22.7 us), hence the asm below.
+// `start`: the workgroup's place in the turn.
 template <bool MULTI, int TS, int NT, class F>
-__device__ __forceinline__ void untouched_chunk(const DrawParams &d0, const BatchArgs &b, uint32_t chunk,
-                                                uint32_t *kinds, F &&tile_fn)
+__device__ __forceinline__ void untouched_tiles(const DrawParams &d0, const BatchArgs &b, uint32_t start, F &&tile_fn)
 {
-    uint32_t g0 = chunk * kClearChunk;
-    if (threadIdx.x < kClearChunk) {
-        uint32_t gt = g0 + threadIdx.x, kind = 0u, di = 0u;
-        if (gt < b.total_tiles && b.tile_count[gt] == 0u) {
-            uint32_t tile = gt;
+    constexpr uint32_t WAVES = NT / 64;
+    uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t total = b.total_tiles;
+    uint32_t shift = b.header[H_BIG] == 0u ? kClearRunShift : (total >= 16u * gridDim.x ? 1u : 0u);
+    uint32_t step = gridDim.x << shift;   // (below 2^25 tiles: no overflow)
+    for (uint32_t base = start << shift; base < total; base += (64u >> shift) * step) {
+        // the k-th of the 64 (no register is held for it over the tiles' work)
+        auto nth = [&](uint32_t k) { return base + (k >> shift) * step + (k & ((1u << shift) - 1u)); };
+        uint32_t lane = lane_id();
+        asm volatile("" : "+v"(lane));   // computed here, not held in registers over the tiles' work
+        uint32_t gt = nth(lane), kind = 0u;
+        if (gt < total && b.tile_count[gt] == 0u) {
+            uint32_t tile = gt, di = 0u;
             if constexpr (MULTI) {
                 di = b.tile_draw[gt];
                 tile = gt - b.tile_base[di];
@@ -2133,19 +2167,17 @@ __device__ __forceinline__ void untouched_chunk(const DrawParams &d0, const Batc
             const DrawParams &d = draw_at<MULTI>(d0, b, di);
             kind = in_big_union(d, tile) ? 2u : (d.init_clear && b.any_clear ? 1u : 0u);
         }
-        kinds[threadIdx.x] = kind | (di << 2);
+        uint64_t clears = __ballot(kind == 1u), tiles = __ballot(kind == 2u);
+        auto each = [&](uint32_t k, auto &&fn) {
+            uint32_t g = nth(k), di = 0u;
+            if constexpr (MULTI) di = __builtin_amdgcn_readfirstlane(b.tile_draw[g]);
+            const DrawParams &d = draw_at<MULTI>(d0, b, di);
+            fn(d, g - d.s.tile0);
+        };
+        for (uint32_t k = 0; clears; ++k, clears &= clears - 1u)
+            if (k % WAVES == wave) each((uint32_t)__ffsll((unsigned long long)clears) - 1u, clear_tile<TS>);
+        for (; tiles; tiles &= tiles - 1u) each((uint32_t)__ffsll((unsigned long long)tiles) - 1u, tile_fn);
     }
-    __syncthreads();
-    for (uint32_t i = 0; i < kClearChunk; ++i) {
-        uint32_t kd = __builtin_amdgcn_readfirstlane(kinds[i]);
-        if ((kd & 3u) == 0u) continue;
-        uint32_t di = kd >> 2, gt = g0 + i;
-        const DrawParams &d = draw_at<MULTI>(d0, b, di);
-        uint32_t tile = gt - d.s.tile0;
-        if ((kd & 3u) == 1u) clear_tile<TS, NT>(d, tile);
-        else tile_fn(d, tile);
-    }
-    __syncthreads();  // kinds is rewritten by the next chunk
 }
 
 // Whether the untouched tiles need a pass: some draw clears, or has big
@@ -2230,8 +2262,7 @@ __device__ __forceinline__ void count_fragments(const DrawParams &d0, const Batc
 // Ordered draws (blending, NotEqual + write), persistent: each tile's
 // fragments are applied in API order.  Work items are entries of the active
 // list, or four of them: a wave takes each if it can (light_tile), and the
-// workgroup the ones it could not, together.  Then the untouched tiles in
-// chunks, strided over the whole grid.
+// workgroup the ones it could not, together.  Then the untouched tiles.
 // MERGED: consecutive draws of one pass (d0 the first of them), one list of
 // tiles for all.
 // 200k blended triangles over 2560x2440, the pass: 446 us with a workgroup
@@ -2256,7 +2287,6 @@ __global__ __launch_bounds__(NT, 4) void k_raster(DrawParams d0, BatchArgs b)
     __shared__ uint32_t ticket;
     __shared__ uint32_t heavy[WAVES];
     __shared__ uint32_t wave_frags[NT / 64];
-    __shared__ uint32_t kinds[kClearChunk];
 
     ActiveSchedule w(b);
     uint32_t frag_acc = 0;
@@ -2300,18 +2330,16 @@ __global__ __launch_bounds__(NT, 4) void k_raster(DrawParams d0, BatchArgs b)
         if (!waves) raw = w.load(b, item);
     }
     __syncthreads();
-    // workgroups late in the schedule have the fewest active tiles: chunks from there
+    // workgroups late in the schedule have the fewest active tiles: from there
     if (untouched_pass(b))
-        for (uint32_t c = gridDim.x - 1u - w.first; c < b.n_chunks; c += gridDim.x)
-            untouched_chunk<MULTI, TS, NT>(d0, b, c, kinds, [&](const DrawParams &d, uint32_t tile) {
-                raster_tile<PROG, TS, NT, MERGED>(d, b, tile, u.together.sh, u.together.olist, olist_n, frag_acc);
-            });
+        untouched_tiles<MULTI, TS, NT>(d0, b, gridDim.x - 1u - w.first, [&](const DrawParams &d, uint32_t tile) {
+            raster_tile<PROG, TS, NT, MERGED>(d, b, tile, u.together.sh, u.together.olist, olist_n, frag_acc);
+        });
     count_fragments<MULTI, NT>(d0, b, frag_acc, wave_frags);
 }
 
 // Order-independent draws: visibility and shading of every active tile
-// (raster_tile_oi), then the untouched tiles in chunks, strided over the
-// whole grid.
+// (raster_tile_oi), then the untouched tiles.
 template <int PROG, bool MULTI, int TS, int NT, bool MERGED = false>
 __global__ __launch_bounds__(NT, (TilesOccupancy<TS, NT>::value)) void k_tiles(DrawParams d0, BatchArgs b)
 {
@@ -2321,7 +2349,6 @@ __global__ __launch_bounds__(NT, (TilesOccupancy<TS, NT>::value)) void k_tiles(D
     __shared__ VisShared<TS, NT> sh;
     __shared__ uint32_t ticket;
     __shared__ uint32_t wave_frags[NT / 64];
-    __shared__ uint32_t kinds[kClearChunk];
     __shared__ float srgb[256];   // the sRGB decode table (one device table for every draw)
 
     // read only when shading, after the first tile's barriers; every draw
@@ -2351,12 +2378,11 @@ __global__ __launch_bounds__(NT, (TilesOccupancy<TS, NT>::value)) void k_tiles(D
         item = w.index_of(ticket);
         raw = w.load(b, item);
     }
-    // workgroups late in the schedule have the fewest active tiles: chunks from there
+    // workgroups late in the schedule have the fewest active tiles: from there
     if (untouched_pass(b))
-        for (uint32_t c = gridDim.x - 1u - w.first; c < b.n_chunks; c += gridDim.x)
-            untouched_chunk<MULTI, TS, NT>(d0, b, c, kinds, [&](const DrawParams &d, uint32_t tile) {
-                raster_tile_oi<PROG, TS, NT, MERGED>(d, b, tile, 0u, sh, srgb, frag_acc);
-            });
+        untouched_tiles<MULTI, TS, NT>(d0, b, gridDim.x - 1u - w.first, [&](const DrawParams &d, uint32_t tile) {
+            raster_tile_oi<PROG, TS, NT, MERGED>(d, b, tile, 0u, sh, srgb, frag_acc);
+        });
     count_fragments<MULTI, NT>(d0, b, frag_acc, wave_frags);
 }
 

@@ -2521,7 +2521,6 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
     gl.lp = nullptr;
     b.n = (uint32_t)st.draws.size();
     b.total_tiles = (uint32_t)total_tiles;
-    b.n_chunks = (uint32_t)((total_tiles + kClearChunk - 1) / kClearChunk);
     b.header = gl.header;
     b.tile_count = gl.tile_count;
     b.active_list = (uint32_t *)(base + o_al);
@@ -2541,7 +2540,6 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
     }
     b.preclear = preclear ? 1u : 0u;
     b.any_clear = (any_clear && !b.preclear) ? 1u : 0u;
-    b.pad = 0;
     if (!st.multi && !st.merged) {
         b.draws = nullptr;
         b.prim_base = nullptr;
@@ -2560,7 +2558,7 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
     } else {
         occ = raster_blocks_per_cu(gl.program, gl.ordered != 0, st.multi, gl.raster_cfg);
     }
-    gl.raster_grid = resident_grid(dev, occ, total_tiles + b.n_chunks);
+    gl.raster_grid = resident_grid(dev, occ, total_tiles);
     uint64_t tile_base = 0, bin_base = 0, prim_base = 0;
     for (size_t k = 0; k < st.draws.size(); ++k) {
         uint32_t i = st.merged ? 0u : (uint32_t)k;   // the draw's target

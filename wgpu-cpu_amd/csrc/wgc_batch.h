@@ -20,7 +20,7 @@ struct BatchArgs {
     const uint32_t *tile_base;   // n + 1 prefix of tiles
     const uint32_t *wave_draw;   // the draw of every 64 primitives (the padded prefix)
     const uint32_t *tile_draw;   // the draw of every tile
-    uint32_t n, total_prims, total_tiles, n_chunks;
+    uint32_t n, total_prims, total_tiles;
     uint32_t *header;            // H_* words
     uint32_t *tile_count;        // all tiles of the group
     uint32_t *active_list;       // tiles with binned records, in the order they were first binned
@@ -28,10 +28,9 @@ struct BatchArgs {
     uint32_t n_counters;
     uint32_t any_clear;          // the tile kernel stores LoadOp::Clear values into untouched tiles
     uint32_t preclear;           // one target: setup stores the LoadOp::Clear values into the whole of it
-    uint32_t pad;
 };
 
-constexpr uint32_t kClearChunk = 8;     // tiles per work item of the untouched-tile pass
+constexpr uint32_t kClearRunShift = 3;  // log2 of the consecutive tiles a workgroup of the untouched-tile pass takes
 
 // Raster tile shapes: tile side x threads per workgroup.
 enum RasterCfg : uint32_t {
