@@ -251,3 +251,27 @@ def test_tiled_lines_every_octant_at_tile_edges(gpu_device, gpu_device_ext, blen
                            semantics=wgc.SEMANTICS_EXTENDED if blend else wgc.SEMANTICS_REFERENCE,
                            name=f"lines of every octant blend={blend}")
     both(spec, gpu_device_ext if blend else gpu_device)
+
+
+def test_most_lines_without_allocation(gpu_device_ext):
+    """2^19 blended lines (the most of a draw) on a target of 65,536 tiles: records and bins
+    together stay within the scratch of the allocation-free submission."""
+    announce("2^19 lines without allocation")
+    n, side = 1 << 19, 4096
+    p = scenes.splitmix_f32(6500, 2 * n).reshape(n, 2).astype(np.float64) * side
+    q = p + scenes.splitmix_f32(6501, 2 * n).reshape(n, 2) * 12.0 - 6.0
+    vb = np.zeros((2 * n, 8), np.float32)
+    for k, e in enumerate((p, q)):
+        vb[k::2, 0] = e[:, 0] / side * 2.0 - 1.0
+        vb[k::2, 1] = 1.0 - e[:, 1] / side * 2.0
+    vb[:, 2], vb[:, 3], vb[:, 7] = 0.5, 1.0, 0.4
+    vb[:, 4:7] = scenes.splitmix_f32(6502, 6 * n).reshape(-1, 3)
+    spec = scenes.PassSpec(side, side, clear_color=(0.1, 0.2, 0.3, 1.0),
+                           draws=[draw(vb, LINES, depth=None, blend=wgc.BLEND_ALPHA)],
+                           semantics=wgc.SEMANTICS_EXTENDED)
+    gpu_device_ext.enable_fragment_counts(0, 0)
+    pp = runner.PreparedPass(gpu_device_ext, spec)
+    pp.submit()
+    want = pp.results()[0].color
+    gpu_device_ext.submit_noalloc([pp.command_buffer])
+    np.testing.assert_array_equal(pp.results()[0].color, want)
