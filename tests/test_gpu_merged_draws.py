@@ -110,3 +110,29 @@ def test_noalloc_draws_one_at_a_time_equals_the_group(gpu_device):
     for r in (want, got):
         assert np.array_equal(r.color, ref.color)
         assert np.array_equal(r.depth.view(np.uint32), ref.depth.view(np.uint32))
+
+
+@pytest.mark.parametrize("blend", [False, True])
+def test_each_draw_keeps_its_clip_slots(gpu_device_ext, blend):
+    """Small draws whose triangles cross most of the clip planes: each has
+    more sub-triangles than two per primitive (about ten), which a draw of
+    few primitives has slots for, and so have the draws of a pass together."""
+    w, h, n = 150, 110, 60
+    draws, subs = [], 0
+    for k in range(12):
+        u = scenes.splitmix_f32(7400 + k, n * 8).reshape(n, 8)
+        vb = np.zeros((n, 3, 8), np.float32)
+        ang = 2.0 * np.pi * (u[:, :1] + np.arange(3) / 3.0)
+        vb[:, :, 0], vb[:, :, 1] = 2.2 * np.cos(ang), 2.2 * np.sin(ang)
+        vb[:, :, 2] = np.where(u[:, 1:2] < 0.5, (-0.4, 0.5, 1.5), (1.4, -0.3, 0.6))
+        vb[:, :, 3] = 1.0
+        vb[:, :, 4:8] = u[:, None, 4:8]
+        of_draw = sum(len(bridge.clip_triangle(t[:, :4])) for t in vb)
+        assert 2 * n < of_draw <= 2 * n + 1024
+        subs += of_draw
+        draws.append(clip_color_draw(vb, depth=None if blend else (wgc.LESS, True),
+                                     blend=wgc.BLEND_ALPHA if blend else wgc.BLEND_REPLACE))
+    assert subs > 2 * 64 * len(draws) + 1024
+    spec = scenes.PassSpec(w, h, has_depth=not blend, clear_depth=1.0, draws=draws, semantics=wgc.SEMANTICS_EXTENDED,
+                           name=f"clip slots of merged draws blend={blend}")
+    both(spec, gpu_device_ext)

@@ -2408,6 +2408,9 @@ static uint64_t group_prims(const Step &st, const DrawParams &d)
     return st.multi || st.merged ? align_up(d.total_prims, 64) : d.total_prims;
 }
 
+// Clipped sub-triangles that a draw has slots for beyond two per primitive.
+static constexpr uint64_t kClipSlots = 1024;
+
 // A group's words in the zero region: its header, per-draw counters, tile
 // counts and split-tile tickets.
 static size_t zone_bytes(const Step &st)
@@ -2451,14 +2454,16 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
         total_tiles += (uint64_t)d.tiles_x * d.tiles_y;
         any_clear = any_clear || d.init_clear;
     }
+    // clipped sub-triangles: the draws of a pass have together what each of
+    // them has alone
     for (size_t k = 0; k < st.draws.size(); ++k) {
+        uint64_t unit = st.merged ? group_prims(st, st.draws[k]) : st.draws[k].total_prims;
+        uint64_t clip = 2ull * unit + kClipSlots;
         prims += st.draws[k].total_prims;
         all_prims += group_prims(st, st.draws[k]);
-        unit_prims[st.merged ? 0 : k] += st.merged ? group_prims(st, st.draws[k]) : st.draws[k].total_prims;
-    }
-    for (uint32_t i = 0; i < n; ++i) {
-        clip_cap[i] = 2ull * unit_prims[i] + 1024ull;
-        clip_rec_cap += clip_cap[i];
+        unit_prims[st.merged ? 0 : k] += unit;
+        clip_cap[st.merged ? 0 : k] += clip;
+        clip_rec_cap += clip;
     }
     // bins, per target: slots for twice the tile's pixels, or four times the
     // target's primitives per tile when that is more (a bin rarely fills; the
@@ -2692,8 +2697,10 @@ static bool same_group(const DrawParams &a, const DrawParams &b)
 
 // Primitives of a merged group at most: its scratch is about 1.1 KB a
 // primitive for all its draws at once, and launches of this size are long
-// against the gaps between them (a draw of 500k triangles runs 100 us).
+// against the gaps between them (a draw of 500k triangles runs 100 us).  A
+// draw counts with its clip slots, which a primitive has two of.
 static constexpr uint64_t kMergedPrims = 1ull << 20;
+static uint64_t merged_size(const DrawParams &d) { return align_up(d.total_prims, 64) + kClipSlots / 2; }
 
 // A launch group of one draw, of independent draws, or (`merged`) of
 // consecutive draws of a pass (16x16 tiles under every tile option).
@@ -2838,12 +2845,12 @@ static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, 
                     // over 1366x768: 616 us a draw at a time, 60 us as
                     // one group
                     std::vector<DrawParams> run{dw.d};
-                    uint64_t prims = align_up(dw.d.total_prims, 64);
+                    uint64_t size = merged_size(dw.d);
                     while (!noalloc && !restart_strip(dw.d) && k + 1 < pw.draws.size() &&
                            same_group(dw.d, pw.draws[k + 1].d) &&
-                           prims + align_up(pw.draws[k + 1].d.total_prims, 64) <= kMergedPrims) {
+                           size + merged_size(pw.draws[k + 1].d) <= kMergedPrims) {
                         run.push_back(pw.draws[++k].d);
-                        prims += align_up(run.back().total_prims, 64);
+                        size += merged_size(run.back());
                     }
                     bool merged = run.size() > 1;
                     add_group(plan.steps, std::move(run), cfg, stage++, merged);
