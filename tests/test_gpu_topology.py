@@ -275,3 +275,30 @@ def test_most_lines_without_allocation(gpu_device_ext):
     want = pp.results()[0].color
     gpu_device_ext.submit_noalloc([pp.command_buffer])
     np.testing.assert_array_equal(pp.results()[0].color, want)
+
+
+@pytest.mark.parametrize("mode", ["less", "blend"])
+@pytest.mark.parametrize("scissor", [None, (0, 0, 0, 0), (9100, 3, 40, 30)], ids=["whole", "empty", "past"])
+def test_line_of_too_many_steps(mode, scissor):
+    """An error wherever the line's steps fall; the first 8192 of them are drawn."""
+    announce(f"line of too many steps {mode} {scissor}")
+    w, h, x0 = 9200, 40, 13
+    ends = np.array([[(x0, 5), (9190, 5)], [(x0, 11), (9190, 30)], [(x0, 36), (x0 + 8192, 33)]], np.float64) + 0.5
+    vb = np.zeros((6, 8), np.float32)
+    vb[:, 0] = ends.reshape(-1, 2)[:, 0] / w * 2.0 - 1.0
+    vb[:, 1] = 1.0 - ends.reshape(-1, 2)[:, 1] / h * 2.0
+    vb[:, 2], vb[:, 3], vb[:, 7] = 0.5, 1.0, 0.4
+    vb[:, 4:7] = scenes.splitmix_f32(6600, 18).reshape(6, 3)
+    d = draw(vb, LINES, depth=(wgc.LESS, True) if mode == "less" else None,
+             blend=wgc.BLEND_ALPHA if mode == "blend" else wgc.BLEND_REPLACE)
+    d.scissor = scissor
+    spec = scenes.PassSpec(w, h, has_depth=mode == "less", clear_depth=1.0, clear_color=(0.2, 0.4, 0.6, 1.0), draws=[d],
+                           semantics=wgc.SEMANTICS_EXTENDED)
+    want = bridge.render(spec).color.copy()
+    want[:, x0 + 8192:] = want[0, 0]
+    pp = runner.PreparedPass(wgc.Device(0, wgc.SEMANTICS_EXTENDED), spec)
+    pp.submit()
+    with pytest.raises(wgc.WgcError):
+        pp.device.poll()
+    color, _ = pp.res[0].read()
+    np.testing.assert_array_equal(color, want)

@@ -2504,8 +2504,9 @@ __device__ __forceinline__ bool lp_setup(const DrawParams &d, const VsOut *v, Lp
 // the walk runs in, the minor coordinate after k steps is the k-th partial
 // sum of the error term, floor(k * q / n), an exact integer, so any step's
 // pixel is found without walking to it.  (t, the running binary32 sum of
-// 1/n, is not: see lp_time.)  n and q are at most kLineSteps for the lines
-// that are drawn, so the products fit in 32 bits.
+// 1/n, is not: see lp_time.)  n and q of a line within kLineSteps are so
+// small that the products fit in 32 bits; a longer one (an error) is drawn
+// for its first kLineSteps steps.
 struct LineWalk {
     int32_t m0, c0, sm, sc;   // first pixel and direction along the major and the minor axis
     uint32_t n, q;
@@ -2523,14 +2524,19 @@ struct LineWalk {
         sm = dm < 0 ? -1 : 1;
         sc = dc < 0 ? -1 : 1;
     }
-    // a line of no steps draws nothing; one of too many raised its error
-    __device__ __forceinline__ bool drawn() const { return n != 0u && n <= kLineSteps; }
-    __device__ __forceinline__ int32_t minor(uint32_t k) const { return c0 + sc * (int32_t)(k * q / n); }
+    __device__ __forceinline__ uint32_t steps() const { return min(n, kLineSteps); }   // none: nothing is drawn
+    // (a * b + c) / d
+    __device__ __forceinline__ uint32_t ratio(uint32_t a, uint32_t b, uint32_t c, uint32_t d) const
+    {
+        return n <= kLineSteps ? (a * b + c) / d : (uint32_t)(((uint64_t)a * b + c) / d);
+    }
+    __device__ __forceinline__ uint32_t rise(uint32_t k) const { return ratio(k, q, 0u, n); }
+    __device__ __forceinline__ int32_t minor(uint32_t k) const { return c0 + sc * (int32_t)rise(k); }
     // The steps [k0, k1] whose major coordinate lies in [lo, hi]; empty: k0 > k1.
     __device__ __forceinline__ void major_steps(int32_t lo, int32_t hi, int32_t &k0, int32_t &k1) const
     {
         k0 = max(sm > 0 ? lo - m0 : m0 - hi, 0);
-        k1 = min(sm > 0 ? hi - m0 : m0 - lo, (int32_t)n - 1);
+        k1 = min(sm > 0 ? hi - m0 : m0 - lo, (int32_t)steps() - 1);
     }
     // The steps inside [x0, x1] x [y0, y1] (consecutive: both coordinates
     // move one way).  floor(k q / n) >= f  <=>  k >= ceil(f n / q).
@@ -2542,8 +2548,8 @@ struct LineWalk {
         int32_t lo = xmajor ? y0 : x0, hi = xmajor ? y1 : x1;
         int32_t f0 = sc > 0 ? lo - c0 : c0 - hi, f1 = sc > 0 ? hi - c0 : c0 - lo;
         if (f1 < 0 || f0 > (int32_t)q) return 0u;
-        if (f0 > 0) k0 = max(k0, (int32_t)(((uint32_t)f0 * n + q - 1u) / q));   // q >= f0 > 0
-        if (f1 < (int32_t)q) k1 = min(k1, (int32_t)((((uint32_t)f1 + 1u) * n + q - 1u) / q) - 1);
+        if (f0 > 0) k0 = max(k0, (int32_t)ratio((uint32_t)f0, n, q - 1u, q));   // q >= f0 > 0
+        if (f1 < (int32_t)q) k1 = min(k1, (int32_t)ratio((uint32_t)f1 + 1u, n, q - 1u, q) - 1);
         first = (uint32_t)k0;
         return k1 >= k0 ? (uint32_t)(k1 - k0) + 1u : 0u;
     }
@@ -2756,7 +2762,11 @@ __global__ __launch_bounds__(256) void k_lp_prep(DrawParams d, LpRec<N> *recs)
         if (N == 1) r.fb[0][0] = r.fb[0][1] = kNoPoint;
     }
     if (sub == 0u) recs[p] = r;
-    if (!ok || !d.scissor[2] || !d.scissor[3]) return;
+    if (!ok) return;
+    // a line of more than kLineSteps steps is an error, wherever they fall
+    if constexpr (N == 2)
+        if (LineWalk(r.fb[0], r.fb[1]).n > kLineSteps) atomicOr(d.s.error, (uint32_t)ERR_COORD_RANGE);
+    if (!d.scissor[2] || !d.scissor[3]) return;
     // the tiles that meet the scissor rect (inside the target, checked by the host)
     int32_t sx0 = (int32_t)(d.scissor[0] / kLpTile), sx1 = (int32_t)((d.scissor[0] + d.scissor[2] - 1u) / kLpTile);
     int32_t sy0 = (int32_t)(d.scissor[1] / kLpTile), sy1 = (int32_t)((d.scissor[1] + d.scissor[3] - 1u) / kLpTile);
@@ -2765,10 +2775,8 @@ __global__ __launch_bounds__(256) void k_lp_prep(DrawParams d, LpRec<N> *recs)
         lp_bin(d, (uint32_t)ty * d.tiles_x + (uint32_t)tx, p, tx >= sx0 && tx <= sx1 && ty >= sy0 && ty <= sy1);
     } else {
         LineWalk w(r.fb[0], r.fb[N - 1]);
-        // a line of more than kLineSteps steps is an error
-        if (w.n > kLineSteps) atomicOr(d.s.error, (uint32_t)ERR_COORD_RANGE);
-        if (!w.drawn()) return;
-        int32_t ma = w.m0, mb = w.m0 + w.sm * (int32_t)(w.n - 1u);
+        if (!w.n) return;
+        int32_t ma = w.m0, mb = w.m0 + w.sm * (int32_t)(w.steps() - 1u);
         int32_t lo = w.xmajor ? sx0 : sy0, hi = w.xmajor ? sx1 : sy1;          // scissor, major
         int32_t clo = w.xmajor ? sy0 : sx0, chi = w.xmajor ? sy1 : sx1;        // scissor, minor
         int32_t t0 = max(min(ma, mb) / (int32_t)kLpTile, lo), t1 = min(max(ma, mb) / (int32_t)kLpTile, hi);
@@ -2943,7 +2951,7 @@ __global__ __launch_bounds__(64) void k_lp_tiles(DrawParams d, const LpRec<N> *r
                         if constexpr (N == 1)
                             nf = mine[0] >= (uint32_t)cx0 && mine[0] <= (uint32_t)cx1 && mine[1] >= (uint32_t)cy0 &&
                                          mine[1] <= (uint32_t)cy1 ? 1u : 0u;
-                        else if (w.drawn()) nf = w.steps_inside(cx0, cy0, cx1, cy1, k0);
+                        else if (w.n) nf = w.steps_inside(cx0, cy0, cx1, cy1, k0);
                     }
                     uint32_t sum = wave_inclusive_sum(nf);
                     uint32_t n_frag = lane_value(sum, 63);
@@ -2952,7 +2960,7 @@ __global__ __launch_bounds__(64) void k_lp_tiles(DrawParams d, const LpRec<N> *r
                     } else if (nf) {
                         first[lane] = k0;
                         float dt = 1.0f / (float)w.n, t = lp_time(0.0f, dt, k0);
-                        uint32_t kq = k0 * w.q, quo = kq / w.n, rem = kq - quo * w.n;
+                        uint32_t quo = w.rise(k0), rem = k0 * w.q - quo * w.n;
                         int32_t m = w.m0 + w.sm * (int32_t)k0 - (int32_t)(w.xmajor ? x0 : y0);
                         int32_t c = w.c0 + w.sc * (int32_t)quo - (int32_t)(w.xmajor ? y0 : x0);
                         for (uint32_t j = 0, o = sum - nf; j < nf; ++j, ++o) {
