@@ -428,7 +428,9 @@ typedef enum WgcOption {
      * pixels with 1, 2, 4 or 8 waves) */
     WGC_OPTION_RASTER_TILE = 1,
     /* 1 (default): consecutive independent passes with one draw each share
-     * their launches (the batched form); 0: one launch set per draw */
+     * their launches (the batched form), and so do consecutive draws of a
+     * pass with the same shaders and depth / blend state; 0: one launch set
+     * per draw */
     WGC_OPTION_BATCHING = 2,
     /* 1: a command buffer's launches are captured once into a hipGraph and
      * replayed on every later submission; 0 (default): launched directly

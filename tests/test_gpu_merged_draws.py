@@ -136,3 +136,23 @@ def test_each_draw_keeps_its_clip_slots(gpu_device_ext, blend):
     spec = scenes.PassSpec(w, h, has_depth=not blend, clear_depth=1.0, draws=draws, semantics=wgc.SEMANTICS_EXTENDED,
                            name=f"clip slots of merged draws blend={blend}")
     both(spec, gpu_device_ext)
+
+
+def test_batching_off_is_one_launch_set_per_draw(gpu_device):
+    announce("draws of one pass, batching off")
+    w, h = 171, 133
+    draws = [triangles(n, 7500 + n, w, h, (wgc.LESS, True)) for n in (40, 300, 65)]
+    spec = scenes.PassSpec(w, h, has_depth=True, clear_depth=1.0, draws=draws)
+
+    def launches(spec):
+        got = runner.render(spec, gpu_device)
+        assert np.array_equal(got.color, bridge.render(spec).color)
+        return gpu_device.last_pass_stats().kernel_launches
+
+    merged = launches(spec)
+    gpu_device.set_option(wgc.OPTION_BATCHING, 0)
+    try:
+        alone = [launches(scenes.PassSpec(w, h, has_depth=True, clear_depth=1.0, draws=[d])) for d in draws]
+        assert launches(spec) == sum(alone) > merged
+    finally:
+        gpu_device.set_option(wgc.OPTION_BATCHING, 1)

@@ -589,7 +589,7 @@ struct WgcDevice_T : Object {
     uint64_t last_prims = 0, last_launches = 0;
     uint32_t cu_count = 256;        // compute units of the device
     uint32_t raster_cfg = RASTER_16x16_256;
-    bool batching = true;          // merge independent single-draw passes into launch groups
+    bool batching = true;          // draws share launches: independent single-draw passes, the draws of a pass
     // replay cached plans as hipGraphs (WGC_OPTION_GRAPHS).  Off by default:
     // on this ROCm a graph launch costs 22-27 us of host time per
     // submission against 7 us for the same launches made directly, and the
@@ -2840,13 +2840,13 @@ static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, 
                 DrawWork &dw = pw.draws[k];
                 if (!is_point_or_line(dw.d)) {
                     // consecutive draws with the same shaders and per-pixel
-                    // rule run as one group (the allocation-free form has no
-                    // table of draws).  24 objects of about 3000 triangles
+                    // rule run as one group (not with batching switched off;
+                    // the allocation-free form has no table of draws).  24 objects of about 3000 triangles
                     // over 1366x768: 616 us a draw at a time, 60 us as
                     // one group
                     std::vector<DrawParams> run{dw.d};
                     uint64_t size = merged_size(dw.d);
-                    while (!noalloc && !restart_strip(dw.d) && k + 1 < pw.draws.size() &&
+                    while (dev->batching && !noalloc && !restart_strip(dw.d) && k + 1 < pw.draws.size() &&
                            same_group(dw.d, pw.draws[k + 1].d) &&
                            size + merged_size(pw.draws[k + 1].d) <= kMergedPrims) {
                         run.push_back(pw.draws[++k].d);
