@@ -15,9 +15,11 @@
  *  - Return codes: WGC_OK (0) or a negative WgcStatus.  Where the reference
  *    panics (unwrap / expect / todo!), libwgc returns an error and keeps a
  *    thread-local message readable with wgc_last_error().
- *  - One HIP stream per device executes submissions in order, as the
- *    reference's single engine thread does (wgpu-cpu/src/engine.rs:26-46).
- *    Queue writes are ordered with respect to submissions.
+ *  - Submissions take effect in order, as on the reference's single engine
+ *    thread (wgpu-cpu/src/engine.rs:26-46), and queue writes are ordered with
+ *    respect to them.  A device executes on one HIP stream, and on a second
+ *    one submissions of a single pass that share no written resource with
+ *    those still running; "the device stream" below is both in that order.
  *  - Semantics: WGC_SEMANTICS_REFERENCE reproduces the reference bit for bit
  *    (integer scanline coverage, corner sampling, nearest texel rounding,
  *    no sRGB decode, no blending).  WGC_SEMANTICS_EXTENDED additionally
@@ -425,7 +427,9 @@ typedef enum WgcOption {
     /* raster tile shape: 0 = 16x16 px / 256 lanes, 1 = 8x8 / 64, 2 = 16x16 / 64,
      * 3 = 32x32 / 256, 4 = 16x16 / 128, 5 = 32x32 / 128, 6 = 32x32 / 512,
      * 7 = 32x32 / 64 (the autotuner's search space: tiles of 8, 16 and 32
-     * pixels with 1, 2, 4 or 8 waves) */
+     * pixels with 1, 2, 4 or 8 waves).  Draws with WGSL shaders, draws
+     * applied in API order, points and lines, and draws of a pass that share
+     * their launches use 16x16 px whatever the option says */
     WGC_OPTION_RASTER_TILE = 1,
     /* 1 (default): consecutive independent passes with one draw each share
      * their launches (the batched form), and so do consecutive draws of a
