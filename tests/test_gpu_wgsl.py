@@ -13,6 +13,7 @@
 import copy
 import struct
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -273,3 +274,25 @@ fn fs_main(f: VsOut) -> @location(0) vec4f {
         runner.render(spec, gpu_device)
     assert e.value.code == wgc.ERR_EXECUTION
     assert_parity(scenes.config1_plain_small(), gpu_device)
+
+
+def test_pipelines_of_one_shader_share_their_kernels(gpu_device_ext):
+    """A second pipeline that differs in its state compiles what the first
+    did not: a blended one the ordered raster (with setup and clipping it is
+    more than an opaque one), one that both cover nothing."""
+    announce("pipelines of one shader")
+    dev = gpu_device_ext
+    module = dev.create_shader_module_wgsl(
+        CLIP_VS + "@fragment\nfn fs_main(f: VsOut) -> @location(0) vec4f { return f.color * 0.8125; }\n")
+
+    def seconds(**state):
+        t = time.perf_counter()
+        keep.append(dev.create_render_pipeline(module, [(32, wgc.STEP_VERTEX, [(wgc.FLOAT32X4, 0, 0),
+                                                                               (wgc.FLOAT32X4, 16, 1)])], **state))
+        return time.perf_counter() - t
+
+    keep = []
+    opaque, blended = seconds(depth=(wgc.LESS, True)), seconds(blend=wgc.BLEND_ALPHA)
+    print(f"opaque {opaque:.2f} s, blended {blended:.2f} s", flush=True)
+    assert blended < opaque
+    assert seconds(depth=(wgc.NOT_EQUAL, True)) < 0.2 * opaque

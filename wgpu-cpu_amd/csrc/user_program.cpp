@@ -33,31 +33,39 @@ const char *const kRtcOptions[] = {
     "-fhip-fp32-correctly-rounded-divide-sqrt", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 };
 
-struct Compiled {
+struct Kernel {
     std::shared_ptr<RtcModule> code;
-    std::vector<hipFunction_t> fns;
+    hipFunction_t fn = nullptr;
 };
 
 std::mutex g_cache_mu;
-std::map<std::pair<int, std::string>, Compiled> g_cache;   // (device, source and kernels) -> program
+std::map<std::pair<int, std::string>, std::map<std::string, Kernel>> g_cache;   // (device, source) -> kernels by name
 
-// Compiles `src` (with the embedded headers and `extra` headers) and loads
-// it on device `hip_device` (< 0: compile only); `names` are name
-// expressions of the kernels.
+// The kernels `all` (name expressions) of `src` (with the embedded headers
+// and `extra` headers), loaded on device `hip_device` (< 0: compile only).
+// Those that no earlier call compiled are compiled together: pipelines of one
+// shader that differ in their state (opaque and blended, triangles and
+// lines) share the kernels that both reach.
 bool rtc_build(int hip_device, const std::string &src, const std::vector<std::pair<std::string, std::string>> &extra,
-               const std::vector<std::string> &names, Compiled &out, std::string &err)
+               const std::vector<std::string> &all, std::vector<Kernel> &out, std::string &err)
 {
     std::string key = src;
     for (auto &h : extra) key += "\n//--" + h.first + "\n" + h.second;
-    for (auto &n : names) key += "\n//--" + n;
+    std::map<std::string, Kernel> have;
     {
         std::lock_guard<std::mutex> g(g_cache_mu);
         auto it = g_cache.find({hip_device, key});
-        if (it != g_cache.end()) {
-            out = it->second;
-            return true;
-        }
+        if (it != g_cache.end()) have = it->second;
     }
+    std::vector<std::string> names;
+    for (auto &n : all)
+        if (!have.count(n)) names.push_back(n);
+    auto give = [&] {
+        out.clear();
+        for (auto &n : all) out.push_back(have[n]);
+        return true;
+    };
+    if (names.empty()) return give();
     std::vector<const char *> hdr, hdr_names;
     for (size_t i = 0; i < kEmbeddedCount; ++i) {
         hdr.push_back(kEmbeddedSources[i]);
@@ -108,21 +116,19 @@ bool rtc_build(int hip_device, const std::string &src, const std::vector<std::pa
         err = std::string("hipModuleLoadData: ") + hipGetErrorString(e);
         return false;
     }
-    Compiled c;
-    c.code = mod;
-    for (auto &lw : lowered) {
+    for (size_t i = 0; i < names.size(); ++i) {
         hipFunction_t f = nullptr;
-        e = hipModuleGetFunction(&f, mod->module, lw.c_str());
+        e = hipModuleGetFunction(&f, mod->module, lowered[i].c_str());
         if (e != hipSuccess) {
             err = std::string("hipModuleGetFunction: ") + hipGetErrorString(e);
             return false;
         }
-        c.fns.push_back(f);
+        have[names[i]] = Kernel{mod, f};
     }
     std::lock_guard<std::mutex> g(g_cache_mu);
-    g_cache[{hip_device, key}] = c;
-    out = c;
-    return true;
+    auto &kept = g_cache[{hip_device, key}];
+    for (auto &n : names) kept[n] = have[n];
+    return give();
 }
 
 uint32_t occupancy(hipFunction_t f, int threads)
@@ -383,8 +389,7 @@ bool build_user_program(int hip_device, const wgsl::Module &vm, const std::strin
     g += "}  // namespace wgc\n";
     // the glue follows the kernels: it uses their staged-triangle type
     std::string src = "#define WGC_USER_PROGRAM 1\n#include \"kernels_dev.h\"\n#include \"wgc_user.h\"\n";
-    // the kernels the pipeline can reach (each costs compile time: all of
-    // them about a third more than those of one triangle pipeline)
+    // the kernels the pipeline can reach (each costs compile time)
     UserKernels &k = out.kernels;
     bool ordered = uses.ordered || out.discards || out.early_depth || out.frag_depth_tested;
     bool free_order = !(out.discards || out.early_depth || out.frag_depth_tested);
@@ -418,12 +423,13 @@ bool build_user_program(int hip_device, const wgsl::Module &vm, const std::strin
     }
     std::vector<std::string> names;
     for (auto &w : want) names.push_back("wgc::" + w.first);
-    Compiled c;
-    if (!rtc_build(hip_device, src, {{"wgc_user.h", g}}, names, c, err)) return false;
+    std::vector<Kernel> fns;
+    if (!rtc_build(hip_device, src, {{"wgc_user.h", g}}, names, fns, err)) return false;
     if (hip_device < 0) return true;
-    out.code = c.code;
-    k.module = c.code->module;
-    for (size_t i = 0; i < want.size(); ++i) *want[i].second = c.fns[i];
+    for (size_t i = 0; i < want.size(); ++i) {
+        *want[i].second = fns[i].fn;
+        out.code.push_back(fns[i].code);
+    }
     auto occ = [](hipFunction_t f) { return f ? occupancy(f, 256) : 1u; };
     for (int m = 0; m < 2; ++m) {
         k.occ_tiles[m] = occ(k.tiles[m]);
@@ -480,10 +486,12 @@ bool build_entry_run(int hip_device, const wgsl::Module &m, const std::string &e
                     "}\n"
                     "}  // namespace wgc\n";
     std::string src = "#include \"wgc_core.h\"\n#include \"wgc_run.h\"\n";
-    Compiled c;
-    if (!rtc_build(hip_device, src, {{"wgc_run.h", g}}, {"wgc::k_run"}, c, err)) return false;
-    out.code = c.code;
-    out.fn = c.fns[0];
+    std::vector<Kernel> fns;
+    if (!rtc_build(hip_device, src, {{"wgc_run.h", g}}, {"wgc::k_run"}, fns, err)) return false;
+    if (hip_device >= 0) {
+        out.code = fns[0].code;
+        out.fn = fns[0].fn;
+    }
     out.slots = m.resources;
     out.stage = e.stage;
     return true;

@@ -22,7 +22,7 @@ struct RtcModule {
 
 // The shader program of one pipeline.
 struct UserProgram {
-    std::shared_ptr<RtcModule> code;
+    std::vector<std::shared_ptr<RtcModule>> code;   // of each kernel
     UserKernels kernels;
     struct Slot {
         uint32_t group = 0, binding = 0;
@@ -49,8 +49,8 @@ struct PipelineUses {
 // Pairs a vertex entry point with an optional fragment entry point (entry
 // names may be empty: the module's only entry point of that stage), checks
 // the stage interface and compiles the kernels that `uses` can reach
-// (hip_device < 0: compile only, without loading).  `extended` allows the perspective interpolation
-// the reference leaves as todo!().
+// (hip_device < 0: compile only, without loading).  `extended` allows the
+// perspective interpolation the reference leaves as todo!().
 bool build_user_program(int hip_device, const wgsl::Module &vm, const std::string &vs_entry,
                         const wgsl::Module *fm, const std::string &fs_entry, bool extended, const PipelineUses &uses,
                         UserProgram &out, std::string &err);

@@ -92,7 +92,6 @@ struct KernelTimer {
 // for PROG_USER of the kernels that run shader code, compiled with hipRTC
 // (index: 0 single draw, 1 batched), and their resident workgroups per CU.
 struct UserKernels {
-    hipModule_t module = nullptr;
     hipFunction_t setup[2]{}, clip[2]{}, tiles[2]{}, raster[2]{};
     hipFunction_t point_vis{}, point_shade{};
     hipFunction_t lp_prep[2]{}, lp_ordered[2]{}, lp_tiles{};   // index: points 0, lines 1; lp_tiles: lines
