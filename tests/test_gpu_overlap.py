@@ -151,3 +151,75 @@ def test_written_between_submissions():
     dev.poll()
     for s, r in zip(specs, res):
         np.testing.assert_array_equal(r.read()[0], bridge.render(s).color)
+
+
+def test_heap_targets_reused_between_lanes():
+    """Targets from a heap that is full with four of them: each is released
+    as soon as its picture has been copied, and the next takes its place while
+    passes on other targets run."""
+    announce("heap targets reused between lanes")
+    dev = wgc.Device(0, wgc.SEMANTICS_EXTENDED)
+    heap = dev.create_heap(4 * SIZE * SIZE * 4)
+    specs = [scenes.PassSpec(SIZE, SIZE, clear_color=(0.1 * i, 0.2, 0.3, 1.0), draws=[blended(150 + 400 * i, 8400 + i)],
+                             semantics=wgc.SEMANTICS_EXTENDED) for i in range(5)]
+    refs = [bridge.render(s).color for s in specs]
+    keep, cache, out = [], {}, []
+    for n in range(40):
+        target = heap.create_texture(SIZE, SIZE, wgc.RGBA8_UNORM)
+        if target is None:      # full until the last submissions of released ones have executed
+            dev.poll()
+            target = heap.create_texture(SIZE, SIZE, wgc.RGBA8_UNORM)
+        enc = dev.create_command_encoder()
+        runner.record_pass(dev, enc, specs[n % 5], SimpleNamespace(color=target, depth=None), keep, cache)
+        draw = enc.finish()
+        dev.submit([draw])
+        if n % 3 == 0:
+            dev.submit([draw])
+        enc = dev.create_command_encoder()
+        buf = dev.create_buffer(SIZE * 512)
+        enc.copy_texture_to_buffer(target, (0, 0), buf, 0, 512, SIZE, SIZE)
+        dev.submit([enc.finish()])
+        out.append(buf)
+        target.release()
+    dev.poll()
+    for n, buf in enumerate(out):
+        got = np.frombuffer(buf.read(), np.uint8).reshape(SIZE, 512)[:, :SIZE * 4].reshape(SIZE, SIZE, 4)
+        np.testing.assert_array_equal(got, refs[n % 5])
+
+
+def test_mapped_between_submissions():
+    """A vertex buffer written through a mapping between submissions on
+    several targets, some of them running on the other lane."""
+    announce("mapped between submissions")
+    dev = wgc.Device(0, wgc.SEMANTICS_EXTENDED)
+    datas = [random_clip_triangles(300, 8500 + i, SIZE, SIZE, alpha=(0.2, 0.8)) for i in range(6)]
+    specs = [scenes.PassSpec(SIZE, SIZE, clear_color=(0.0, 0.0, 0.0, 1.0),
+                             draws=[clip_color_draw(v, depth=None, blend=wgc.BLEND_ALPHA)],
+                             semantics=wgc.SEMANTICS_EXTENDED) for v in datas]
+    cache, keep = {}, []
+    data = specs[0].draws[0].vertex_data
+    vb = dev.create_buffer_init(data)
+    cache[("buf", data)] = vb
+    others = [runner.PreparedPass(dev, scenes.PassSpec(SIZE, SIZE, draws=[blended(900, 8600 + i)],
+                                                       semantics=wgc.SEMANTICS_EXTENDED)) for i in range(2)]
+    res = [runner._PassResources(dev, specs[0], keep) for _ in specs]
+    buffers = []
+    for r in res:
+        enc = dev.create_command_encoder()
+        runner.record_pass(dev, enc, specs[0], r, keep, cache)
+        buffers.append(enc.finish())
+    for _ in range(3):
+        for s, cb in zip(specs, buffers):
+            vb.map_async(wgc.MAP_WRITE)
+            dev.poll()
+            np.frombuffer(vb.get_mapped_range(), np.uint8)[:] = np.frombuffer(s.draws[0].vertex_data, np.uint8)
+            for o in others:
+                o.submit()
+            vb.unmap()
+            for o in others:
+                o.submit()
+            dev.submit([cb])
+            dev.submit([cb])
+    dev.poll()
+    for s, r in zip(specs, res):
+        np.testing.assert_array_equal(r.read()[0], bridge.render(s).color)
