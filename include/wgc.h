@@ -451,6 +451,13 @@ int32_t wgc_device_get_option(WgcDevice device, uint32_t option, uint32_t *value
 int32_t wgc_device_debug_fragment_counts(WgcDevice device, uint32_t width, uint32_t height,
                                          uint32_t *host_out);
 
+/* Debug aid with no reference counterpart: waits for the queue, lets the
+ * scratch arenas go, and from then on has their allocations fail as if memory
+ * had run out where the device's arenas would exceed `arena_bytes` together,
+ * and gives allocation-free submissions `static_bytes` of their scratch
+ * (0: no limit but the memory there is). */
+int32_t wgc_device_debug_scratch_limit(WgcDevice device, uint64_t arena_bytes, uint64_t static_bytes);
+
 /* ---- measurement (no reference counterpart; render_pass/mod.rs:346,392 only
  *      logs the pass time) ---- */
 /* Records an event on the device stream into slot (0..63). */

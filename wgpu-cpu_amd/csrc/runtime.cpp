@@ -560,6 +560,9 @@ struct WgcDevice_T : Object {
     std::mutex mu;
     Lane lanes[2];                  // lanes[0].stream == stream
     hipEvent_t mark = nullptr;      // lane 1 starts after what lane 0 held then
+    // debug limits (wgc_device_debug_scratch_limit): of both arenas together,
+    // and of the static scratch
+    size_t arena_limit = SIZE_MAX, static_limit = SIZE_MAX;
     uint64_t main_ops = 0;          // transfers, fills and timestamps on lane 0 so far; their number
     uint64_t ops_lane1 = 0;         // when lane 1 was last made to wait for them, and
     uint64_t ops_last = 0;          // at the last submission
@@ -904,6 +907,53 @@ static hipError_t before_main_op(WgcDevice_T *d, const void *resource = nullptr)
     return wait_for(d, d->stream, index);
 }
 
+// Lets a lane's arena go once its stream has drained.  The plans laid out in
+// it are built again.
+static hipError_t drop_arena(Lane &l)
+{
+    l.arena_gen++;
+    hipError_t e = hipStreamSynchronize(l.stream);
+    if (e == hipSuccess && l.arena) e = hipFree(l.arena);
+    if (e == hipSuccess) {
+        l.arena = nullptr;
+        l.arena_size = l.zone_size = l.keep_size = 0;
+    }
+    return e;
+}
+
+// hipMalloc; when memory has run out, lane 1's arena, which only lets passes
+// run beside each other, makes room.  `locked`: the caller holds the device's
+// lock.
+template <class T>
+static hipError_t device_malloc(WgcDevice_T *d, T **p, size_t bytes, bool locked = false)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    {
+        std::unique_lock<std::mutex> lk(d->mu, std::defer_lock);
+        if (!locked) lk.lock();
+        if (!d->lanes[1].arena || drop_arena(d->lanes[1]) != hipSuccess) return e;
+    }
+    return hipMalloc(p, bytes);
+}
+
+// The arena of a lane.
+static hipError_t arena_malloc(WgcDevice_T *d, Lane &lane, size_t bytes)
+{
+    const bool first = &lane == &d->lanes[0];
+    Lane &other = d->lanes[first ? 1 : 0];
+    for (;;) {
+        hipError_t e = hipErrorOutOfMemory;
+        if (bytes <= d->arena_limit && other.arena_size <= d->arena_limit - bytes) e = hipMalloc(&lane.arena, bytes);
+        if (e == hipSuccess) return e;
+        (void)hipGetLastError();
+        lane.arena = nullptr;
+        // lane 0 has the room of lane 1's, never the other way round
+        if (e != hipErrorOutOfMemory || !first || !other.arena || drop_arena(other) != hipSuccess) return e;
+    }
+}
+
 static int32_t resolve_timers(WgcDevice_T *d)
 {
     for (auto &p : d->timer.pending) {
@@ -1023,10 +1073,23 @@ extern "C" int32_t wgc_device_debug_fragment_counts(WgcDevice device, uint32_t w
         device->frag_px_size = 0;
     }
     if (need) {
-        HIP_TRY(hipMalloc(&device->frag_px, need), "hipMalloc");
+        HIP_TRY(device_malloc(device, &device->frag_px, need, true), "hipMalloc");
         HIP_TRY(stream_zero(device->stream, device->frag_px, need), "hipMemset");
         device->frag_px_size = need;
     }
+    return WGC_OK;
+}
+
+extern "C" int32_t wgc_device_debug_scratch_limit(WgcDevice device, uint64_t arena_bytes, uint64_t static_bytes)
+{
+    if (!device) return set_error(WGC_ERR_INVALID, "null device");
+    std::lock_guard<std::mutex> lk(device->mu);
+    HIP_TRY(hipSetDevice(device->hip_device), "hipSetDevice");
+    int32_t r = drain(device);
+    if (r != WGC_OK) return r;
+    for (auto &l : device->lanes) HIP_TRY(drop_arena(l), "arena");
+    device->arena_limit = arena_bytes ? (size_t)arena_bytes : SIZE_MAX;
+    device->static_limit = static_bytes ? (size_t)static_bytes : SIZE_MAX;
     return WGC_OK;
 }
 
@@ -1043,7 +1106,7 @@ extern "C" int32_t wgc_buffer_create(WgcDevice device, uint64_t size, WgcBuffer 
     retain(device);
     b->size = size;
     if (size) {
-        hipError_t e = hipMalloc(&b->ptr, size);
+        hipError_t e = device_malloc(device, &b->ptr, size);
         if (e == hipSuccess) {
             std::lock_guard<std::mutex> lk(device->mu);
             e = before_main_op(device, b);
@@ -1248,7 +1311,7 @@ extern "C" int32_t wgc_texture_create(WgcDevice device, uint32_t width, uint32_t
     t->height = height;
     t->format = format;
     t->size = (uint64_t)width * height * tb;
-    hipError_t e = hipMalloc(&t->ptr, t->size);
+    hipError_t e = device_malloc(device, &t->ptr, t->size);
     if (e == hipSuccess) {
         std::lock_guard<std::mutex> lk(device->mu);
         e = before_main_op(device, t);
@@ -1276,7 +1339,7 @@ extern "C" int32_t wgc_heap_create(WgcDevice device, uint64_t size, WgcHeap *out
     h->dev = device;
     retain(device);
     size = (size + RangeAllocator::kAlign - 1) / RangeAllocator::kAlign * RangeAllocator::kAlign;
-    if (hipMalloc(&h->base, size) != hipSuccess) {
+    if (device_malloc(device, &h->base, size) != hipSuccess) {
         h->base = nullptr;
         release(h);
         return set_error(WGC_ERR_OUT_OF_MEMORY, "heap: cannot allocate " + std::to_string(size) + " bytes");
@@ -1556,7 +1619,7 @@ extern "C" int32_t wgc_shader_module_run(WgcDevice device, WgcShaderModule modul
     if (rc != WGC_OK) return rc;
     uint32_t *d_out = nullptr;
     size_t bytes = (size_t)count * kRunWords * 4u;
-    HIP_TRY(hipMalloc(&d_out, bytes), "run results");
+    HIP_TRY(device_malloc(device, &d_out, bytes, true), "run results");
     void *args[] = {&d, &first_index, &count, &d_out};
     hipError_t e = hipModuleLaunchKernel(run->fn, (count + 63u) / 64u, 1, 1, 64, 1, 1, 0, device->stream, args, nullptr);
     if (e == hipSuccess) e = stream_copy(device->stream, results, d_out, bytes, hipMemcpyDeviceToHost);
@@ -2792,7 +2855,9 @@ static void copy_step(const PassCommand &pc, Step &s)
 static constexpr size_t kLane1Arena = 2ull << 30;
 static constexpr int32_t kNoLane1 = 1;
 
-static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, Plan &plan, bool noalloc)
+// `merge_max`: the size of a merged group at most; `merged`: whether there is one.
+static int32_t lay_out_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, Plan &plan, bool noalloc,
+                            uint64_t merge_max, bool &merged)
 {
     plan.reset();
     plan.noalloc = noalloc;
@@ -2848,12 +2913,13 @@ static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, 
                     uint64_t size = merged_size(dw.d);
                     while (dev->batching && !noalloc && !restart_strip(dw.d) && k + 1 < pw.draws.size() &&
                            same_group(dw.d, pw.draws[k + 1].d) &&
-                           size + merged_size(pw.draws[k + 1].d) <= kMergedPrims) {
+                           size + merged_size(pw.draws[k + 1].d) <= merge_max) {
                         run.push_back(pw.draws[++k].d);
                         size += merged_size(run.back());
                     }
-                    bool merged = run.size() > 1;
-                    add_group(plan.steps, std::move(run), cfg, stage++, merged);
+                    bool several = run.size() > 1;
+                    merged = merged || several;
+                    add_group(plan.steps, std::move(run), cfg, stage++, several);
                     continue;
                 }
                 // points and lines: the tile kernel applies the pass's clear (if
@@ -2961,11 +3027,11 @@ static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, 
         // the static scratch: zero region, kept-zero region, then the stages
         size_t zone = align_up(zneed, 256), keep = align_up(kneed, 256);
         if (tables) return set_error(WGC_ERR_INVALID, "batched launch group in an allocation-free plan");
-        if (zone + keep + need > kScratchBytes)
+        size_t have = std::min(kScratchBytes, dev->static_limit);
+        if (zone + keep + need > have)
             return set_error(WGC_ERR_OUT_OF_MEMORY,
                              "the command buffer needs " + std::to_string(zone + keep + need) +
-                                 " bytes of scratch; the allocation-free submission has " +
-                                 std::to_string(kScratchBytes));
+                                 " bytes of scratch; the allocation-free submission has " + std::to_string(have));
         if (!dev->scratch) return set_error(WGC_ERR_DEVICE, "no scratch address for this device");
         zone_base = dev->scratch;
         keep_base = dev->scratch + zone;
@@ -2976,15 +3042,8 @@ static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, 
         size_t keep = align_up(std::max(kneed, lane.keep_size), 4096);
         size_t grow = zone + keep + std::max(need, (size_t)64 << 20);
         if (&lane != &dev->lanes[0] && grow > kLane1Arena) return kNoLane1;
-        HIP_TRY(hipStreamSynchronize(lane.stream), "arena");
-        if (lane.arena) HIP_TRY(hipFree(lane.arena), "arena");
-        lane.arena = nullptr;
-        lane.arena_size = 0;
-        lane.arena_gen++;   // (also when the allocation fails: the old arena is gone)
-        if (hipMalloc(&lane.arena, grow) != hipSuccess) {
-            lane.arena = nullptr;
-            lane.zone_size = lane.keep_size = 0;
-            (void)hipGetLastError();
+        HIP_TRY(drop_arena(lane), "arena");
+        if (arena_malloc(dev, lane, grow) != hipSuccess) {
             if (&lane != &dev->lanes[0]) return kNoLane1;
             return set_error(WGC_ERR_OUT_OF_MEMORY, "scratch arena");
         }
@@ -3001,12 +3060,17 @@ static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, 
     // draw tables: pooled device memory, uploaded from pooled pinned staging
     // without a host wait (the upload is ordered before the plan's launches)
     if (tables) {
-        HIP_TRY(dev->table_pool.alloc(tables, plan.d_tables), "draw tables");
-        hipError_t e = dev->staging_pool.alloc(tables, plan.h_tables);
+        hipError_t e = dev->table_pool.alloc(tables, plan.d_tables);
+        if (e == hipSuccess) {
+            e = dev->staging_pool.alloc(tables, plan.h_tables);
+            if (e != hipSuccess) {
+                dev->table_pool.release(plan.d_tables, tables);
+                plan.d_tables = nullptr;
+            }
+        }
         if (e != hipSuccess) {
-            dev->table_pool.release(plan.d_tables, tables);
-            plan.d_tables = nullptr;
-            return hip_fail(e, "draw table staging");
+            int32_t r = hip_fail(e, "draw tables");
+            return merged ? WGC_ERR_OUT_OF_MEMORY : r;   // (draws one after another need none)
         }
         plan.tables_size = tables;
         plan.dev = dev;
@@ -3065,6 +3129,18 @@ static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, 
     plan.raster_cfg = cfg;
     plan.batching = dev->batching;
     return WGC_OK;
+}
+
+// Merged groups hold the scratch of all their draws at once, where draws
+// launched one after another share that of the largest: a pass for which
+// there is no memory is merged in smaller groups, and not at all in the end.
+static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, Plan &plan, bool noalloc)
+{
+    for (uint64_t merge_max = kMergedPrims;; merge_max = merge_max >= 4096 ? merge_max / 16 : 0) {
+        bool merged = false;
+        int32_t r = lay_out_plan(dev, lane, cb, plan, noalloc, merge_max, merged);
+        if (r != WGC_ERR_OUT_OF_MEMORY || !merged) return r;
+    }
 }
 
 static hipError_t launch_step(WgcDevice_T *dev, const Step &s, hipStream_t st, KernelTimer *kt)

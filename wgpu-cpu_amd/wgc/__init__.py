@@ -246,6 +246,7 @@ SIGNATURES = {
     "wgc_device_set_option": (C.c_int32, [_P, C.c_uint32, C.c_uint32]),
     "wgc_device_get_option": (C.c_int32, [_P, C.c_uint32, C.POINTER(C.c_uint32)]),
     "wgc_device_debug_fragment_counts": (C.c_int32, [_P, C.c_uint32, C.c_uint32, C.c_void_p]),
+    "wgc_device_debug_scratch_limit": (C.c_int32, [_P, C.c_uint64, C.c_uint64]),
     "wgc_device_timestamp": (C.c_int32, [_P, C.c_uint32]),
     "wgc_device_elapsed_ms": (C.c_int32, [_P, C.c_uint32, C.c_uint32, C.POINTER(C.c_float)]),
     "wgc_device_set_kernel_timing": (C.c_int32, [_P, C.c_uint32]),
@@ -756,6 +757,11 @@ class Device:
         f, n = C.c_uint64(), C.c_uint64()
         _check(self._lib.wgc_device_totals(self._ptr, C.byref(f), C.byref(n)))
         return f.value, n.value
+
+    def debug_scratch_limit(self, arena_bytes: int = 0, static_bytes: int = 0):
+        """Debug aid: limits of the scratch arenas and of the allocation-free
+        submission's scratch (0: none)."""
+        _check(self._lib.wgc_device_debug_scratch_limit(self._ptr, arena_bytes, static_bytes))
 
     def enable_fragment_counts(self, width: int, height: int):
         _check(self._lib.wgc_device_debug_fragment_counts(self._ptr, width, height, None))
