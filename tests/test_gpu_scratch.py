@@ -9,6 +9,7 @@ from oracle import bridge
 from wgc import runner, scenes
 
 from test_gpu_parity import announce, clip_color_draw, random_clip_triangles
+from test_gpu_topology import crowded_lines
 
 pytestmark = pytest.mark.gpu
 
@@ -128,3 +129,27 @@ def test_failed_submissions_beside_running_ones():
         p.submit()
     dev.poll()
     assert dev.totals()[0] - before == fragments
+
+
+@pytest.mark.parametrize("wgsl", [False, True])
+@pytest.mark.parametrize("mode", ["less", "last", "blend"])
+def test_lines_without_room(mode, wgsl):
+    """Crowded lines with their winners in global memory (2 MiB for this
+    target), without (tile bins, 1 MiB), and with records alone (0.12 MiB),
+    from an arena (64 MiB at least) and from the static scratch."""
+    announce(f"lines without room, {mode} wgsl={wgsl}")
+    dev = wgc.Device(0, wgc.SEMANTICS_EXTENDED)
+    spec = crowded_lines(1300, 512, 512, mode)
+    ref = bridge.render(spec)
+    p = runner.PreparedPass(dev, scenes.as_wgsl(spec) if wgsl else spec)
+    rng = np.random.default_rng(3)
+    for arena, static in ((0, 0), (65 * MIB, 1500 << 10), (64 * MIB + 2048, 200 << 10)):
+        dev.debug_scratch_limit(arena, static)
+        for submit in (p.submit, lambda: dev.submit_noalloc([p.command_buffer])):
+            dev.write_texture(p.res[0].color, rng.integers(0, 256, 512 * 512 * 4, dtype=np.uint8).tobytes())
+            submit()
+            check([p], [ref])
+    dev.debug_scratch_limit(0, 100 << 10)
+    with pytest.raises(wgc.WgcError) as e:
+        dev.submit_noalloc([p.command_buffer])
+    assert e.value.code == wgc.ERR_OUT_OF_MEMORY

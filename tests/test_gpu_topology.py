@@ -197,18 +197,12 @@ def test_strip_restart_format_mismatch_is_an_error(gpu_device):
         runner.render(spec, gpu_device)
 
 
-# The tiled line path: lists of up to one wave's keys, sorted in LDS, past
-# the sort's 1024 keys and past a tile's bin (256 slots here), so that the
-# tile tests every primitive; and lines of every octant around the tile edges.
-@pytest.mark.parametrize("n", [40, 200, 1300])
-@pytest.mark.parametrize("mode", ["less", "last", "blend"])
-def test_tiled_lines_crowded_tile(gpu_device, gpu_device_ext, n, mode):
-    w, h = 77, 45
+def crowded_lines(n, w, h, mode, corner=(16, 16)):
+    """n lines through the 16x16 tile at `corner`, one in eight anywhere."""
     u = scenes.splitmix_f32(6100 + n, n * 4).reshape(n, 4).astype(np.float64)
-    # through the 16x16 tile at (16, 16), one in eight anywhere
     far = (np.arange(n) % 8 == 0)[:, None]
-    a = np.where(far, u[:, 0:2] * (w, h), 17.0 + 14.0 * u[:, 0:2])
-    b = np.where(far, u[:, 2:4] * (w, h), 17.0 + 14.0 * u[:, 2:4])
+    a = np.where(far, u[:, 0:2] * (w, h), np.add(corner, 1.0) + 14.0 * u[:, 0:2])
+    b = np.where(far, u[:, 2:4] * (w, h), np.add(corner, 1.0) + 14.0 * u[:, 2:4])
     vb = np.zeros((2 * n, 8), np.float32)
     for k, p in ((0, a), (1, b)):
         vb[k::2, 0] = p[:, 0] / w * 2.0 - 1.0
@@ -217,13 +211,53 @@ def test_tiled_lines_crowded_tile(gpu_device, gpu_device_ext, n, mode):
     vb[:, 3] = 1.0
     vb[:, 4:8] = scenes.splitmix_f32(6300 + n, 2 * n * 4).reshape(-1, 4)
     vb[:, 7] = 0.4
-    depth = (wgc.LESS, True) if mode == "less" else None
+    depth = {"less": (wgc.LESS, True), "greater_equal": (wgc.GREATER_EQUAL, True),
+             "less_no_write": (wgc.LESS, False)}.get(mode)
     d = draw(vb, LINES, depth=depth, blend=wgc.BLEND_ALPHA if mode == "blend" else wgc.BLEND_REPLACE)
-    ext = mode == "blend"
-    spec = scenes.PassSpec(w, h, has_depth=depth is not None, clear_depth=1.0, draws=[d],
-                           semantics=wgc.SEMANTICS_EXTENDED if ext else wgc.SEMANTICS_REFERENCE,
+    return scenes.PassSpec(w, h, has_depth=depth is not None, clear_depth=0.5 if mode != "less" else 1.0, draws=[d],
+                           clear_color=(0.1, 0.2, 0.3, 1.0), semantics=wgc.SEMANTICS_EXTENDED,
                            name=f"crowded line tile n={n} {mode}")
-    both(spec, gpu_device_ext if ext else gpu_device)
+
+
+# The tiled line path.  Order-independent: lists within a tile's bin (64
+# slots) and past it, where the other lines go to winners in global memory.
+# In API order (256 slots on these 1024 tiles, 512 for n=8200): lists of up to one wave's keys,
+# of one sort in LDS, and past the bin, so that the tile tests every primitive.
+@pytest.mark.parametrize("n", [40, 64, 75, 240, 1300, 8200])
+@pytest.mark.parametrize("mode", ["less", "greater_equal", "less_no_write", "last", "blend"])
+def test_tiled_lines_crowded_tile(gpu_device_ext, n, mode):
+    both(crowded_lines(n, 512, 512, mode), gpu_device_ext)
+
+
+@pytest.mark.parametrize("mode", ["less", "last", "blend"])
+def test_tiled_lines_crowded_corner(gpu_device_ext, mode):
+    """The crowded tile is the target's last, partly outside it and the
+    scissor rect, on top of what the target holds."""
+    w, h = 77, 45
+    spec = crowded_lines(700, w, h, mode, corner=(64, 32))
+    spec.draws[0].scissor = (9, 5, 61, 37)
+    spec.clear_color = None
+    spec.color_init = np.random.default_rng(4).integers(0, 256, w * h * 4, dtype=np.uint8).tobytes()
+    if spec.has_depth:
+        spec.clear_depth = None
+        spec.depth_init = np.random.default_rng(5).random(w * h, dtype=np.float32).tobytes()
+    both(spec, gpu_device_ext)
+
+
+def test_ordered_points_crowded_tile(gpu_device_ext):
+    """More points in a tile than one sort takes, within its bin and past it."""
+    w, h, n = 256, 256, 90000
+    for k in (1500, 7000):
+        u = scenes.splitmix_f32(6700 + k, n * 6).reshape(n, 6)
+        vb = np.zeros((n, 8), np.float32)
+        x, y = u[:, 0] * w, u[:, 1] * h
+        x[::n // k], y[::n // k] = 32.0 + 15.9 * u[::n // k, 0], 48.0 + 15.9 * u[::n // k, 1]
+        vb[:, 0], vb[:, 1] = x / w * 2.0 - 1.0, 1.0 - y / h * 2.0
+        vb[:, 2], vb[:, 3], vb[:, 4:7], vb[:, 7] = 0.5, 1.0, u[:, 2:5], 0.4
+        spec = scenes.PassSpec(w, h, draws=[draw(vb, POINTS, depth=None, blend=wgc.BLEND_ALPHA)],
+                               clear_color=(0.1, 0.2, 0.3, 1.0), semantics=wgc.SEMANTICS_EXTENDED,
+                               name=f"crowded point tile {k}")
+        both(spec, gpu_device_ext)
 
 
 @pytest.mark.parametrize("blend", [False, True])

@@ -270,7 +270,7 @@ uint32_t lp_prep_grid(const DrawParams &d)
     return (uint32_t)((lanes + 255u) / 256u);
 }
 
-uint32_t lp_tiles_grid(const DrawParams &d) { return std::min(d.tiles_x * d.tiles_y, 1u << 20); }
+uint32_t lp_tiles_grid(const DrawParams &d) { return d.tiles_x * d.tiles_y; }   // (below 2^25)
 
 static hipError_t launch_lines_user(const UserKernels &k, const DrawParams &d0, const GroupLaunch &gl, hipStream_t st,
                                     KernelTimer *kt)

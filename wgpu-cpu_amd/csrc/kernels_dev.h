@@ -2525,10 +2525,17 @@ struct LineWalk {
         sc = dc < 0 ? -1 : 1;
     }
     __device__ __forceinline__ uint32_t steps() const { return min(n, kLineSteps); }   // none: nothing is drawn
-    // (a * b + c) / d
+    // (a * b + c) / d.  In the longer line's 60 bits the quotient, below 2^30,
+    // is estimated in binary64 (within one of it) and corrected by its
+    // remainder: a tenth of the general 64-bit division's code, which cost
+    // every line draw a microsecond.
     __device__ __forceinline__ uint32_t ratio(uint32_t a, uint32_t b, uint32_t c, uint32_t d) const
     {
-        return n <= kLineSteps ? (a * b + c) / d : (uint32_t)(((uint64_t)a * b + c) / d);
+        if (n <= kLineSteps) return (a * b + c) / d;
+        uint64_t x = (uint64_t)a * b + c;
+        uint32_t e = (uint32_t)((double)x / (double)d);
+        int64_t r = (int64_t)(x - (uint64_t)e * d);
+        return r < 0 ? e - 1u : (r >= (int64_t)d ? e + 1u : e);
     }
     __device__ __forceinline__ uint32_t rise(uint32_t k) const { return ratio(k, q, 0u, n); }
     __device__ __forceinline__ int32_t minor(uint32_t k) const { return c0 + sc * (int32_t)rise(k); }
@@ -2726,20 +2733,110 @@ constexpr uint32_t kNoPoint = 0xFFFFFFFFu;
 // length is made of, so they are spread over lanes rather than walked.
 constexpr uint32_t kLpLanes = 8;
 
-__device__ __forceinline__ void lp_bin(const DrawParams &d, uint32_t tile, uint32_t p, bool has)
+// The primitive's place among the tile's, in its bin if there is room (0
+// where the draw has no bins).  The lanes on the first one's tile take theirs
+// together, since lines that crowd one tile meet on its counter (20000 lines
+// in 14x14 px: prep 261 us with an atomic each, 125 so).
+__device__ __forceinline__ uint32_t lp_bin(const DrawParams &d, uint32_t tile, uint32_t p)
 {
-    if (!has) return;
-    uint32_t slot = atomicAdd(&d.s.tile_count[tile], 1u);
+    if (!d.s.bin_cap) return 0u;
+    bool mine = tile == (uint32_t)__builtin_amdgcn_readfirstlane(tile);
+    uint64_t same = __ballot(mine);
+    uint32_t rank = (uint32_t)__popcll(same & lanes_below()), slot = 0u;
+    if (!mine || rank == 0u) slot = atomicAdd(&d.s.tile_count[tile], mine ? (uint32_t)__popcll(same) : 1u);
+    if (mine) slot = (uint32_t)__builtin_amdgcn_readfirstlane(slot) + rank;
     if (slot < d.s.bin_cap) d.s.bins[(size_t)tile * d.s.bin_cap + slot] = p;
+    return slot;
 }
 
-template <int PROG, int N>
-__global__ __launch_bounds__(256) void k_lp_prep(DrawParams d, LpRec<N> *recs)
+// The coefficient of a line's second end point at t (raster.rs:251-254: the
+// lerp of the clip alphas), and one component of the fragment, the
+// coefficient applied to the clipped end points.
+__device__ __forceinline__ float lp_coefficient(const float *al, float t)
 {
-    constexpr uint32_t LANES = N == 1 ? 1u : kLpLanes;
-    uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t p = g / LANES, sub = g % LANES;
-    if (p >= d.total_prims) return;
+    float u = 1.0f - t;
+    float l0 = al[0] * u;
+    float l1 = al[1] * t;
+    return l0 + l1;
+}
+
+__device__ __forceinline__ float lp_lerp(float from, float to, float L)
+{
+    float mv = 1.0f - L;
+    float a = from * mv;
+    float b = to * L;
+    return a + b;
+}
+
+// The fragment of a record (as words) at t (points: any): its depth and
+// position, and the vertices its varyings come from.
+template <int N>
+__device__ __forceinline__ void lp_fragment(const float *rf, float t, VsOut (&v)[N], LpFrag &f)
+{
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        v[k].clip[0] = v[k].clip[1] = v[k].clip[2] = 0.0f;
+        v[k].clip[3] = rf[6 * N + kMaxVar * N + k];
+#pragma unroll
+        for (int c = 0; c < kMaxVar; ++c) v[k].var[c] = rf[6 * N + k * kMaxVar + c];
+    }
+    f.L = N == 1 ? 0.0f : lp_coefficient(rf + N * 6 + N * kMaxVar + N, t);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) f.pos[c] = N == 1 ? rf[2 + c] : lp_lerp(rf[2 * N + c], rf[2 * N + 4 + c], f.L);
+    f.z = f.pos[2];
+}
+
+// A line's fragments in one tile, straight to the tile's winners in global
+// memory (complemented, so that zero means none): what an order-independent
+// tile does with the lines that its bin has no slot for.  `slot`: the line's
+// place in the tile.  `t` is the line's t at step `at`, and is left at the step
+// past the tile.  The line's steps come in ascending order.
+__device__ __forceinline__ uint32_t lp_overflow(const DrawParams &d, const LpRec<2> &r, const LineWalk &w, uint32_t p,
+                                                int32_t tx, int32_t ty, uint32_t slot, float &t, uint32_t &at)
+{
+    int32_t x0 = tx * (int32_t)kLpTile, y0 = ty * (int32_t)kLpTile;
+    int32_t sx1 = (int32_t)(d.scissor[0] + d.scissor[2]), sy1 = (int32_t)(d.scissor[1] + d.scissor[3]);
+    uint32_t k = 0;
+    uint32_t n = w.steps_inside(max(x0, (int32_t)d.scissor[0]), max(y0, (int32_t)d.scissor[1]),
+                                min(x0 + (int32_t)kLpTile, sx1) - 1, min(y0 + (int32_t)kLpTile, sy1) - 1, k);
+    if (!n) return 0u;
+    float dt = 1.0f / (float)w.n;
+    t = lp_time(t, dt, k - at);
+    at = k + n;
+    uint32_t quo = w.rise(k), rem = k * w.q - quo * w.n;
+    int32_t m = w.m0 + w.sm * (int32_t)k, c = w.c0 + w.sc * (int32_t)quo;
+    unsigned long long *win = d.s.gvis + ((size_t)ty * d.tiles_x + (uint32_t)tx) * (kLpTile * kLpTile);
+    bool clears = d.init_clear && d.clear_depth_on;
+    for (uint32_t j = 0; j < n; ++j) {
+        uint32_t x = (uint32_t)(w.xmajor ? m : c), y = (uint32_t)(w.xmajor ? c : m);
+        uint32_t pix = y * d.width + x;
+        lp_count_fragment(d, pix);
+        float z = lp_lerp(r.fr[0][2], r.fr[1][2], lp_coefficient(r.al, t));
+        float init = clears ? d.clear_depth : (d.depth ? d.depth[pix] : 0.0f);
+        uint32_t key = lp_key(p, k + j, 2);
+        if (oi_pass(d, z, init)) {
+            unsigned long long v = ~(d.resolve == RES_LAST ? (unsigned long long)(~key) : oi_value(d.resolve, z, key));
+            unsigned long long *px = &win[(y % kLpTile) * kLpTile + x % kLpTile];
+            // (winners only grow, so one that is too small for what was there
+            // some time ago cannot win; 20000 lines in 14x14 px, the atomics
+            // queue: prep 125 -> 46 us; with few the read is one wait a step)
+            if (slot < kLineCrowd || v > *px) atomicMax(px, v);
+        }
+        t = t + dt;
+        m += w.sm;
+        rem += w.q;
+        if (rem >= w.n) {
+            rem -= w.n;
+            c += w.sc;
+        }
+    }
+    return n;
+}
+
+// Returns the fragments that went past full bins.
+template <int PROG, int N>
+__device__ __forceinline__ uint32_t lp_prep(const DrawParams &d, LpRec<N> *recs, uint32_t p, uint32_t sub)
+{
     VsOut v[N];
     LpSetup s;
     bool ok = shade_primitive<PROG, N>(d, p, v) && lp_setup<N>(d, v, s) && s.visible;
@@ -2762,36 +2859,58 @@ __global__ __launch_bounds__(256) void k_lp_prep(DrawParams d, LpRec<N> *recs)
         if (N == 1) r.fb[0][0] = r.fb[0][1] = kNoPoint;
     }
     if (sub == 0u) recs[p] = r;
-    if (!ok) return;
+    if (!ok) return 0u;
     // a line of more than kLineSteps steps is an error, wherever they fall
     if constexpr (N == 2)
         if (LineWalk(r.fb[0], r.fb[1]).n > kLineSteps) atomicOr(d.s.error, (uint32_t)ERR_COORD_RANGE);
-    if (!d.scissor[2] || !d.scissor[3]) return;
+    if (!d.s.tile_count || !d.scissor[2] || !d.scissor[3]) return 0u;
     // the tiles that meet the scissor rect (inside the target, checked by the host)
     int32_t sx0 = (int32_t)(d.scissor[0] / kLpTile), sx1 = (int32_t)((d.scissor[0] + d.scissor[2] - 1u) / kLpTile);
     int32_t sy0 = (int32_t)(d.scissor[1] / kLpTile), sy1 = (int32_t)((d.scissor[1] + d.scissor[3] - 1u) / kLpTile);
     if constexpr (N == 1) {
         int32_t tx = (int32_t)(r.fb[0][0] / kLpTile), ty = (int32_t)(r.fb[0][1] / kLpTile);
-        lp_bin(d, (uint32_t)ty * d.tiles_x + (uint32_t)tx, p, tx >= sx0 && tx <= sx1 && ty >= sy0 && ty <= sy1);
+        if (tx >= sx0 && tx <= sx1 && ty >= sy0 && ty <= sy1) (void)lp_bin(d, (uint32_t)ty * d.tiles_x + (uint32_t)tx, p);
+        return 0u;
     } else {
         LineWalk w(r.fb[0], r.fb[N - 1]);
-        if (!w.n) return;
+        if (!w.n) return 0u;
         int32_t ma = w.m0, mb = w.m0 + w.sm * (int32_t)(w.steps() - 1u);
         int32_t lo = w.xmajor ? sx0 : sy0, hi = w.xmajor ? sx1 : sy1;          // scissor, major
         int32_t clo = w.xmajor ? sy0 : sx0, chi = w.xmajor ? sy1 : sx1;        // scissor, minor
         int32_t t0 = max(min(ma, mb) / (int32_t)kLpTile, lo), t1 = min(max(ma, mb) / (int32_t)kLpTile, hi);
-        for (int32_t t = t0 + (int32_t)sub; t <= t1; t += (int32_t)kLpLanes) {
+        float time = 0.0f;
+        uint32_t at = 0u, frags = 0u;
+        for (int32_t i = (int32_t)sub; i <= t1 - t0; i += (int32_t)kLpLanes) {
             // the steps in this column of tiles: fewer than kLpTile pixels
             // along the minor axis, so at most two tiles
+            int32_t t = w.sm > 0 ? t0 + i : t1 - i;   // in the order of the line's steps
             int32_t k0, k1;
             w.major_steps(t * (int32_t)kLpTile, t * (int32_t)kLpTile + (int32_t)kLpTile - 1, k0, k1);
             int32_t ca = w.minor((uint32_t)k0) / (int32_t)kLpTile, cb = w.minor((uint32_t)k1) / (int32_t)kLpTile;
-            uint32_t ta = (uint32_t)(w.xmajor ? ca * (int32_t)d.tiles_x + t : t * (int32_t)d.tiles_x + ca);
-            uint32_t tb = (uint32_t)(w.xmajor ? cb * (int32_t)d.tiles_x + t : t * (int32_t)d.tiles_x + cb);
-            lp_bin(d, ta, p, ca >= clo && ca <= chi);
-            lp_bin(d, tb, p, cb != ca && cb >= clo && cb <= chi);
+#pragma unroll 1
+            for (int32_t c = ca;; c = cb) {
+                if (c >= clo && c <= chi) {
+                    int32_t tx = w.xmajor ? t : c, ty = w.xmajor ? c : t;
+                    uint32_t slot = lp_bin(d, (uint32_t)ty * d.tiles_x + (uint32_t)tx, p);
+                    if (slot >= d.s.bin_cap && d.s.gvis) frags += lp_overflow(d, r, w, p, tx, ty, slot, time, at);
+                }
+                if (c == cb) break;
+            }
         }
+        return frags;
     }
+}
+
+template <int PROG, int N>
+__global__ __launch_bounds__(256) void k_lp_prep(DrawParams d, LpRec<N> *recs)
+{
+    constexpr uint32_t LANES = N == 1 ? 1u : kLpLanes;
+    uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t p = g / LANES, sub = g % LANES;
+    uint32_t frags = p < d.total_prims ? lp_prep<PROG, N>(d, recs, p, sub) : 0u;
+    if (N == 1 || !__ballot(frags != 0u)) return;
+    for (int off = 32; off > 0; off >>= 1) frags += (uint32_t)__shfl_xor((int)frags, off);
+    if (lane_id() == 0u) atomicAdd(&d.s.frags[(g / 64u) % kFragSlots], (unsigned long long)frags);
 }
 
 // Sorts list[0..total) ascending by one wave (the workgroup): up to 64 keys
@@ -2831,8 +2950,11 @@ __device__ __forceinline__ void sort_wave(uint32_t *list, uint32_t total)
 // shader that may discard): the keys are sorted, fragments stand in API
 // order, and of the lanes that hold the same pixel the lowest goes first,
 // round by round (mostly one round).  Otherwise the winner of each pixel is
-// the minimum of oi_value in LDS.  A tile whose list does not fit its bin
-// (or, ordered, the sort) tests every primitive's bounds instead.
+// the minimum of oi_value in LDS, and of the winners that k_lp_prep left in
+// global memory for the lines past a full bin (lp_overflow); such a tile
+// shades each pixel's winner once at the end, from its key.  Without those
+// winners (ordered, points, no memory for them), a tile whose list does not
+// fit its bin, or the sort, tests every primitive's bounds.
 // Bound by latency: a tile has a handful of lines, so what counts is the
 // chain (count, keys, records, walk, fragments, store) and how many tiles
 // are in flight; its VALU work is about a third of the kernel's time.
@@ -2841,7 +2963,10 @@ __device__ __forceinline__ void sort_wave(uint32_t *list, uint32_t total)
 // from its first step with one thread: 1191 us); 1920x1080, 20000
 // depth-tested lines of about 80 px, 33 us (two passes of a lane per line
 // walking over a visibility buffer of the target, and its fill and the
-// clear: 324 us).  Batches of 24 or 32 lines (12 KB of LDS per wave instead
+// clear: 324 us).  With a wave for any list, lines that crowded few tiles took
+// longer than over the visibility buffer: 20000 in 14x14 px of 1080p 84 us
+// there, 3980 by one wave, 100 with winners in global memory; 20000 of 20 px
+// over 256x256 66, 107 and 47 us.  Batches of 24 or 32 lines (12 KB of LDS per wave instead
 // of 9) give 57 and 54 us a pass against 52 on the second, 41 and 40 against
 // 41 on the first.
 template <int PROG, int N, bool ORDERED>
@@ -2877,215 +3002,219 @@ __global__ __launch_bounds__(64) void k_lp_tiles(DrawParams d, const LpRec<N> *r
     __shared__ float dep[PX];
     uint32_t lane = threadIdx.x;
     uint32_t frags = 0;
-    uint32_t n_tiles = d.tiles_x * d.tiles_y;
     uint32_t sx1 = d.scissor[0] + d.scissor[2], sy1 = d.scissor[1] + d.scissor[3];   // inside the target
-    for (uint32_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        uint32_t cnt = d.s.tile_count[tile];
-        __syncthreads();   // every lane has the count (and is done with the last tile)
-        if (cnt && lane == 0u) d.s.tile_count[tile] = 0u;   // kept zero between uses
-        bool clears = d.init_clear && (d.clear_color_on || d.clear_depth_on);
-        if (!cnt && !clears) continue;
-        uint32_t x0 = (tile % d.tiles_x) * TS, y0 = (tile / d.tiles_x) * TS;
-        uint32_t x1 = min(x0 + TS, d.width) - 1u, y1 = min(y0 + TS, d.height) - 1u;
-        bool cc = d.init_clear && d.clear_color_on, cd = d.init_clear && d.clear_depth_on;
+    uint32_t tile = blockIdx.x;
+    uint32_t cnt = d.s.tile_count && d.s.bin_cap ? d.s.tile_count[tile] : 0xFFFFFFFFu;
+    __syncthreads();   // every lane has the count
+    if (cnt && d.s.tile_count && d.s.bin_cap && lane == 0u) d.s.tile_count[tile] = 0u;   // kept zero between uses
+    bool clears = d.init_clear && (d.clear_color_on || d.clear_depth_on);
+    if (!cnt && !clears) return;
+    uint32_t x0 = (tile % d.tiles_x) * TS, y0 = (tile / d.tiles_x) * TS;
+    uint32_t x1 = min(x0 + TS, d.width) - 1u, y1 = min(y0 + TS, d.height) - 1u;
+    bool cc = d.init_clear && d.clear_color_on, cd = d.init_clear && d.clear_depth_on;
+    const bool over = !ORDERED && N == 2 && d.s.gvis && cnt > d.s.bin_cap;
 #pragma unroll
-        for (uint32_t k = 0; k < PX / 64u; ++k) {
-            uint32_t q = lane + k * 64u, px = x0 + q % TS, py = y0 + q / TS;
-            size_t pix = (size_t)py * d.width + px;
-            bool in = cnt && px <= x1 && py <= y1;
-            uint32_t c = d.clear_rgba;
-            float z = cd ? d.clear_depth : 0.0f;
-            if (in && d.color && !cc && ORDERED) c = reinterpret_cast<const uint32_t *>(d.color)[pix];
-            if (in && d.depth && !cd) z = d.depth[pix];
-            col[q] = c;
-            dep[q] = z;
-            if constexpr (ORDERED) claim[q] = 0xFFFFFFFFu;
-            else best[q] = ~0ull;
+    for (uint32_t k = 0; k < PX / 64u; ++k) {
+        uint32_t q = lane + k * 64u, px = x0 + q % TS, py = y0 + q / TS;
+        size_t pix = (size_t)py * d.width + px;
+        bool in = cnt && px <= x1 && py <= y1;
+        uint32_t c = d.clear_rgba;
+        float z = cd ? d.clear_depth : 0.0f;
+        if (in && d.color && !cc && ORDERED) c = reinterpret_cast<const uint32_t *>(d.color)[pix];
+        if (in && d.depth && !cd) z = d.depth[pix];
+        col[q] = c;
+        dep[q] = z;
+        if constexpr (ORDERED) {
+            claim[q] = 0xFFFFFFFFu;
+        } else {
+            unsigned long long g = 0ull;
+            if (over) {
+                unsigned long long *win = d.s.gvis + (size_t)tile * PX + q;
+                g = *win;
+                if (g) *win = 0ull;   // kept zero between uses
+            }
+            best[q] = ~g;
         }
-        // the tile's primitives: its bin, or every primitive of the draw
-        bool list = cnt <= d.s.bin_cap && (!ORDERED || cnt <= kLpSort);
-        uint32_t *bin = d.s.bins + (size_t)tile * d.s.bin_cap;
-        if (ORDERED && list && cnt > 1u) {
-            // sorted in place (a lane reads back the slots it writes)
-            for (uint32_t i = lane; i < cnt; i += 64u) sh.sort[i] = bin[i];
+    }
+    // the tile's primitives: its bin (what did not fit there is among the
+    // winners above), or every primitive of the draw
+    bool list = (cnt <= d.s.bin_cap && (!ORDERED || cnt <= kLpSort)) || over;
+    uint32_t *bin = d.s.bins + (size_t)tile * d.s.bin_cap;
+    if (ORDERED && list && cnt > 1u) {
+        // sorted in place (a lane reads back the slots it writes)
+        for (uint32_t i = lane; i < cnt; i += 64u) sh.sort[i] = bin[i];
+        __syncthreads();
+        sort_wave(sh.sort, cnt);
+        for (uint32_t i = lane; i < cnt; i += 64u) bin[i] = sh.sort[i];
+        __syncthreads();
+    }
+    uint32_t total = list ? min(cnt, d.s.bin_cap) : d.total_prims;
+    for (uint32_t sweep = 0; sweep < (over ? 1u : SWEEPS); ++sweep)
+        for (uint32_t at = 0; at < total; at += 64u) {
+            uint32_t nk = min(64u, total - at);
+            if (list) {
+                if (lane < nk) keys[lane] = bin[at + lane];
+            } else {
+                bool t = false;
+                if (lane < nk) {
+                    const LpRec<N> &r = recs[at + lane];
+                    uint32_t ax = r.fb[0][0], ay = r.fb[0][1], bx = r.fb[N - 1][0], by = r.fb[N - 1][1];
+                    t = min(ax, bx) <= x1 && max(ax, bx) >= x0 && min(ay, by) <= y1 && max(ay, by) >= y0;
+                }
+                uint64_t m = __ballot(t);
+                if (t) keys[__popcll(m & lanes_below())] = at + lane;
+                nk = (uint32_t)__popcll(m);
+            }
             __syncthreads();
-            sort_wave(sh.sort, cnt);
-            for (uint32_t i = lane; i < cnt; i += 64u) bin[i] = sh.sort[i];
-            __syncthreads();
-        }
-        uint32_t total = list ? cnt : d.total_prims;
-        for (uint32_t sweep = 0; sweep < SWEEPS; ++sweep)
-            for (uint32_t at = 0; at < total; at += 64u) {
-                uint32_t nk = min(64u, total - at);
-                if (list) {
-                    if (lane < nk) keys[lane] = bin[at + lane];
-                } else {
-                    bool t = false;
-                    if (lane < nk) {
-                        const LpRec<N> &r = recs[at + lane];
-                        uint32_t ax = r.fb[0][0], ay = r.fb[0][1], bx = r.fb[N - 1][0], by = r.fb[N - 1][1];
-                        t = min(ax, bx) <= x1 && max(ax, bx) >= x0 && min(ay, by) <= y1 && max(ay, by) >= y0;
-                    }
-                    uint64_t m = __ballot(t);
-                    if (t) keys[__popcll(m & lanes_below())] = at + lane;
-                    nk = (uint32_t)__popcll(m);
+            for (uint32_t b = 0; b < nk; b += LINES) {
+                uint32_t nl = min(LINES, nk - b);
+                for (uint32_t i = lane; i < nl * QUADS; i += 64u) {
+                    uint32_t l = i / QUADS, part = i % QUADS;
+                    uint4 v = reinterpret_cast<const uint4 *>(recs + keys[b + l])[part];
+                    uint32_t *o = st + l * STRIDE + part * 4u;
+                    o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
                 }
                 __syncthreads();
-                for (uint32_t b = 0; b < nk; b += LINES) {
-                    uint32_t nl = min(LINES, nk - b);
-                    for (uint32_t i = lane; i < nl * QUADS; i += 64u) {
-                        uint32_t l = i / QUADS, part = i % QUADS;
-                        uint4 v = reinterpret_cast<const uint4 *>(recs + keys[b + l])[part];
-                        uint32_t *o = st + l * STRIDE + part * 4u;
-                        o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
-                    }
-                    __syncthreads();
-                    // a lane per primitive: its fragments inside the tile and
-                    // the scissor rect
-                    uint32_t nf = 0, k0 = 0;
-                    const uint32_t *mine = st + (lane < nl ? lane : 0u) * STRIDE;
-                    LineWalk w(mine, mine + (N == 1 ? 0 : 2));
-                    int32_t cx0 = (int32_t)max(x0, d.scissor[0]), cx1 = (int32_t)min(x1 + 1u, sx1) - 1;
-                    int32_t cy0 = (int32_t)max(y0, d.scissor[1]), cy1 = (int32_t)min(y1 + 1u, sy1) - 1;
-                    if (lane < nl && cx0 <= cx1 && cy0 <= cy1) {
-                        if constexpr (N == 1)
-                            nf = mine[0] >= (uint32_t)cx0 && mine[0] <= (uint32_t)cx1 && mine[1] >= (uint32_t)cy0 &&
-                                         mine[1] <= (uint32_t)cy1 ? 1u : 0u;
-                        else if (w.n) nf = w.steps_inside(cx0, cy0, cx1, cy1, k0);
-                    }
-                    uint32_t sum = wave_inclusive_sum(nf);
-                    uint32_t n_frag = lane_value(sum, 63);
-                    if constexpr (N == 1) {
-                        if (nf) flist[sum - 1u] = lane | (((mine[1] - y0) * TS + (mine[0] - x0)) << 8);
-                    } else if (nf) {
-                        first[lane] = k0;
-                        float dt = 1.0f / (float)w.n, t = lp_time(0.0f, dt, k0);
-                        uint32_t quo = w.rise(k0), rem = k0 * w.q - quo * w.n;
-                        int32_t m = w.m0 + w.sm * (int32_t)k0 - (int32_t)(w.xmajor ? x0 : y0);
-                        int32_t c = w.c0 + w.sc * (int32_t)quo - (int32_t)(w.xmajor ? y0 : x0);
-                        for (uint32_t j = 0, o = sum - nf; j < nf; ++j, ++o) {
-                            flist[o] = lane | ((uint32_t)(w.xmajor ? c * (int32_t)TS + m : m * (int32_t)TS + c) << 8) |
-                                       (j << 16);
-                            time[o] = t;
-                            t = t + dt;
-                            m += w.sm;
-                            rem += w.q;
-                            if (rem >= w.n) {
-                                rem -= w.n;
-                                c += w.sc;
-                            }
+                // a lane per primitive: its fragments inside the tile and
+                // the scissor rect
+                uint32_t nf = 0, k0 = 0;
+                const uint32_t *mine = st + (lane < nl ? lane : 0u) * STRIDE;
+                LineWalk w(mine, mine + (N == 1 ? 0 : 2));
+                int32_t cx0 = (int32_t)max(x0, d.scissor[0]), cx1 = (int32_t)min(x1 + 1u, sx1) - 1;
+                int32_t cy0 = (int32_t)max(y0, d.scissor[1]), cy1 = (int32_t)min(y1 + 1u, sy1) - 1;
+                if (lane < nl && cx0 <= cx1 && cy0 <= cy1) {
+                    if constexpr (N == 1)
+                        nf = mine[0] >= (uint32_t)cx0 && mine[0] <= (uint32_t)cx1 && mine[1] >= (uint32_t)cy0 &&
+                                     mine[1] <= (uint32_t)cy1 ? 1u : 0u;
+                    else if (w.n) nf = w.steps_inside(cx0, cy0, cx1, cy1, k0);
+                }
+                uint32_t sum = wave_inclusive_sum(nf);
+                uint32_t n_frag = lane_value(sum, 63);
+                if constexpr (N == 1) {
+                    if (nf) flist[sum - 1u] = lane | (((mine[1] - y0) * TS + (mine[0] - x0)) << 8);
+                } else if (nf) {
+                    first[lane] = k0;
+                    float dt = 1.0f / (float)w.n, t = lp_time(0.0f, dt, k0);
+                    uint32_t quo = w.rise(k0), rem = k0 * w.q - quo * w.n;
+                    int32_t m = w.m0 + w.sm * (int32_t)k0 - (int32_t)(w.xmajor ? x0 : y0);
+                    int32_t c = w.c0 + w.sc * (int32_t)quo - (int32_t)(w.xmajor ? y0 : x0);
+                    for (uint32_t j = 0, o = sum - nf; j < nf; ++j, ++o) {
+                        flist[o] = lane | ((uint32_t)(w.xmajor ? c * (int32_t)TS + m : m * (int32_t)TS + c) << 8) |
+                                   (j << 16);
+                        time[o] = t;
+                        t = t + dt;
+                        m += w.sm;
+                        rem += w.q;
+                        if (rem >= w.n) {
+                            rem -= w.n;
+                            c += w.sc;
                         }
                     }
-                    __syncthreads();
-                    // a lane per fragment
-                    for (uint32_t f0 = 0; f0 < n_frag; f0 += 64u) {
-                        bool valid = f0 + lane < n_frag;
-                        uint32_t e = valid ? flist[f0 + lane] : 0u;
-                        uint32_t l = e & 255u, q = (e >> 8) & 255u, j = e >> 16;
-                        const float *rf = reinterpret_cast<const float *>(st + l * STRIDE);
-                        uint32_t p = keys[b + l];
-                        LpFrag f;
-                        f.x = x0 + q % TS;
-                        f.y = y0 + q / TS;
-                        VsOut v[N];
-#pragma unroll
-                        for (int k = 0; k < N; ++k) {
-                            v[k].clip[0] = v[k].clip[1] = v[k].clip[2] = 0.0f;
-                            v[k].clip[3] = rf[6 * N + kMaxVar * N + k];
-#pragma unroll
-                            for (int c = 0; c < kMaxVar; ++c) v[k].var[c] = rf[6 * N + k * kMaxVar + c];
+                }
+                __syncthreads();
+                // a lane per fragment
+                for (uint32_t f0 = 0; f0 < n_frag; f0 += 64u) {
+                    bool valid = f0 + lane < n_frag;
+                    uint32_t e = valid ? flist[f0 + lane] : 0u;
+                    uint32_t l = e & 255u, q = (e >> 8) & 255u, j = e >> 16;
+                    const float *rf = reinterpret_cast<const float *>(st + l * STRIDE);
+                    uint32_t p = keys[b + l];
+                    LpFrag f;
+                    f.x = x0 + q % TS;
+                    f.y = y0 + q / TS;
+                    VsOut v[N];
+                    f.k = N == 1 ? 0u : first[l] + j;
+                    lp_fragment<N>(rf, N == 1 || !valid ? 0.0f : time[f0 + lane], v, f);
+                    if (valid && sweep == 0u) {
+                        ++frags;
+                        lp_count_fragment(d, f.y * d.width + f.x);
+                    }
+                    if constexpr (!ORDERED) {
+                        uint32_t key = lp_key(p, f.k, N);
+                        bool pass = valid && oi_pass(d, f.z, dep[q]);
+                        unsigned long long val =
+                            d.resolve == RES_LAST ? (unsigned long long)(~key) : oi_value(d.resolve, f.z, key);
+                        if (pass && sweep == 0u) atomicMin(&best[q], val);
+                        __syncthreads();
+                        // the pixel's winner so far (of this wave's fragments,
+                        // one lane: values are distinct) shades it
+                        if (pass && !over && sweep == SWEEPS - 1u && best[q] == val) {
+                            float color[4];
+                            float unused = f.z;
+                            (void)lp_color<PROG, N>(d, v, f, p, color, &unused);
+                            col[q] = pack_color(color, d.color_bgra);
+                            zwin[q] = f.z;
                         }
-                        if constexpr (N == 1) {
-                            f.k = 0u;
-                            f.L = 0.0f;
-#pragma unroll
-                            for (int c = 0; c < 4; ++c) f.pos[c] = rf[2 + c];
-                        } else {
-                            f.k = first[l] + j;
-                            float t = valid ? time[f0 + lane] : 0.0f;
-                            // raster.rs:251-254: L = lerp of the clip alphas; the
-                            // fragment is L applied to the clipped end points
-                            float u = 1.0f - t;
-                            float l0 = rf[N * 6 + N * kMaxVar + N] * u;
-                            float l1 = rf[N * 6 + N * kMaxVar + N + 1] * t;
-                            f.L = l0 + l1;
-                            float mv = 1.0f - f.L;
-#pragma unroll
-                            for (int c = 0; c < 4; ++c) {
-                                float a = rf[2 * N + c] * mv;
-                                float bb = rf[2 * N + 4 + c] * f.L;
-                                f.pos[c] = a + bb;
-                            }
+                        __syncthreads();
+                    } else {
+                        float color[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                        if constexpr (PROG != PROG_USER) {
+                            // the built-in shaders have no side effects and
+                            // do not abort: once for all rounds
+                            float unused = f.z;
+                            (void)lp_color<PROG, N>(d, v, f, p, color, &unused);
                         }
-                        f.z = f.pos[2];
-                        if (valid && sweep == 0u) {
-                            ++frags;
-                            lp_count_fragment(d, f.y * d.width + f.x);
-                        }
-                        if constexpr (!ORDERED) {
-                            uint32_t key = lp_key(p, f.k, N);
-                            bool pass = valid && oi_pass(d, f.z, dep[q]);
-                            unsigned long long val =
-                                d.resolve == RES_LAST ? (unsigned long long)(~key) : oi_value(d.resolve, f.z, key);
-                            if (pass && sweep == 0u) atomicMin(&best[q], val);
+                        for (bool pending = valid; __ballot(pending);) {
+                            if (pending) atomicMin(&claim[q], lane);
                             __syncthreads();
-                            // the pixel's winner so far (of this wave's fragments,
-                            // one lane: values are distinct) shades it
-                            if (pass && sweep == SWEEPS - 1u && best[q] == val) {
-                                float color[4];
-                                float unused = f.z;
-                                (void)lp_color<PROG, N>(d, v, f, p, color, &unused);
-                                col[q] = pack_color(color, d.color_bgra);
-                                zwin[q] = f.z;
+                            bool mine = pending && claim[q] == lane;
+                            __syncthreads();
+                            if (mine) {
+                                float z = dep[q];
+                                bool ok = depth_and_shade(d, f.z, z, [&](float *frag_depth) {
+                                    if constexpr (PROG == PROG_USER)
+                                        return lp_color<PROG, N>(d, v, f, p, color, frag_depth);
+                                    else return true;
+                                });
+                                if (d.depth_test && d.depth_write) dep[q] = z;
+                                if (ok)
+                                    col[q] = d.blend ? blend_over(color, col[q], d.color_bgra)
+                                                     : pack_color(color, d.color_bgra);
+                                claim[q] = 0xFFFFFFFFu;
+                                pending = false;
                             }
                             __syncthreads();
-                        } else {
-                            float color[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                            if constexpr (PROG != PROG_USER) {
-                                // the built-in shaders have no side effects and
-                                // do not abort: once for all rounds
-                                float unused = f.z;
-                                (void)lp_color<PROG, N>(d, v, f, p, color, &unused);
-                            }
-                            for (bool pending = valid; __ballot(pending);) {
-                                if (pending) atomicMin(&claim[q], lane);
-                                __syncthreads();
-                                bool mine = pending && claim[q] == lane;
-                                __syncthreads();
-                                if (mine) {
-                                    float z = dep[q];
-                                    bool ok = depth_and_shade(d, f.z, z, [&](float *frag_depth) {
-                                        if constexpr (PROG == PROG_USER)
-                                            return lp_color<PROG, N>(d, v, f, p, color, frag_depth);
-                                        else return true;
-                                    });
-                                    if (d.depth_test && d.depth_write) dep[q] = z;
-                                    if (ok)
-                                        col[q] = d.blend ? blend_over(color, col[q], d.color_bgra)
-                                                         : pack_color(color, d.color_bgra);
-                                    claim[q] = 0xFFFFFFFFu;
-                                    pending = false;
-                                }
-                                __syncthreads();
-                            }
                         }
                     }
                 }
             }
-        // the pixels the pass changes (ordered: the whole tile, which is this
-        // wave's own)
-#pragma unroll
-        for (uint32_t k = 0; k < PX / 64u; ++k) {
-            uint32_t q = lane + k * 64u, px = x0 + q % TS, py = y0 + q / TS;
-            if (px > x1 || py > y1) continue;
-            size_t pix = (size_t)py * d.width + px;
-            bool won = ORDERED ? cnt != 0u : best[ORDERED ? 0u : q] != ~0ull;
-            float z = dep[q];
-            if (!ORDERED && won) z = zwin[ORDERED ? 0u : q];
-            if (d.color && (won || cc)) store_color(d, pix, won ? col[q] : d.clear_rgba);
-            if (d.depth && ((won && d.depth_test && d.depth_write) || cd))
-                store_depth(d, pix, won && d.depth_test && d.depth_write ? z : (ORDERED ? dep[q] : d.clear_depth));
         }
+    if constexpr (!ORDERED && N == 2) {
+        // a tile whose bin was full: every winner known, each shaded once
+        if (over) {
+            for (uint32_t k = 0; k < PX / 64u; ++k) {
+                uint32_t q = lane + k * 64u;
+                if (best[q] == ~0ull) continue;
+                uint32_t key = oi_key(d.resolve, best[q]), p = key >> 13;
+                const float *rf = reinterpret_cast<const float *>(recs + p);
+                const uint32_t *ends = reinterpret_cast<const uint32_t *>(recs + p);
+                LpFrag f;
+                f.x = x0 + q % TS;
+                f.y = y0 + q / TS;
+                f.k = key & 8191u;
+                VsOut v[N];
+                lp_fragment<N>(rf, lp_time(0.0f, 1.0f / (float)LineWalk(ends, ends + 2).n, f.k), v, f);
+                float color[4];
+                float unused = f.z;
+                (void)lp_color<PROG, N>(d, v, f, p, color, &unused);
+                col[q] = pack_color(color, d.color_bgra);
+                zwin[q] = f.z;
+            }
+        }
+    }
+    // the pixels the pass changes (ordered: the whole tile, which is this
+    // wave's own)
+#pragma unroll
+    for (uint32_t k = 0; k < PX / 64u; ++k) {
+        uint32_t q = lane + k * 64u, px = x0 + q % TS, py = y0 + q / TS;
+        if (px > x1 || py > y1) continue;
+        size_t pix = (size_t)py * d.width + px;
+        bool won = ORDERED ? cnt != 0u : best[ORDERED ? 0u : q] != ~0ull;
+        float z = dep[q];
+        if (!ORDERED && won) z = zwin[ORDERED ? 0u : q];
+        if (d.color && (won || cc)) store_color(d, pix, won ? col[q] : d.clear_rgba);
+        if (d.depth && ((won && d.depth_test && d.depth_write) || cd))
+            store_depth(d, pix, won && d.depth_test && d.depth_write ? z : (ORDERED ? dep[q] : d.clear_depth));
     }
     for (int off = 32; off > 0; off >>= 1) frags += (uint32_t)__shfl_xor((int)frags, off);
     if (lane == 0u && frags) atomicAdd(&d.s.frags[blockIdx.x % kFragSlots], (unsigned long long)frags);

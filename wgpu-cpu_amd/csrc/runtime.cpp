@@ -2418,27 +2418,48 @@ static bool tiled_lines(const DrawParams &d)
     return d.topology != TOPO_POINT_LIST || d.resolve == RES_ORDERED;
 }
 
-// Key slots per tile of a tiled point / line draw: 256, or sixteen times
-// the draw's primitives per tile when that is more (a tile whose list is
-// longer tests every primitive's bounds instead), at most as many as there
-// are primitives and, together, 64 MiB (the allocation-free form's 128 MiB
-// hold them beside the records of 2^19 lines, the most of a draw).
-static uint64_t line_bin_cap(const DrawParams &d)
+// How much scratch the tiled point / line draws of a plan take: all of it; no
+// winners in global memory (a tile whose list is longer than its bin tests
+// every primitive's bounds instead); or the records alone (every tile does).
+enum LineScratch : uint32_t { LINES_ALL, LINES_NO_WINNERS, LINES_RECORDS };
+
+// Whether the lines that a tile's bin has no slot for go to winners in
+// global memory, 8 bytes per pixel: order-independent ones can.
+static bool line_winners(const DrawParams &d, LineScratch how)
 {
+    return how == LINES_ALL && d.topology != TOPO_POINT_LIST && d.resolve != RES_ORDERED && d.total_prims > kLineBin;
+}
+
+// Key slots per tile of a tiled point / line draw: kLineBin beside winners in
+// global memory (64: clusters 8 to 11 us less, but 2000 lines of 200 px over
+// 256x256, 100 a tile, 98 us a pass instead of 84), and none where lines are
+// dense, which then all go there: 5000 of 80 px over 256x256 (20 a tile) 46 us,
+// 77 with bins; 100000 of 15 px over 1080p (12 a tile) 64 us with bins, 125
+// without; 2000 of 30 px over 256x256 (8 a tile) 29 and 40.  Small targets
+// have few tile waves to hide a long list behind, so their line is lower.
+// Else 256, or sixteen times the draw's primitives per tile
+// when that is more, at most as many as there are primitives and, together,
+// 64 MiB (the allocation-free form's 128 MiB hold them beside the records of
+// 2^19 lines, the most of a draw).
+static uint64_t line_bin_cap(const DrawParams &d, LineScratch how)
+{
+    if (how == LINES_RECORDS) return 0;
     uint64_t tiles = std::max<uint64_t>((uint64_t)d.tiles_x * d.tiles_y, 1);
+    if (line_winners(d, how)) return d.total_prims >= (tiles <= 1024 ? 16 : 32) * tiles ? 0 : kLineBin;
     uint64_t cap = std::max<uint64_t>(256, (16ull * d.total_prims + tiles - 1) / tiles);
     return std::min<uint64_t>(std::min<uint64_t>(cap, d.total_prims), (64ull << 20) / (4 * tiles));
 }
 
 // Scratch of a point / line draw: the per-pixel visibility values, or the
-// set-up primitives and the tiles' bins.  `zone`: the tile counts (all
-// point / line steps of a plan share them: each tile kernel leaves them zero).
-static size_t layout_lines(Step &st, uint8_t *base, uint8_t *zone, uint32_t *frag_px, size_t frag_px_size,
-                           const Lane &lane)
+// set-up primitives and the tiles' bins.  `zone`: the tile counts, `keep`: the
+// winners in global memory (all point / line steps of a plan share them: each
+// tile kernel leaves them zero).
+static size_t layout_lines(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep, LineScratch how, uint32_t *frag_px,
+                           size_t frag_px_size, const Lane &lane)
 {
     DrawParams &d = st.draws[0];
     bool tiled = tiled_lines(d);
-    uint64_t cap = line_bin_cap(d), tiles = (uint64_t)d.tiles_x * d.tiles_y;
+    uint64_t cap = line_bin_cap(d, how), tiles = (uint64_t)d.tiles_x * d.tiles_y;
     size_t rec = align_up((uint64_t)(d.topology == TOPO_POINT_LIST ? kPointRecBytes : kLineRecBytes) * d.total_prims, 256);
     size_t bytes = tiled ? align_up(std::max<uint64_t>(rec + 4 * cap * tiles, 256), 256)
                          : align_up(8ull * d.width * d.height, 256);
@@ -2447,7 +2468,8 @@ static size_t layout_lines(Step &st, uint8_t *base, uint8_t *zone, uint32_t *fra
     st.gl.lp = tiled ? (void *)base : nullptr;
     d.s.bins = tiled ? (uint32_t *)(base + rec) : nullptr;
     d.s.bin_cap = (uint32_t)cap;
-    d.s.tile_count = (uint32_t *)zone;
+    d.s.tile_count = how == LINES_RECORDS ? nullptr : (uint32_t *)zone;
+    d.s.gvis = line_winners(d, how) ? (unsigned long long *)keep : nullptr;
     d.s.frags = lane.d_frags;
     d.s.error = lane.d_error;
     d.s.frag_px = (frag_px && frag_px_size == (size_t)d.width * d.height * 4u) ? frag_px : nullptr;
@@ -2855,9 +2877,24 @@ static void copy_step(const PassCommand &pc, Step &s)
 static constexpr size_t kLane1Arena = 2ull << 30;
 static constexpr int32_t kNoLane1 = 1;
 
-// `merge_max`: the size of a merged group at most; `merged`: whether there is one.
+// What a plan may take of scratch, and what of it a smaller choice would save.
+struct ScratchUse {
+    uint64_t merge_max = kMergedPrims;   // the size of a merged group at most
+    LineScratch lines = LINES_ALL;
+    bool merged = false, lines_more = false;
+    // the next smaller choice; false: there is none
+    bool less()
+    {
+        if (merged) merge_max = merge_max >= 4096 ? merge_max / 16 : 0;
+        else if (lines_more) lines = lines == LINES_ALL ? LINES_NO_WINNERS : LINES_RECORDS;
+        else return false;
+        merged = lines_more = false;
+        return true;
+    }
+};
+
 static int32_t lay_out_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, Plan &plan, bool noalloc,
-                            uint64_t merge_max, bool &merged)
+                            ScratchUse &use)
 {
     plan.reset();
     plan.noalloc = noalloc;
@@ -2913,12 +2950,12 @@ static int32_t lay_out_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb
                     uint64_t size = merged_size(dw.d);
                     while (dev->batching && !noalloc && !restart_strip(dw.d) && k + 1 < pw.draws.size() &&
                            same_group(dw.d, pw.draws[k + 1].d) &&
-                           size + merged_size(pw.draws[k + 1].d) <= merge_max) {
+                           size + merged_size(pw.draws[k + 1].d) <= use.merge_max) {
                         run.push_back(pw.draws[++k].d);
                         size += merged_size(run.back());
                     }
                     bool several = run.size() > 1;
-                    merged = merged || several;
+                    use.merged = use.merged || several;
                     add_group(plan.steps, std::move(run), cfg, stage++, several);
                     continue;
                 }
@@ -2985,7 +3022,7 @@ static int32_t lay_out_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb
     }
     // 3. scratch: the groups of a stage side by side, stages reusing the
     //    arena (they run one after another)
-    size_t need = 0, zneed = 0, kneed = 0, line_zone = 0;
+    size_t need = 0, zneed = 0, kneed = 0, line_zone = 0, line_keep = 0;
     size_t tables = 0;
     size_t stage_off = 0;
     uint32_t cur_stage = UINT32_MAX;
@@ -2998,12 +3035,17 @@ static int32_t lay_out_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb
         s.arena_off = stage_off;
         s.zone_off = zneed;
         s.keep_off = kneed;
-        size_t bytes = s.kind == StepKind::Lines ? layout_lines(s, nullptr, nullptr, nullptr, 0, lane)
+        size_t bytes = s.kind == StepKind::Lines ? layout_lines(s, nullptr, nullptr, nullptr, use.lines, nullptr, 0, lane)
                                                   : layout_group(s, nullptr, nullptr, nullptr, nullptr, 0, dev, lane);
         stage_off = align_up(stage_off + bytes, 256);
         need = std::max(need, stage_off);
-        if (s.kind == StepKind::Lines && tiled_lines(s.draws[0]))
-            line_zone = std::max<size_t>(line_zone, align_up(4ull * group_tiles(s), 256));
+        if (s.kind == StepKind::Lines && tiled_lines(s.draws[0])) {
+            uint64_t tiles = group_tiles(s);
+            use.lines_more = use.lines != LINES_RECORDS;
+            if (use.lines != LINES_RECORDS) line_zone = std::max<size_t>(line_zone, align_up(4ull * tiles, 256));
+            if (line_winners(s.draws[0], use.lines))
+                line_keep = std::max<size_t>(line_keep, align_up(8ull * kLpTile * kLpTile * tiles, 256));
+        }
         if (s.kind == StepKind::Group) {
             // active-list entries hold the global tile in kItemShift bits
             if (group_tiles(s) >= (1ull << kItemShift))
@@ -3020,8 +3062,9 @@ static int32_t lay_out_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb
             tables = align_up(tables + n * sizeof(DrawParams) + 8 * (n + 1) + 4 * (waves + tiles), 256);
         }
     }
-    size_t line_zone_off = zneed;
+    size_t line_zone_off = zneed, line_keep_off = kneed;
     zneed += line_zone;
+    kneed += line_keep;
     uint8_t *zone_base, *keep_base, *arena_base;
     if (noalloc) {
         // the static scratch: zero region, kept-zero region, then the stages
@@ -3070,7 +3113,7 @@ static int32_t lay_out_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb
         }
         if (e != hipSuccess) {
             int32_t r = hip_fail(e, "draw tables");
-            return merged ? WGC_ERR_OUT_OF_MEMORY : r;   // (draws one after another need none)
+            return use.merged ? WGC_ERR_OUT_OF_MEMORY : r;   // (draws one after another need none)
         }
         plan.tables_size = tables;
         plan.dev = dev;
@@ -3078,7 +3121,8 @@ static int32_t lay_out_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb
     }
     for (Step &s : plan.steps) {
         if (s.kind == StepKind::Lines) {
-            layout_lines(s, arena_base + s.arena_off, zone_base + line_zone_off, dev->frag_px, dev->frag_px_size, lane);
+            layout_lines(s, arena_base + s.arena_off, zone_base + line_zone_off, keep_base + line_keep_off, use.lines,
+                         dev->frag_px, dev->frag_px_size, lane);
             plan.launches += s.draws[0].total_prims == 0 ? 0 : (tiled_lines(s.draws[0]) ? 2 : 3);
             plan.prims += s.draws[0].total_prims;
             continue;
@@ -3134,12 +3178,13 @@ static int32_t lay_out_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb
 // Merged groups hold the scratch of all their draws at once, where draws
 // launched one after another share that of the largest: a pass for which
 // there is no memory is merged in smaller groups, and not at all in the end.
+// Point / line draws then do without what only makes them faster.
 static int32_t build_plan(WgcDevice_T *dev, Lane &lane, WgcCommandBuffer_T *cb, Plan &plan, bool noalloc)
 {
-    for (uint64_t merge_max = kMergedPrims;; merge_max = merge_max >= 4096 ? merge_max / 16 : 0) {
-        bool merged = false;
-        int32_t r = lay_out_plan(dev, lane, cb, plan, noalloc, merge_max, merged);
-        if (r != WGC_ERR_OUT_OF_MEMORY || !merged) return r;
+    ScratchUse use;
+    for (;;) {
+        int32_t r = lay_out_plan(dev, lane, cb, plan, noalloc, use);
+        if (r != WGC_ERR_OUT_OF_MEMORY || !use.less()) return r;
     }
 }
 

@@ -53,6 +53,8 @@ constexpr uint32_t kLineSteps = 8192;   // Bresenham steps per line (the fragmen
 constexpr uint32_t kPointRecBytes = 64;  // scratch per primitive of a tiled point / line draw (LpRec)
 constexpr uint32_t kLineRecBytes = 96;
 constexpr uint32_t kLpTile = 16;         // screen tiles of the tiled point / line path
+constexpr uint32_t kLineBin = 128;       // bin slots per tile of order-independent lines; the others go to global memory
+constexpr uint32_t kLineCrowd = 1024;    // past as many lines of a tile, its winners are read before they are contested
 constexpr uint32_t kLpSort = 1024;       // keys an ordered point / line tile sorts (a tile with more tests every primitive)
 enum Compare : uint32_t {
     CMP_NEVER = 1, CMP_LESS = 2, CMP_EQUAL = 3, CMP_LESS_EQUAL = 4,
@@ -126,7 +128,8 @@ struct Scratch {
     unsigned long long *frags;  // kFragSlots fragment counters of the submission (summed on read)
     uint32_t *error;
     uint32_t *frag_px;       // optional per-pixel fragment count
-    unsigned long long *gvis;   // split tiles: the merged winners, TS*TS per tile (kept zero between uses)
+    unsigned long long *gvis;   // the winners of split tiles, and of the lines past a full bin: TS*TS per tile (kept
+                             // zero between uses)
     uint32_t *tile_done;     // split tiles: their items that have finished (zero region)
     uint32_t tile0;          // global index of the draw's first tile
     uint32_t key_base;       // draws of one pass in one group: the first of this draw's primitives among
