@@ -156,3 +156,29 @@ def test_batching_off_is_one_launch_set_per_draw(gpu_device):
         assert launches(spec) == sum(alone) > merged
     finally:
         gpu_device.set_option(wgc.OPTION_BATCHING, 1)
+
+
+# Groups too large for setup to clip in place (a launch for the clipper, no
+# clear ahead of the tiles), with tiles of several batches that stay whole,
+# and one of more primitives than a group takes.
+@pytest.mark.parametrize("mode,count,n,launches", [("less", 5, 60000, 3), ("no_depth", 5, 60000, 3),
+                                                   ("blend", 5, 60000, 3), ("less", 9, 125000, 5)],
+                         ids=["less", "no_depth", "blend", "two_groups"])
+def test_large_groups(gpu_device_ext, mode, count, n, launches):
+    w, h = 1600, 900
+    depth, blend = (wgc.LESS, True) if mode == "less" else None, wgc.BLEND_ALPHA if mode == "blend" else wgc.BLEND_REPLACE
+    draws = []
+    for k in range(count):
+        vb = random_clip_triangles(n, 7600 + k, w, h, spread=1.03, size_px=(1.0, 14.0 if count < 9 else 5.0),
+                                   w_range=(0.5, 2.0), z_levels=[0.3, 0.5, 0.7], alpha=(0.2, 0.8))
+        vb[::9, :, 2] = -0.2 * vb[::9, :, 3]
+        vb[4::13, 0, 2] = 1.3 * vb[4::13, 0, 3]
+        draws.append(clip_color_draw(vb, depth=depth, blend=blend))
+    draws[1].cull_mode = wgc.CULL_BACK
+    draws[2].viewport = (-20.0, 9.0, 1700.0, 870.0, 0.0, 1.0)
+    spec = scenes.PassSpec(w, h, clear_color=(0.1, 0.2, 0.3, 1.0), has_depth=depth is not None, clear_depth=1.0,
+                           draws=draws, semantics=wgc.SEMANTICS_EXTENDED, name=f"large groups {mode} {count} x {n}")
+    assert_parity(spec, gpu_device_ext)
+    assert gpu_device_ext.last_pass_stats().kernel_launches == launches
+    if count < 9:
+        assert_parity(scenes.as_wgsl(spec), gpu_device_ext)

@@ -2519,11 +2519,21 @@ static size_t keep_bytes(const Step &st)
 // its kernel lasts as long as its slowest tile) while ordinary ones stay
 // whole.  Order-independent groups of one target only: ordered tiles are
 // never split, and a batched group has many tiles per workgroup anyway.
-static uint32_t split_for(const Step &st)
+// The draws of a pass together often fill every tile past that; where each
+// workgroup has several tiles, splitting all of them only adds the merging, so
+// an item then holds eight times the primitives per tile (a triangle of some
+// ten pixels has about four).  1920x1080, us a pass with every tile split at a
+// batch -> so (one draw after another): 2 draws of 130000 triangles of 15 px
+// 429 -> 185 (253), 4 of 80000 492 -> 235 (398), 3 of 250000 of 4 px 517 -> 199
+// (302).
+static uint32_t split_for(const Step &st, uint64_t prims, uint64_t tiles)
 {
     if (st.gl.ordered || st.multi) return 0;
     uint32_t cfg = st.gl.user ? (uint32_t)RASTER_16x16_256 : st.gl.raster_cfg;
-    return vis_batch_size(1u << raster_tile_shift(cfg), raster_threads(cfg));
+    uint32_t batch = vis_batch_size(1u << raster_tile_shift(cfg), raster_threads(cfg));
+    if (!st.merged || tiles < 2ull * st.gl.raster_grid) return batch;
+    uint64_t batches = std::min<uint64_t>(8 * prims / tiles / batch, 512);   // (16 items stay below 2^24 entries)
+    return batch * (uint32_t)std::max<uint64_t>(batches, 1);
 }
 
 static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep, uint32_t *frag_px,
@@ -2597,7 +2607,6 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
     gl.counters = (uint32_t *)(zone + align_up(4ull * H_NUM, 256));
     gl.tile_count = (uint32_t *)(zone + align_up(4ull * H_NUM, 256) + align_up(4ull * C_NUM * n, 256));
     uint32_t *tile_done = gl.tile_count + align_up(4ull * total_tiles, 256) / 4;
-    uint32_t split = split_for(st);
     gl.clip_list = (uint2 *)(base + o_cl);
     gl.clip_cap = (uint32_t)prims;
     // a group of one target whose setup workgroups are all resident at once
@@ -2650,6 +2659,7 @@ static size_t layout_group(Step &st, uint8_t *base, uint8_t *zone, uint8_t *keep
         occ = raster_blocks_per_cu(gl.program, gl.ordered != 0, st.multi, gl.raster_cfg);
     }
     gl.raster_grid = resident_grid(dev, occ, total_tiles);
+    uint32_t split = split_for(st, all_prims, total_tiles);
     uint64_t tile_base = 0, bin_base = 0, prim_base = 0;
     for (size_t k = 0; k < st.draws.size(); ++k) {
         uint32_t i = st.merged ? 0u : (uint32_t)k;   // the draw's target
