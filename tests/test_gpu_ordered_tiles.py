@@ -11,6 +11,8 @@ import wgc
 from oracle import bridge
 from wgc import runner, scenes
 
+from test_gpu_parity import clip_color_draw
+
 pytestmark = pytest.mark.gpu
 
 
@@ -219,6 +221,55 @@ def test_ordered_tiles_by_single_waves(gpu_device, gpu_device_ext, mode):
         ref = bridge.render(s)
         dev.enable_fragment_counts(0, 0)
         got = runner.render(s, dev)
+        assert got.fragments == ref.fragments
+        assert np.array_equal(got.color, ref.color)
+        if depth is not None:
+            assert np.array_equal(got.depth.view(np.uint32), ref.depth.view(np.uint32))
+
+
+# Single waves are left out where half of the tiles lie under big triangles
+# (over 16 tiles) or are met by clipped ones.  The states around those lines:
+# big triangles over a third of the 4347 tiles ("some") and over all ("most"),
+# a band of clipped triangles along one edge and clipped ones everywhere.
+@pytest.mark.parametrize("mode", ["blend", "not_equal", "two_draws"])
+@pytest.mark.parametrize("big,clipped", [("none", "none"), ("some", "edge"), ("most", "none"), ("none", "all")])
+def test_ordered_tiles_single_waves_or_not(gpu_device_ext, mode, big, clipped):
+    w, h, n = 1103, 1005, 24000
+    count = n if mode != "two_draws" else n // 2
+    depth = (wgc.NOT_EQUAL, True) if mode == "not_equal" else None
+    draws = []
+    for seed in (8200, 8201)[:n // count]:
+        u = scenes.splitmix_f32(seed, count * 8).reshape(count, 8)
+        k = np.arange(count)
+        size = np.full(count, 12.0)
+        x, y = 15.0 + u[:, 0] * (w - 30), 15.0 + u[:, 1] * (h - 30)
+        if big != "none":
+            large = k % 300 == 0
+            size[large] = 70.0
+            if big == "some":
+                x[large], y[large] = 80.0 + 250.0 * u[large, 0], 80.0 + 800.0 * u[large, 1]
+        if clipped == "edge":
+            x[k % 40 == 1] = w
+        crowd = k % 90 == 7
+        x[crowd], y[crowd] = 700.0 + 25.0 * u[crowd, 0], 400.0 + 25.0 * u[crowd, 1]
+        size[crowd] = 4.0
+        vb = np.zeros((count, 3, 8), np.float32)
+        for c in range(3):
+            ang = 2.1 * c + 6.28 * u[:, 2]
+            vb[:, c, 0] = (x + size * np.cos(ang)) / w * 2 - 1
+            vb[:, c, 1] = 1 - (y + size * np.sin(ang)) / h * 2
+        vb[:, :, 2], vb[:, :, 3], vb[:, :, 4:8] = u[:, 3:4], 1.0, u[:, None, 4:8]
+        if clipped == "all":
+            vb[k % 3 == 0, 1, 2] = -0.2
+        draws.append(clip_color_draw(vb, depth=depth,
+                                     blend=wgc.BLEND_REPLACE if depth else wgc.BLEND_ALPHA))
+    spec = scenes.PassSpec(w, h, has_depth=depth is not None, clear_depth=0.6, draws=draws,
+                           semantics=wgc.SEMANTICS_EXTENDED, name=f"single waves or not {mode} {big} {clipped}")
+    gpu_device_ext.enable_fragment_counts(0, 0)   # (with per-pixel counts the workgroup's form runs)
+    for s in (spec, scenes.as_wgsl(spec)):
+        announce(s.name)
+        ref = bridge.render(s)
+        got = runner.render(s, gpu_device_ext)
         assert got.fragments == ref.fragments
         assert np.array_equal(got.color, ref.color)
         if depth is not None:

@@ -2524,7 +2524,7 @@ static size_t keep_bytes(const Step &st)
 // an item then holds eight times the primitives per tile (a triangle of some
 // ten pixels has about four).  1920x1080, us a pass with every tile split at a
 // batch -> so (one draw after another): 2 draws of 130000 triangles of 15 px
-// 429 -> 185 (253), 4 of 80000 492 -> 235 (398), 3 of 250000 of 4 px 517 -> 199
+// 429 -> 185 (253), 4 of 80000 492 -> 230 (398), 3 of 250000 of 4 px 517 -> 199
 // (302).
 static uint32_t split_for(const Step &st, uint64_t prims, uint64_t tiles)
 {
