@@ -103,11 +103,15 @@ def test_noalloc_draws_one_at_a_time_equals_the_group(gpu_device):
     spec = scenes.PassSpec(w, h, has_depth=True, clear_depth=1.0, draws=draws)
     pp = runner.PreparedPass(gpu_device, spec)
     pp.submit()
-    want = pp.results()[0]
+    want = pp.result()
+    rng = np.random.default_rng(7)
+    gpu_device.write_texture(pp.res[0].color, rng.integers(0, 256, w * h * 4, dtype=np.uint8).tobytes())
+    gpu_device.write_texture(pp.res[0].depth, rng.random(w * h, dtype=np.float32).tobytes())
     gpu_device.submit_noalloc([pp.command_buffer])
-    got = pp.results()[0]
+    got = pp.result()
     ref = bridge.render(spec)
     for r in (want, got):
+        assert r.fragments == ref.fragments
         assert np.array_equal(r.color, ref.color)
         assert np.array_equal(r.depth.view(np.uint32), ref.depth.view(np.uint32))
 

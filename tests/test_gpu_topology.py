@@ -306,9 +306,13 @@ def test_most_lines_without_allocation(gpu_device_ext):
     gpu_device_ext.enable_fragment_counts(0, 0)
     pp = runner.PreparedPass(gpu_device_ext, spec)
     pp.submit()
-    want = pp.results()[0].color
+    want = pp.result()
+    noise = np.random.default_rng(6).integers(0, 256, side * side * 4, dtype=np.uint8)
+    gpu_device_ext.write_texture(pp.res[0].color, noise.tobytes())
     gpu_device_ext.submit_noalloc([pp.command_buffer])
-    np.testing.assert_array_equal(pp.results()[0].color, want)
+    got = pp.result()
+    np.testing.assert_array_equal(got.color, want.color)
+    assert got.fragments == want.fragments > n
 
 
 @pytest.mark.parametrize("mode", ["less", "blend"])
