@@ -245,9 +245,10 @@ def test_tiled_lines_crowded_corner(gpu_device_ext, mode):
 
 
 def test_ordered_points_crowded_tile(gpu_device_ext):
-    """More points in a tile than one sort takes, within its bin and past it."""
+    """More points in a tile than one sort takes, in two, three and six runs of
+    its bin, and past it (5625 slots here)."""
     w, h, n = 256, 256, 90000
-    for k in (1500, 7000):
+    for k in (1500, 2500, 5000, 7000):
         u = scenes.splitmix_f32(6700 + k, n * 6).reshape(n, 6)
         vb = np.zeros((n, 8), np.float32)
         x, y = u[:, 0] * w, u[:, 1] * h

@@ -55,7 +55,7 @@ constexpr uint32_t kLineRecBytes = 96;
 constexpr uint32_t kLpTile = 16;         // screen tiles of the tiled point / line path
 constexpr uint32_t kLineBin = 128;       // bin slots per tile of order-independent lines; the others go to global memory
 constexpr uint32_t kLineCrowd = 1024;    // past as many lines of a tile, its winners are read before they are contested
-constexpr uint32_t kLpSort = 1024;       // keys an ordered point / line tile sorts (a tile with more tests every primitive)
+constexpr uint32_t kLpSort = 1024;       // keys that an ordered point / line tile sorts at once
 enum Compare : uint32_t {
     CMP_NEVER = 1, CMP_LESS = 2, CMP_EQUAL = 3, CMP_LESS_EQUAL = 4,
     CMP_GREATER = 5, CMP_NOT_EQUAL = 6, CMP_GREATER_EQUAL = 7, CMP_ALWAYS = 8,
