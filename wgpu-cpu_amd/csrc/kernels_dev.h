@@ -2526,6 +2526,7 @@ struct LineWalk {
     int32_t m0, c0, sm, sc;   // first pixel and direction along the major and the minor axis
     uint32_t n, q;
     bool xmajor;
+    bool wide;   // one of the wave's lines is longer than kLineSteps (uniform)
     __device__ __forceinline__ LineWalk(const uint32_t a[2], const uint32_t b[2])
     {
         int32_t dx = (int32_t)b[0] - (int32_t)a[0], dy = (int32_t)b[1] - (int32_t)a[1];
@@ -2538,15 +2539,15 @@ struct LineWalk {
         int32_t dm = xmajor ? dx : dy, dc = xmajor ? dy : dx;
         sm = dm < 0 ? -1 : 1;
         sc = dc < 0 ? -1 : 1;
+        wide = __ballot(n > kLineSteps) != 0u;
     }
     __device__ __forceinline__ uint32_t steps() const { return min(n, kLineSteps); }   // none: nothing is drawn
     // (a * b + c) / d.  In the longer line's 60 bits the quotient, below 2^30,
     // is estimated in binary64 (within one of it) and corrected by its
-    // remainder: a tenth of the general 64-bit division's code, which cost
-    // every line draw a microsecond.
+    // remainder, in a tenth of the general 64-bit division's code.
     __device__ __forceinline__ uint32_t ratio(uint32_t a, uint32_t b, uint32_t c, uint32_t d) const
     {
-        if (n <= kLineSteps) return (a * b + c) / d;
+        if (!wide) return (a * b + c) / d;
         uint64_t x = (uint64_t)a * b + c;
         uint32_t e = (uint32_t)((double)x / (double)d);
         int64_t r = (int64_t)(x - (uint64_t)e * d);
