@@ -220,9 +220,10 @@ def crowded_lines(n, w, h, mode, corner=(16, 16)):
 
 
 # The tiled line path.  Order-independent: lists within a tile's bin (64
-# slots) and past it, where the other lines go to winners in global memory.
-# In API order (256 slots on these 1024 tiles, 512 for n=8200): lists of up to one wave's keys,
-# of one sort in LDS, and past the bin, so that the tile tests every primitive.
+# slots, 256 from n = 256 on) and past it, where the other lines go to winners
+# in global memory, which past 1024 lines of a tile are read first.  In API
+# order (256 slots): lists of up to one wave's keys, sorted in LDS, and past the
+# bin, so that the tile tests every primitive.
 @pytest.mark.parametrize("n", [40, 64, 75, 240, 1300, 8200])
 @pytest.mark.parametrize("mode", ["less", "greater_equal", "less_no_write", "last", "blend"])
 def test_tiled_lines_crowded_tile(gpu_device_ext, n, mode):

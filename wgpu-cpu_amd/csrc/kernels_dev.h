@@ -2749,22 +2749,6 @@ constexpr uint32_t kNoPoint = 0xFFFFFFFFu;
 // length is made of, so they are spread over lanes rather than walked.
 constexpr uint32_t kLpLanes = 8;
 
-// The primitive's place among the tile's, in its bin if there is room (0
-// where the draw has no bins).  The lanes on the first one's tile take theirs
-// together, since lines that crowd one tile meet on its counter (20000 lines
-// in 14x14 px: prep 261 us with an atomic each, 125 so).
-__device__ __forceinline__ uint32_t lp_bin(const DrawParams &d, uint32_t tile, uint32_t p)
-{
-    if (!d.s.bin_cap) return 0u;
-    bool mine = tile == (uint32_t)__builtin_amdgcn_readfirstlane(tile);
-    uint64_t same = __ballot(mine);
-    uint32_t rank = (uint32_t)__popcll(same & lanes_below()), slot = 0u;
-    if (!mine || rank == 0u) slot = atomicAdd(&d.s.tile_count[tile], mine ? (uint32_t)__popcll(same) : 1u);
-    if (mine) slot = (uint32_t)__builtin_amdgcn_readfirstlane(slot) + rank;
-    if (slot < d.s.bin_cap) d.s.bins[(size_t)tile * d.s.bin_cap + slot] = p;
-    return slot;
-}
-
 // The coefficient of a line's second end point at t (raster.rs:251-254: the
 // lerp of the clip alphas), and one component of the fragment, the
 // coefficient applied to the clipped end points.
@@ -2885,7 +2869,10 @@ __device__ __forceinline__ uint32_t lp_prep(const DrawParams &d, LpRec<N> *recs,
     int32_t sy0 = (int32_t)(d.scissor[1] / kLpTile), sy1 = (int32_t)((d.scissor[1] + d.scissor[3] - 1u) / kLpTile);
     if constexpr (N == 1) {
         int32_t tx = (int32_t)(r.fb[0][0] / kLpTile), ty = (int32_t)(r.fb[0][1] / kLpTile);
-        if (tx >= sx0 && tx <= sx1 && ty >= sy0 && ty <= sy1) (void)lp_bin(d, (uint32_t)ty * d.tiles_x + (uint32_t)tx, p);
+        if (tx >= sx0 && tx <= sx1 && ty >= sy0 && ty <= sy1) {
+            uint32_t tile = (uint32_t)ty * d.tiles_x + (uint32_t)tx, slot = atomicAdd(&d.s.tile_count[tile], 1u);
+            if (slot < d.s.bin_cap) d.s.bins[(size_t)tile * d.s.bin_cap + slot] = p;
+        }
         return 0u;
     } else {
         LineWalk w(r.fb[0], r.fb[N - 1]);
@@ -2895,7 +2882,7 @@ __device__ __forceinline__ uint32_t lp_prep(const DrawParams &d, LpRec<N> *recs,
         int32_t clo = w.xmajor ? sy0 : sx0, chi = w.xmajor ? sy1 : sx1;        // scissor, minor
         int32_t t0 = max(min(ma, mb) / (int32_t)kLpTile, lo), t1 = min(max(ma, mb) / (int32_t)kLpTile, hi);
         float time = 0.0f;
-        uint32_t at = 0u, frags = 0u;
+        uint32_t at = 0u, frags = 0u, cap = d.s.bin_cap;
         for (int32_t i = (int32_t)sub; i <= t1 - t0; i += (int32_t)kLpLanes) {
             // the steps in this column of tiles: fewer than kLpTile pixels
             // along the minor axis, so at most two tiles
@@ -2903,14 +2890,42 @@ __device__ __forceinline__ uint32_t lp_prep(const DrawParams &d, LpRec<N> *recs,
             int32_t k0, k1;
             w.major_steps(t * (int32_t)kLpTile, t * (int32_t)kLpTile + (int32_t)kLpTile - 1, k0, k1);
             int32_t ca = w.minor((uint32_t)k0) / (int32_t)kLpTile, cb = w.minor((uint32_t)k1) / (int32_t)kLpTile;
-#pragma unroll 1
-            for (int32_t c = ca;; c = cb) {
-                if (c >= clo && c <= chi) {
-                    int32_t tx = w.xmajor ? t : c, ty = w.xmajor ? c : t;
-                    uint32_t slot = lp_bin(d, (uint32_t)ty * d.tiles_x + (uint32_t)tx, p);
-                    if (slot >= d.s.bin_cap && d.s.gvis) frags += lp_overflow(d, r, w, p, tx, ty, slot, time, at);
+            uint32_t ta = (uint32_t)(w.xmajor ? ca * (int32_t)d.tiles_x + t : t * (int32_t)d.tiles_x + ca);
+            uint32_t tb = (uint32_t)(w.xmajor ? cb * (int32_t)d.tiles_x + t : t * (int32_t)d.tiles_x + cb);
+            bool a = ca >= clo && ca <= chi, b = cb != ca && cb >= clo && cb <= chi;
+            uint32_t slot_a, slot_b;   // (set where `a`, `b`; a value to merge with would be waited for)
+            if (cap) {
+                // both counters asked before either answer is used.  The lanes
+                // on the first one's tile take their slots together: lines
+                // that crowd one tile meet on its counter (20000 in 14x14 px:
+                // prep 261 us with an atomic each, 125 so)
+                bool same = false;
+                uint32_t rank = 0u;
+                if (a) {
+                    same = ta == (uint32_t)__builtin_amdgcn_readfirstlane(ta);
+                    uint64_t all = __ballot(same);
+                    rank = (uint32_t)__popcll(all & lanes_below());
+                    if (!same || rank == 0u) slot_a = atomicAdd(&d.s.tile_count[ta], same ? (uint32_t)__popcll(all) : 1u);
                 }
-                if (c == cb) break;
+                if (b) slot_b = atomicAdd(&d.s.tile_count[tb], 1u);
+                if (a) {
+                    if (same) slot_a = (uint32_t)__builtin_amdgcn_readfirstlane(slot_a) + rank;
+                    if (slot_a < cap) d.s.bins[(size_t)ta * cap + slot_a] = p;
+                }
+                if (b && slot_b < cap) d.s.bins[(size_t)tb * cap + slot_b] = p;
+            }
+            if (!d.s.gvis) continue;
+            if (cap) {
+                a = a && slot_a >= cap;
+                b = b && slot_b >= cap;
+            } else {
+                slot_a = slot_b = 0u;   // (no counts)
+            }
+            if (!(a || b)) continue;
+#pragma unroll 1
+            for (uint32_t k = a ? 0u : 1u; k < (b ? 2u : 1u); ++k) {   // (the steps' order)
+                int32_t c = k ? cb : ca;
+                frags += lp_overflow(d, r, w, p, w.xmajor ? t : c, w.xmajor ? c : t, k ? slot_b : slot_a, time, at);
             }
         }
         return frags;
@@ -3045,10 +3060,10 @@ __device__ __forceinline__ bool lp_sorted(uint32_t n, uint32_t prims)
 // walking over a visibility buffer of the target, and its fill and the
 // clear: 324 us).  With a wave for any list, lines that crowded few tiles took
 // longer than over the visibility buffer: 20000 in 14x14 px of 1080p 84 us
-// there, 3980 by one wave, 100 with winners in global memory; 20000 of 20 px
-// over 256x256 66, 107 and 47 us.  Batches of 24 or 32 lines (12 KB of LDS per wave instead
-// of 9) give 57 and 54 us a pass against 52 on the second, 41 and 40 against
-// 41 on the first.
+// there, 3440 by one wave, 125 with winners in global memory; 20000 of 20 px
+// over 256x256 66, 107 and 47 us.  Batches of 24 or 32 lines (12 KB of LDS per
+// wave instead of 9) give 57 and 54 us a pass against 52 on the second, 41 and
+// 40 against 41 on the first.
 template <int PROG, int N, bool ORDERED>
 __global__ __launch_bounds__(64) void k_lp_tiles(DrawParams d, const LpRec<N> *recs)
 {

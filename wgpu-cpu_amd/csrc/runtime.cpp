@@ -2430,22 +2430,29 @@ static bool line_winners(const DrawParams &d, LineScratch how)
     return how == LINES_ALL && d.topology != TOPO_POINT_LIST && d.resolve != RES_ORDERED && d.total_prims > kLineBin;
 }
 
-// Key slots per tile of a tiled point / line draw: kLineBin beside winners in
-// global memory (64: clusters 8 to 11 us less, but 2000 lines of 200 px over
-// 256x256, 100 a tile, 98 us a pass instead of 84), and none where lines are
-// dense, which then all go there: 5000 of 80 px over 256x256 (20 a tile) 46 us,
-// 77 with bins; 100000 of 15 px over 1080p (12 a tile) 64 us with bins, 125
-// without; 2000 of 30 px over 256x256 (8 a tile) 29 and 40.  Small targets
-// have few tile waves to hide a long list behind, so their line is lower.
-// Else 256, or sixteen times the draw's primitives per tile
-// when that is more, at most as many as there are primitives and, together,
-// 64 MiB (the allocation-free form's 128 MiB hold them beside the records of
-// 2^19 lines, the most of a draw).
+// Key slots per tile of a tiled point / line draw.  Beside winners in global
+// memory:
+//  - none where lines are dense: all go there.  5000 of 80 px over 256x256 (20
+//    a tile) 46 us a pass, 77 with bins; 100000 of 15 px over 1920x1080 (12 a
+//    tile) 64 us with bins, 125 without; 2000 of 30 px over 256x256 (8 a tile)
+//    29 and 40.  Small targets have few tile waves to hide a long list behind,
+//    so their line is lower;
+//  - kLineBinMany where long lines could fill every tile: a strip of 30000 over
+//    1920x1080, half of them across it, 206 us, 382 with 128 slots;
+//  - kLineBin where only a cluster can: 300 to 2000 lines in 14x14 px of
+//    1920x1080 41 to 51 us, 52 to 62 with 128 slots.
+// Else 256, or sixteen times the draw's primitives per tile when that is more,
+// at most as many as there are primitives and, together, 64 MiB (the
+// allocation-free form's 128 MiB hold them beside the records of 2^19 lines,
+// the most of a draw).
 static uint64_t line_bin_cap(const DrawParams &d, LineScratch how)
 {
     if (how == LINES_RECORDS) return 0;
     uint64_t tiles = std::max<uint64_t>((uint64_t)d.tiles_x * d.tiles_y, 1);
-    if (line_winners(d, how)) return d.total_prims >= (tiles <= 1024 ? 16 : 32) * tiles ? 0 : kLineBin;
+    if (line_winners(d, how)) {
+        if (d.total_prims >= (tiles <= 1024 ? 16 : 32) * tiles) return 0;
+        return 4ull * d.total_prims >= tiles ? kLineBinMany : kLineBin;
+    }
     uint64_t cap = std::max<uint64_t>(256, (16ull * d.total_prims + tiles - 1) / tiles);
     return std::min<uint64_t>(std::min<uint64_t>(cap, d.total_prims), (64ull << 20) / (4 * tiles));
 }

@@ -53,7 +53,8 @@ constexpr uint32_t kLineSteps = 8192;   // Bresenham steps per line (the fragmen
 constexpr uint32_t kPointRecBytes = 64;  // scratch per primitive of a tiled point / line draw (LpRec)
 constexpr uint32_t kLineRecBytes = 96;
 constexpr uint32_t kLpTile = 16;         // screen tiles of the tiled point / line path
-constexpr uint32_t kLineBin = 128;       // bin slots per tile of order-independent lines; the others go to global memory
+constexpr uint32_t kLineBin = 64;        // bin slots per tile of few order-independent lines, and
+constexpr uint32_t kLineBinMany = 256;   // of many; the others go to global memory
 constexpr uint32_t kLineCrowd = 1024;    // past as many lines of a tile, its winners are read before they are contested
 constexpr uint32_t kLpSort = 1024;       // keys that an ordered point / line tile sorts at once
 enum Compare : uint32_t {
