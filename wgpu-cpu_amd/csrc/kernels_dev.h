@@ -80,8 +80,8 @@ __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v)
 // scalar loads (the index is uniform) that no store of the kernel orders or
 // repeats.  As plain global memory they were vector loads after the tile's
 // first store, again in every inner loop: 7.2M vector memory instructions in
-// a batched tile kernel of 256 passes, 2.2M with this; the submission 804 ->
-// 684 us, 24 draws of a pass over 1366x768 76 -> 64.
+// a batched tile kernel of 256 passes, 2.2M with this; the submission 824 ->
+// 666 us, 24 draws of a pass over 1366x768 73 -> 60.
 __device__ __forceinline__ const DrawParams &table_draw(const BatchArgs &b, uint32_t i)
 {
     typedef const DrawParams __attribute__((address_space(4))) ConstDraw;
@@ -2098,7 +2098,6 @@ __device__ __forceinline__ void raster_tile_oi(const DrawParams &d, const BatchA
     __syncthreads();  // the next tile resets the per-pixel state
 }
 
-// Stores the clear values into one tile.
 // One wave stores the LoadOp::Clear values into a tile: 16 bytes a lane where
 // the rows allow it (a 16x16 tile is one store per texture).
 template <int TS>

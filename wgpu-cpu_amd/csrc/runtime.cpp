@@ -3368,8 +3368,8 @@ static uint64_t conflict_with(const Lane &l, const PassCommand &pc)
 // GPU idle (a chain of latency-bound launches), so independent single passes
 // alternate between two streams: passes over three targets in turn, 1080p
 // mesh 35 -> 24 us a pass, 24 objects 60 -> 41, 200k blended triangles 312 ->
-// 236 (a third stream: 28, 45 and 256 where two gave 23, 35 and 227).  A pass
-// goes behind the submission that it has to follow (no wait between streams,
+// 236 (a probe with a device object per stream gave 23, 35 and 227 with two
+// and 28, 45 and 256 with three).  A pass goes behind the submission that it has to follow (no wait between streams,
 // 5 to 10 us on an idle one) if that is the last of its lane, or this lane is
 // the shorter one, or next to nothing is queued (with a deep queue the event
 // has long passed when the wait is reached); one that has none to follow goes
