@@ -342,3 +342,25 @@ def test_line_of_too_many_steps(mode, scissor):
         pp.device.poll()
     color, _ = pp.res[0].read()
     np.testing.assert_array_equal(color, want)
+
+
+@pytest.mark.parametrize("mode", ["less", "blend"])
+def test_crowded_lines_replayed(mode):
+    """The crowded draw as a replayed graph, with other work between the
+    replays: counts and winners are zero again after each."""
+    announce(f"crowded lines replayed, {mode}")
+    dev = wgc.Device(0, wgc.SEMANTICS_EXTENDED)
+    dev.set_option(wgc.OPTION_GRAPHS, 1)
+    spec, other = crowded_lines(1300, 512, 512, mode), crowded_lines(240, 512, 512, "last")
+    want, want_other = bridge.render(spec), bridge.render(other)
+    p, q = runner.PreparedPass(dev, spec), runner.PreparedPass(dev, other)
+    rng = np.random.default_rng(8)
+    for _ in range(4):
+        dev.write_texture(p.res[0].color, rng.integers(0, 256, 512 * 512 * 4, dtype=np.uint8).tobytes())
+        p.submit()
+        q.submit()
+        got, got_other = p.results()[0], q.results()[0]
+        np.testing.assert_array_equal(got.color, want.color)
+        np.testing.assert_array_equal(got_other.color, want_other.color)
+        if want.depth is not None:
+            np.testing.assert_array_equal(got.depth.view(np.uint32), want.depth.view(np.uint32))
