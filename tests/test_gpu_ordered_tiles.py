@@ -228,11 +228,14 @@ def test_ordered_tiles_by_single_waves(gpu_device, gpu_device_ext, mode):
 
 
 # Single waves are left out where half of the tiles lie under big triangles
-# (over 16 tiles) or are met by clipped ones.  The states around those lines:
-# big triangles over a third of the 4347 tiles ("some") and over all ("most"),
-# a band of clipped triangles along one edge and clipped ones everywhere.
+# (over 16 tiles), as many sub-triangles are clipped, or a tile has more than
+# 1000 fragments on average.  The states around those lines: big triangles over
+# a third of the 4347 tiles ("some") and over all ("most"), a band of clipped
+# triangles along one edge and clipped ones everywhere, and triangles of about
+# 83 (the others) and 420 px ("heavy"), 460 and 2300 fragments a tile.
 @pytest.mark.parametrize("mode", ["blend", "not_equal", "two_draws"])
-@pytest.mark.parametrize("big,clipped", [("none", "none"), ("some", "edge"), ("most", "none"), ("none", "all")])
+@pytest.mark.parametrize("big,clipped", [("none", "none"), ("some", "edge"), ("most", "none"), ("none", "all"),
+                                         ("heavy", "none")])
 def test_ordered_tiles_single_waves_or_not(gpu_device_ext, mode, big, clipped):
     w, h, n = 1103, 1005, 24000
     count = n if mode != "two_draws" else n // 2
@@ -241,9 +244,9 @@ def test_ordered_tiles_single_waves_or_not(gpu_device_ext, mode, big, clipped):
     for seed in (8200, 8201)[:n // count]:
         u = scenes.splitmix_f32(seed, count * 8).reshape(count, 8)
         k = np.arange(count)
-        size = np.full(count, 12.0)
+        size = np.full(count, 18.0 if big == "heavy" else 8.0)
         x, y = 15.0 + u[:, 0] * (w - 30), 15.0 + u[:, 1] * (h - 30)
-        if big != "none":
+        if big in ("some", "most"):
             large = k % 300 == 0
             size[large] = 70.0
             if big == "some":

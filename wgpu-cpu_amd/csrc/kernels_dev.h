@@ -417,6 +417,7 @@ __global__ __launch_bounds__(256) void k_setup(DrawParams d0, BatchArgs b)
     }
     bool active = p < d.total_prims;
     bool has_rec = false, needs_clip = false;
+    uint32_t area = 0u;
     uint4 rec = make_uint4(0, 0, 0, 0);
     uint32_t ntiles = 0;
     if (active) {
@@ -445,6 +446,7 @@ __global__ __launch_bounds__(256) void k_setup(DrawParams d0, BatchArgs b)
                             uint32_t key = (d.s.key_base + p) << 7;
                             rec = make_uint4(key, tx0 | (ty0 << 16), tx1 | (ty1 << 16), di);
                             ntiles = (tx1 - tx0 + 1) * (ty1 - ty0 + 1);
+                            area = (uint32_t)fminf(fabsf(r.total), 8192.0f);
                             write_record(d.s.tri + (size_t)p * kRecWords, r, v, key, ff);
                         }
                     }
@@ -471,6 +473,13 @@ __global__ __launch_bounds__(256) void k_setup(DrawParams d0, BatchArgs b)
         else atomicOr(d.s.error, (uint32_t)ERR_RECORD_OVERFLOW);
     }
     note_big_wave(d, big && slot < d.s.big_cap, rec);
+    if (d.resolve == RES_ORDERED) {
+        // the binned triangles' area for k_raster, twice, in units of 32 (a
+        // wave's sum is below 2^19; after the binning, whose atomics' answers
+        // would wait for this one)
+        area = wave_inclusive_sum(small ? area : 0u);
+        if (lane_id() == 63u) atomicAdd(d.s.header + H_AREA + kQueueStride * (g / 64u % 8u), area >> 5);
+    }
     if constexpr (CLIP) {
         // every lane of the wave takes part (the clip slots are reserved per wave)
         if (__ballot(needs_clip))
@@ -1500,6 +1509,7 @@ __device__ __forceinline__ void raster_tile(const DrawParams &d, const BatchArgs
 // are not in the record), spilled and big triangles.
 constexpr uint32_t kLightTris = 24;
 constexpr uint32_t kLightFrags = 1024;
+constexpr uint32_t kLightAverage = 1000;   // k_raster: fragments a tile, past which none is tried
 constexpr uint32_t kLightStride = kRecWords + 1;   // odd: lanes reading different triangles meet different banks
 
 struct LightWave {
@@ -2287,14 +2297,17 @@ __global__ __launch_bounds__(NT, 4) void k_raster(DrawParams d0, BatchArgs b)
     __shared__ uint32_t heavy[WAVES];
     __shared__ uint32_t wave_frags[NT / 64];
 
-    // the tiles in the footprint union of the draw's big triangles, and its
-    // clipped sub-triangles (loads in flight with the schedule's)
-    uint32_t heavy_tiles = 0u;
+    // the tiles in the footprint union of the draw's big triangles, its
+    // clipped sub-triangles, and the binned triangles' area (loads in flight
+    // with the schedule's)
+    uint32_t heavy_tiles = 0u, area = 0u;
     if constexpr (!MULTI) {
         const uint32_t *c = d0.s.counters;
         uint32_t big = c[C_BIG], clipped = c[C_CLIP_TRI];
         uint32_t across = c[C_BIG_X1] + c[C_BIG_NX0] - 65534u, down = c[C_BIG_Y1] + c[C_BIG_NY0] - 65534u;
         heavy_tiles = max(big ? across * down : 0u, clipped);
+#pragma unroll
+        for (uint32_t x = 0; x < 8u; ++x) area += b.header[H_AREA + kQueueStride * x];
     }
     ActiveSchedule w(b);
     uint32_t frag_acc = 0;
@@ -2304,11 +2317,13 @@ __global__ __launch_bounds__(NT, 4) void k_raster(DrawParams d0, BatchArgs b)
     uint32_t entries = w.n;
     bool waves = entries > WAVES * gridDim.x;
     // nor where most tiles are not for a single wave: half of them under big
-    // triangles, or as many clipped sub-triangles as half the tiles (four
-    // tiles in a row by one workgroup are then a coarser share of the work;
+    // triangles, as many clipped sub-triangles as half the tiles, or more than
+    // kLightAverage fragments a tile (four tiles in a row by one workgroup are
+    // then a coarser share of the work, and trying each costs a tenth of it;
     // 1920x1080, 20000 triangles of 30 px: 216 us a pass in fours, 197 singly;
-    // 20000 of 20 px, half of them clipped: 212 and 195)
-    waves = waves && 2u * heavy_tiles < b.total_tiles;
+    // 20000 of 20 px, half of them clipped: 212 and 195; 60000 of 24 px, 1300
+    // fragments a tile: 351 and 301; of 18 px, 730 a tile: 226 and 239)
+    waves = waves && 2u * heavy_tiles < b.total_tiles && (uint64_t)area * 16u <= (uint64_t)kLightAverage * entries;
     if (waves) w.n = (entries + WAVES - 1u) / WAVES;
     uint32_t wave = threadIdx.x >> 6;
     bool dyn = w.dynamic();

@@ -160,9 +160,10 @@ enum Counter { C_BIG = 0, C_CLIP_TRI = 1, C_BIG_NX0 = 2, C_BIG_NY0 = 3, C_BIG_X1
 // Group header words: active tiles, primitives to clip, spilled bin
 // entries, big triangles of every draw of the group; then the tile
 // kernels' work queues, one ticket counter per XCD, 128 bytes apart
-// (H_QUEUE + kQueueStride * xcd).
+// (H_QUEUE + kQueueStride * xcd).  Beside them (H_AREA), the area of the binned
+// triangles of ordered draws, over eight words.
 constexpr uint32_t kQueueStride = 32;
-enum Header { H_ACTIVE = 0, H_CLIP = 1, H_SPILL = 2, H_BIG = 3, H_QUEUE = 32, H_NUM = 32 + 8 * 32 };
+enum Header { H_ACTIVE = 0, H_CLIP = 1, H_SPILL = 2, H_BIG = 3, H_QUEUE = 32, H_AREA = 33, H_NUM = 32 + 8 * 32 };
 
 // Triangle record: everything the raster needs about one (sub-)triangle,
 // computed once in setup (the same values the raster would compute).
