@@ -2561,11 +2561,14 @@ struct LineWalk {
     // remainder, in a tenth of the general 64-bit division's code.
     __device__ __forceinline__ uint32_t ratio(uint32_t a, uint32_t b, uint32_t c, uint32_t d) const
     {
-        if (!wide) return (a * b + c) / d;
-        uint64_t x = (uint64_t)a * b + c;
-        uint32_t e = (uint32_t)((double)x / (double)d);
-        int64_t r = (int64_t)(x - (uint64_t)e * d);
-        return r < 0 ? e - 1u : (r >= (int64_t)d ? e + 1u : e);
+        uint32_t e = (a * b + c) / d;   // (in every case: the divisor's reciprocal leaves the loops)
+        if (wide) {
+            uint64_t x = (uint64_t)a * b + c;
+            e = (uint32_t)((double)x / (double)d);
+            int64_t r = (int64_t)(x - (uint64_t)e * d);
+            e = r < 0 ? e - 1u : (r >= (int64_t)d ? e + 1u : e);
+        }
+        return e;
     }
     __device__ __forceinline__ uint32_t rise(uint32_t k) const { return ratio(k, q, 0u, n); }
     __device__ __forceinline__ int32_t minor(uint32_t k) const { return c0 + sc * (int32_t)rise(k); }
